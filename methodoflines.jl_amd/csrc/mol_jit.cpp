@@ -1318,7 +1318,7 @@ std::string Gen::stage_fn(bool lds) {
     return "L[" + istr(f) + " * VOL + ((" + q0 + ") - o0) + EX * (((" + q1 + ") - o1) + EY * ((" + q2 + ") - o2))]";
   };
   if (lds)
-    o << "  static __device__ T stage_lds(const int f, int p0, int p1, int p2, const double t, const T* __restrict__ P,\n"
+    o << "  static __device__ " << (d_->ndim == 1 ? "__forceinline__ " : "") << "T stage_lds(const int f, int p0, int p1, int p2, const double t, const T* __restrict__ P,\n"
          "                               const T* __restrict__ L, const int o0, const int o1, const int o2,\n"
          "                               const JPtrs& jp) {\n"
          "    (void)t; (void)P; (void)jp;\n";
@@ -1979,6 +1979,10 @@ std::string Gen::source_fused(bool f64) {
     reach[a] = us.reach[a];
     halo[a] = 4 * g_.fsteps * us.reach[a];
   }
+  // one 1D tile holding the whole system: the kernel runs any number of steps per launch with
+  // the state in registers (mol_rk4_ring), whose window has one reach more on either side
+  const bool resident = g_.ntile[0] * g_.ntile[1] * g_.ntile[2] == 1 && d_->ndim == 1 && g_.tile[0] >= halo[0];
+  if (resident) halo[0] += us.reach[0];
   std::ostringstream o;
   o << "// generated fused RK4 step of one PDE system\n";
   o << "#define MOL_T " << (f64 ? "double" : "float") << "\n";
@@ -2002,21 +2006,22 @@ std::string Gen::source_fused(bool f64) {
   const bool diam = us.separable && allper && d_->ndim == 2 && reach[0] == 1 && reach[1] == 1;
   o << "  static constexpr bool DIAM = " << (diam ? "true" : "false") << ";\n";
   if (!allper) o << stage_fn(true);
+  int kmax = 1;   // unknowns next to an end that a ghost combines
+  for (int k = 0; k < d_->nclosures; ++k) kmax = std::max(kmax, d_->closures_h[k].K);
+  o << "  static constexpr int KMAX = " << kmax << ";\n";
   o << close;
-  // one 1D tile holding the whole system: nsub resident steps per launch; otherwise one step
-  const bool resident = g_.ntile[0] * g_.ntile[1] * g_.ntile[2] == 1 && d_->ndim == 1 && g_.tile[0] >= halo[0];
   o << "extern \"C\" __global__ void __launch_bounds__(" << g_.nthr
-    << ") mol_rk4_fused(const T* __restrict__ u, T* __restrict__ unew, Epi ep, JPtrs jp, int nsub) {\n"
-       "  __shared__ T U[GeoF::NST * GeoF::VOL];\n  __shared__ T Ya[GeoF::NST * GeoF::VOL];\n"
-       "  __shared__ T Yb[GeoF::NST * GeoF::VOL];\n";
+    << ") mol_rk4_fused(const T* __restrict__ u, T* __restrict__ unew, Epi ep, JPtrs jp, int nsub) {\n";
+  if (resident) o << "  __shared__ T X[MolRing<GeoF>::XN];\n";
+  else o << "  __shared__ T U[GeoF::NST * GeoF::VOL];\n  __shared__ T Ya[GeoF::NST * GeoF::VOL];\n"
+            "  __shared__ T Yb[GeoF::NST * GeoF::VOL];\n";
   // two steps per launch: the running sums of the first step's frame positions
   if (g_.fsteps == 2 && !resident) o << "  __shared__ T Ac[GeoF::NST * GeoF::VOL];\n";
-  else o << "  T* const Ac = nullptr;\n";
+  else if (!resident) o << "  T* const Ac = nullptr;\n";
   o << "  // the step's time from the device clock, or (first launch of a call) by value in tofs\n"
        "  const double t = ep.tnow ? ep.tnow[0] : ep.tofs;\n";
   if (resident) {
-    o << "  mol_rk4_fused_resident<GeoF>(U, Ya, Yb, &mol_fc[0][0], (int)(sizeof(mol_fc[0]) / sizeof(double)), mol_fo,\n"
-         "                               u, unew, ep, jp, t, nsub);\n}\n";
+    o << "  mol_rk4_ring<GeoF>(X, &mol_fc[0][0], mol_fo, u, unew, ep, jp, t, nsub);\n}\n";
   } else {
     // nsub steps (1, or 2 with the 8-reach halo); the clock advances as by nsub launches
     o << "  int b = mol_xcd_tile<GeoBase::NBLK>((int)blockIdx.x);\n"

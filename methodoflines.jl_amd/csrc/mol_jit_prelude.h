@@ -864,14 +864,12 @@ __device__ __forceinline__ void mol_rk4_stage(const T* Lin, T* Lout, T* U, T (&U
                                               const int o0, const int o1,
                                               const int o2, const T* __restrict__ u, T* __restrict__ unew,
                                               const Epi& ep, const JPtrs& jp, const double t, const double dt,
-                                              T* Ukeep = nullptr, const bool store = true, T* Ac = nullptr) {
+                                              T* Ac) {
   // M: the stage region is the tile grown by M reach per axis.  ME: the step's result is
   // wanted on the tile grown by ME (ME > 0: the first of two steps in one launch, whose result
   // is the next step's tile + halo); the frame positions inside it keep their running sum in
   // Ac, and stage 4 (M == ME) leaves the new state in U, in place, at every position of its
   // region and in Ur for the tile nodes.
-  // Ukeep (resident steps): stage 4 also leaves the new state in Ukeep and in Ur for the next
-  // step; store: stage 4 writes it to unew
   static_assert(S < 4 ? M == ME + 4 - S : M == ME, "stage regions shrink by one reach per stage");
   constexpr int TVOL = MolFusedItems<G>::TVOL, NJ = MolFusedItems<G>::NJ;
   constexpr int FR = MolFrame2<G, M>::N;
@@ -879,7 +877,6 @@ __device__ __forceinline__ void mol_rk4_stage(const T* Lin, T* Lout, T* U, T (&U
   static_assert(!G::DIAM || (G::RX == 1 && G::RY == 1 && !G::FIX), "L1 stage regions: reach one, periodic");
   const double ts = t + (S == 1 ? 0.0 : (S == 4 ? dt : dt / 2));
   const double cf = S == 1 || S == 2 ? dt / 2 : (S == 3 ? dt : dt / 6);
-  if (ME > 0 && S == 4) Ukeep = U;
   // tile nodes: registers carry u and the running sum
   T out[NJ][G::NF];
 #pragma unroll
@@ -910,9 +907,9 @@ __device__ __forceinline__ void mol_rk4_stage(const T* Lin, T* Lout, T* U, T (&U
         Ar[j][f] = a;
       } else {
         v += (T)cf * Ar[j][f];
-        if (ME == 0 && store && I0 <= G::UHI0 && I1 <= G::UHI1 && I2 <= G::UHI2) unew[G::uidx(f, I0, I1, I2)] = v;
-        if (Ukeep) {
-          Ukeep[f * G::VOL + b] = v;
+        if (ME == 0 && I0 <= G::UHI0 && I1 <= G::UHI1 && I2 <= G::UHI2) unew[G::uidx(f, I0, I1, I2)] = v;
+        if (ME > 0) {
+          U[f * G::VOL + b] = v;
           Ur[j][f] = v;
           Ar[j][f] = T(0);
         }
@@ -993,22 +990,22 @@ __device__ __forceinline__ void mol_rk4_step(T* U, T* Ya, T* Yb, T* Ac, T (&Ur)[
                                              const int o0, const int o1, const int o2, const T* __restrict__ u,
                                              T* __restrict__ unew, const Epi& ep, const JPtrs& jp, const double t,
                                              const double dt) {
-  mol_rk4_stage<G, 1, ME + 3, ME>(U, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, nullptr, true, Ac);
+  mol_rk4_stage<G, 1, ME + 3, ME>(U, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, Ac);
   __syncthreads();
   if constexpr (G::FIX) {
     if (mol_rk4_fix_ghosts<G, ME + 3>(Ya, o0, o1, o2, t + dt / 2, ep.p, jp)) __syncthreads();
   }
-  mol_rk4_stage<G, 2, ME + 2, ME>(Ya, Yb, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, nullptr, true, Ac);
+  mol_rk4_stage<G, 2, ME + 2, ME>(Ya, Yb, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, Ac);
   __syncthreads();
   if constexpr (G::FIX) {
     if (mol_rk4_fix_ghosts<G, ME + 2>(Yb, o0, o1, o2, t + dt / 2, ep.p, jp)) __syncthreads();
   }
-  mol_rk4_stage<G, 3, ME + 1, ME>(Yb, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, nullptr, true, Ac);
+  mol_rk4_stage<G, 3, ME + 1, ME>(Yb, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, Ac);
   __syncthreads();
   if constexpr (G::FIX) {
     if (mol_rk4_fix_ghosts<G, ME + 1>(Ya, o0, o1, o2, t + dt, ep.p, jp)) __syncthreads();
   }
-  mol_rk4_stage<G, 4, ME, ME>(Ya, nullptr, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, nullptr, true, Ac);
+  mol_rk4_stage<G, 4, ME, ME>(Ya, nullptr, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, Ac);
   if constexpr (ME > 0) {
     __syncthreads();
     if constexpr (G::FIX) {
@@ -1081,83 +1078,203 @@ __device__ __forceinline__ void mol_rk4_fused_tile(T* U, T* Ya, T* Yb, T* Ac, do
   mol_rk4_step<G, 0>(U, Ya, Yb, Ac, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt);
 }
 
-// Resident steps of a 1D system held by a single tile: nsub RK4 steps in one launch with the
-// state in LDS (and, for the tile nodes, in registers).  Between steps the halo of U is
-// refreshed: periodic images copied from the tile (which covers the whole ring), ghosts of a
-// non-periodic axis from their closures at the new time.  The time advances by the same
-// sequence of additions as the device clock of one launch per step.
+// Value of the neighbouring lane (lane - 1, lane + 1) of the wave, 0 past its ends: DPP wave
+// shifts, no LDS access.  mol_lane(x, l): lane l's value in every lane (l: the same in every
+// lane).  Off the GPU a wave is one lane.
+#ifdef __AMDGCN__
+constexpr int MOL_WAVE = 64;
+template <int CTRL, class U>
+__device__ __forceinline__ U mol_dpp(const U x) {
+  constexpr int N = sizeof(U) / 4;
+  int w[N];
+  __builtin_memcpy(w, &x, sizeof(U));
+#pragma unroll
+  for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_update_dpp(0, w[k], CTRL, 0xf, 0xf, true);
+  U r;
+  __builtin_memcpy(&r, w, sizeof(U));
+  return r;
+}
+template <class U>
+__device__ __forceinline__ U mol_lane_below(const U x) { return mol_dpp<0x138>(x); }   // wave_shr:1
+template <class U>
+__device__ __forceinline__ U mol_lane_above(const U x) { return mol_dpp<0x130>(x); }   // wave_shl:1
+template <class U>
+__device__ __forceinline__ U mol_lane(const U x, const int l) {
+  constexpr int N = sizeof(U) / 4;
+  int w[N];
+  __builtin_memcpy(w, &x, sizeof(U));
+#pragma unroll
+  for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_readlane(w[k], l);
+  U r;
+  __builtin_memcpy(&r, w, sizeof(U));
+  return r;
+}
+#else
+constexpr int MOL_WAVE = 1;
+template <class U>
+inline U mol_lane_below(const U) { return U(0); }
+template <class U>
+inline U mol_lane_above(const U) { return U(0); }
+template <class U>
+inline U mol_lane(const U x, const int) { return x; }
+#endif
+
+// Resident steps of a 1D system held by a single work-group, the state in registers.  A lane
+// holds NJ consecutive nodes; the taps of its end nodes come from the neighbouring lanes by DPP,
+// so a stage has no LDS access and no barrier.  One wave holds a non-periodic system whole.
+// Otherwise (several waves, or a periodic ring) a wave holds S nodes and, evaluated redundantly,
+// the HL = 4 reach nodes past either end: a whole step needs no other wave, and the end nodes
+// are exchanged once per step through LDS (two buffers in turn, one barrier).
+// What bounds it is the issue of a wave's serial chain (about 100 VALU instructions per step of
+// the 101-node FP64 heat equation: 0.155 us, against 0.88 us for the stages on an LDS tile with
+// two barriers each).
 template <class G>
-__device__ __forceinline__ void mol_rk4_fused_resident(T* U, T* Ya, T* Yb, double* fc, const int fcs, int* fo,
-                                                       const T* __restrict__ u, T* __restrict__ unew, const Epi& ep,
-                                                       const JPtrs& jp, const double t0, const int nsub) {
-  static_assert(G::NBLK == 1 && G::RY == 0 && G::TY == 1, "resident steps: one 1D tile");
+struct MolRing {
+  static constexpr int LN = G::NTHR < MOL_WAVE ? G::NTHR : MOL_WAVE;   // lanes per wave
+  static constexpr int W = G::NTHR / LN;                               // waves
+  static constexpr int R = G::RX, TN = G::TX;                          // reach, nodes
+  static constexpr bool PER = G::PER0 != 0, ONE = W == 1 && !PER;
+  static constexpr int HL = ONE ? 0 : 4 * R;
+  static constexpr int S = (TN + W - 1) / W;                           // nodes of a wave
+  static constexpr int NJ0 = (S + 2 * HL + LN - 1) / LN, NJ = NJ0 > R ? NJ0 : (R > 0 ? R : 1);
+  static constexpr int SL = TN - (W - 1) * S;                          // nodes of the last wave
+  static constexpr int XN = ONE ? 1 : 2 * G::NF * TN;                  // exchange buffers (values)
+  // the ghosts of an end are needed by the wave that holds it only: the waves next to it do not
+  // reach past its own nodes
+  static_assert(W == 1 || (S >= HL + G::KMAX && SL >= HL + G::KMAX), "a wave holds too few nodes");
+  static_assert(NJ + 2 * R <= G::VOL, "register window larger than the printed geometry");
+};
+
+template <class G>
+__device__ __forceinline__ void mol_rk4_ring(T* X, double* fc, int* fo, const T* __restrict__ u,
+                                             T* __restrict__ unew, const Epi& ep, const JPtrs& jp, const double t0,
+                                             const int nsub) {
+  using Q = MolRing<G>;
+  static_assert(G::NBLK == 1 && G::RY == 0 && G::TY == 1 && (Q::PER || G::RX <= 1), "resident steps: one 1D tile");
+  constexpr int R = Q::R, NJ = Q::NJ, NF = G::NF, NI = G::NINV > 0 ? G::NINV : 1;
   const int o0 = G::ULO0, o1 = G::ULO1, o2 = G::ULO2;
   const double dt = ep.tadv;
-  mol_stage_tile<G>(U, o0, o1, o2, mol_stage_mode<G>(0, 0, 0), t0, ep.p, u, jp);
-  {
-    const int org = o0 - G::HX;
-    if (threadIdx.x == 0) fo[0] = org;
-    if (jp.coord[0])
-      for (int e = threadIdx.x; e < G::EX; e += G::NTHR) {
-        int p = org + e;
-        if (G::PER0) p = mol_wrap(mol_wrap(p, G::N0), G::N0);
-        fc[e] = jp.coord[0][min(max(p, 1), (int)G::N0) - 1];
-      }
-  }
+  // coordinates of the tile + halo (periodic images wrapped)
+  if (threadIdx.x == 0) fo[0] = o0 - G::HX;
+  if (jp.coord[0])
+    for (int e = (int)threadIdx.x; e < G::EX; e += G::NTHR) {
+      int p = o0 - G::HX + e;
+      if (Q::PER) p = mol_wrap(mol_wrap(p, G::N0), G::N0);
+      fc[e] = jp.coord[0][min(max(p, 1), (int)G::N0) - 1];
+    }
   __syncthreads();
-  constexpr int NJ = MolFusedItems<G>::NJ;
-  T Ur[NJ][G::NF], Ar[NJ][G::NF];
+  const int wv = (int)threadIdx.x / Q::LN, lane = (int)threadIdx.x % Q::LN;
+  const int i0 = wv * Q::S - Q::HL + lane * NJ;   // node (from 0) of the lane's first slot
+  // node held by slot j: its image on a periodic axis, the end node past a non-periodic end
+  // (such slots are evaluated, their values never reach a node)
+  auto at = [&](const int j) {
+    int i = i0 + j;
+    if (Q::PER) {
+      if (i < 0) i += Q::TN;
+      else if (i >= Q::TN) i -= Q::TN;
+    }
+    return min(max(i, 0), Q::TN - 1);
+  };
+  auto own = [&](const int j) {
+    const int r = lane * NJ + j - Q::HL;
+    return r >= 0 && r < Q::S && wv * Q::S + r < Q::TN;
+  };
+  T U[NJ][NF], A[NJ][NF], y[NJ][NF], Iv[NJ][NI];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    int lx, ly;
-    MolFusedItems<G>::pos(j, lx, ly);
-    const bool ok = MolFusedItems<G>::valid(j);
-    const int b = ok ? (lx + G::HX) + G::EX * (ly + G::HY) : 0;
 #pragma unroll
-    for (int f = 0; f < G::NF; ++f) {
-      Ur[j][f] = ok ? U[f * G::VOL + b] : T(0);
-      Ar[j][f] = T(0);
+    for (int f = 0; f < NF; ++f) {
+      U[j][f] = y[j][f] = u[G::uidx(f, o0 + at(j), o1, o2)];
+      A[j][f] = T(0);
     }
+    if constexpr (G::NINV > 0) G::node_inv(o0 + at(j), o1, o2, ep.p, jp, Iv[j]);
   }
-  MolFusedInv<G> Iv;
-  Iv.init(o0, o1, o2, ep.p, jp);
+  // slot of the first and last node (compile time) and the lane holding it in this wave, or -1
+  constexpr int QL = Q::HL, QH = Q::HL + Q::SL - 1;
+  const bool low = !Q::PER && wv == 0 && lane == QL / NJ, high = !Q::PER && wv == Q::W - 1 && lane == QH / NJ;
   double t = t0;
-  for (int k = 0; k < nsub; ++k) {
-    const bool last = k == nsub - 1;
-    mol_rk4_stage<G, 1>(U, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt);
-    __syncthreads();
-    if constexpr (G::FIX) {
-      if (mol_rk4_fix_ghosts<G, 3>(Ya, o0, o1, o2, t + dt / 2, ep.p, jp)) __syncthreads();
-    }
-    mol_rk4_stage<G, 2>(Ya, Yb, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt);
-    __syncthreads();
-    if constexpr (G::FIX) {
-      if (mol_rk4_fix_ghosts<G, 2>(Yb, o0, o1, o2, t + dt / 2, ep.p, jp)) __syncthreads();
-    }
-    mol_rk4_stage<G, 3>(Yb, Ya, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt);
-    __syncthreads();
-    if constexpr (G::FIX) {
-      if (mol_rk4_fix_ghosts<G, 1>(Ya, o0, o1, o2, t + dt, ep.p, jp)) __syncthreads();
-    }
-    // the stage-4 frame is empty: U is only read at tile positions by stage 4 (through Ur)
-    mol_rk4_stage<G, 4>(Ya, nullptr, U, Ur, Ar, Iv, o0, o1, o2, u, unew, ep, jp, t, dt, U, last);
-    t = t + dt;
-    if (last) break;
-    __syncthreads();
-    // refresh the halo of U for the next step
-    if constexpr (G::PER0) {
-      constexpr int P = G::TX;   // the tile is the whole ring of unknowns
-      for (int q = threadIdx.x; q < 2 * G::HX; q += G::NTHR) {
-        const int lx = q < G::HX ? q - G::HX : G::TX + (q - G::HX);
-        const int src = lx < 0 ? lx + P : lx - P;
+  // one stage: w holds the lane's nodes and R taps on either side
+  auto stage = [&](const int s) {
+    const double ts = t + (s == 1 ? 0.0 : (s == 4 ? dt : dt / 2));
+    const double cf = s <= 2 ? dt / 2 : (s == 3 ? dt : dt / 6);
+    T w[NF * G::VOL];
 #pragma unroll
-        for (int f = 0; f < G::NF; ++f) U[f * G::VOL + lx + G::HX] = U[f * G::VOL + src + G::HX];
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) w[f * G::VOL + R + j] = y[j][f];
+#pragma unroll
+      for (int q = 1; q <= R; ++q) {
+        w[f * G::VOL + R - q] = mol_lane_below(y[NJ - q][f]);
+        w[f * G::VOL + R + NJ - 1 + q] = mol_lane_above(y[q - 1][f]);
       }
-    } else {
-      mol_rk4_fix_ghosts<G, 4>(U, o0, o1, o2, t, ep.p, jp);
     }
-    __syncthreads();
+    if constexpr (G::FIX && R > 0) {
+      // ghosts of the boundary equations from the KMAX nodes next to each end
+      T el[NF * G::VOL], eh[NF * G::VOL];
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int m = 0; m < G::KMAX; ++m) {
+          el[f * G::VOL + m] = mol_lane(y[(QL + m) % NJ][f], (QL + m) / NJ);
+          eh[f * G::VOL + G::KMAX - 1 - m] = mol_lane(y[(QH - m) % NJ][f], (QH - m) / NJ);
+        }
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const T gl = G::stage_lds(f, (int)G::ULO0 - 1, o1, o2, ts, ep.p, el, (int)G::ULO0, o1, o2, jp);
+        const T gh = G::stage_lds(f, (int)G::UHI0 + 1, o1, o2, ts, ep.p, eh, (int)G::UHI0 - (G::KMAX - 1), o1, o2, jp);
+        T& wl = w[f * G::VOL + R + QL % NJ - 1];
+        wl = low ? gl : wl;
+        T& wh = w[f * G::VOL + R + QH % NJ + 1];
+        wh = high ? gh : wh;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      T out[NF];
+      if constexpr (G::NINV > 0) G::node_h(w, R + j, o0 + at(j), o1, o2, ts, ep.p, u, jp, Iv[j], out);
+      else G::node(w, R + j, o0 + at(j), o1, o2, ts, ep.p, u, jp, out);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        T v = (T)cf * out[f];
+        v += U[j][f];
+        if (s < 4) {
+          T a = (s == 1 ? T(1) : T(2)) * out[f];
+          if (s > 1) a += A[j][f];
+          A[j][f] = a;
+        } else {
+          v += (T)cf * A[j][f];
+          U[j][f] = v;
+        }
+        y[j][f] = v;
+      }
+    }
+  };
+  for (int k = 0; k < nsub; ++k) {
+    stage(1);
+    stage(2);
+    stage(3);
+    stage(4);
+    t = t + dt;
+    if (!Q::ONE && k + 1 < nsub) {
+      T* const B = X + (k & 1) * (NF * Q::TN);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          if (own(j)) B[f * Q::TN + at(j)] = U[j][f];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          if (!own(j)) U[j][f] = y[j][f] = B[f * Q::TN + at(j)];
+    }
   }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      if (own(j)) unew[G::uidx(f, o0 + at(j), o1, o2)] = U[j][f];
   if (ep.tnext && threadIdx.x == 0) ep.tnext[0] = t;
 }
 
