@@ -147,46 +147,59 @@ __device__ __noinline__ T mol_powi(T x, int e) {
   return neg ? T(1) / r : r;
 }
 
-// FP64 quotient n / d for the WENO5 weights: the hardware reciprocal (v_rcp_f64) refined by
-// two Newton steps and the quotient corrected by its residual (Markstein): 8 instructions
-// against about 11 for the IEEE division sequence, within an ulp or two of the IEEE quotient.
+// FP64 quotient n / d for the WENO5 weights: the hardware reciprocal (v_rcp_f64, about 23 good
+// bits) refined by one Newton step (46 bits) and the quotient corrected by its residual
+// (Markstein; the correction's relative error is the square of the reciprocal's): 6 instructions
+// against about 11 for the IEEE division sequence, within an ulp of the IEEE quotient.
 // d is a positive normal number here (a product of sums of squares offset by eps).
 __device__ __forceinline__ double mol_quot(const double n, const double d) {
   double r = __builtin_amdgcn_rcp(d);
-  r = fma(r, fma(-d, r, 1.0), r);
   r = fma(r, fma(-d, r, 1.0), r);
   const double q = n * r;
   return fma(r, fma(-d, q, n), q);
 }
 
-// Jiang-Shu WENO5 node derivative (u^-_{i+1/2} - u^+_{i-1/2}) / dx from the five values
-// u(i-2) .. u(i+2).  The candidate reconstructions are written as u(i) + difference/6 so u(i)
-// cancels, and the normalised nonlinear weights gamma_k/q_k / sum_j gamma_j/q_j are cleared
-// to gamma_k P_k / sum_j gamma_j P_j (P_k = product of the other two q_j): one division.  The
-// weights are unchanged when every eps + beta_k is scaled by one factor, so the smoothness
-// sums are formed as 4 (eps + beta_k) = 13/3 D2^2 + a^2 + 4 eps (no 1/4 and 13/12 products).
+// What both forms of the Jiang-Shu WENO5 node derivative (u^-_{i+1/2} - u^+_{i-1/2}) / dx share,
+// from the five values u(i-2) .. u(i+2).  Every candidate reconstruction is the central one plus
+// a multiple of a third difference: with E = D2_{i+1} - D2_i, F = D2_i - D2_{i-1} and weights
+// proportional to g_k w_k (w_k = 1 / (eps + beta_k)^2 up to one common factor),
+//   6 (u^- - u^+) = 3 (u_{i+1} - u_{i-1}) - (3 X + 2 Y) / Dp - (2 X + 3 Y) / Dm,
+//   X = w_1 E,  Y = w_3 F,  Dp = 3 w_1 + 6 w_2 + w_3,  Dm = w_1 + 6 w_2 + 3 w_3
+// (w_1: the stencil i .. i+2).  The smoothness sums are formed as 4 (eps + beta_k) = 13/3 D2^2 +
+// a^2 + 4 eps.  Sums that the neighbouring node along the axis shares (differences, D2, the
+// 13/3 D2^2 terms) are written as expressions of their own.
+template <class U>
+struct MolWeno5 {
+  U a2, E, F, b1, b2, b3;
+  __device__ __forceinline__ MolWeno5(U um2, U um1, U u0, U up1, U up2, T eps) {
+    const U dmm = um1 - um2, dm = u0 - um1, dp = up1 - u0, dpp = up2 - up1;
+    const U D2m = dm - dmm, D20 = dp - dm, D2p = dpp - dp;
+    const U a1 = T(-2) * dp + D2p, a3 = T(2) * dm + D2m;
+    a2 = dm + dp;
+    E = D2p - D20;
+    F = D20 - D2m;
+    const T eps4 = T(4) * eps;
+    b1 = a1 * a1 + ((T(13.0 / 3.0) * D2p) * D2p + eps4);
+    b2 = a2 * a2 + ((T(13.0 / 3.0) * D20) * D20 + eps4);
+    b3 = a3 * a3 + ((T(13.0 / 3.0) * D2m) * D2m + eps4);
+  }
+  // the derivative from the weights
+  __device__ __forceinline__ U apply(const U w1, const U w2, const U w3, const T inv_dx) const {
+    const U X = w1 * E, Y = w3 * F;
+    const U Dp = T(3) * w1 + (T(6) * w2 + w3), Dm = T(3) * w3 + (T(6) * w2 + w1);
+    const U Np = T(3) * X + T(2) * Y, Nm = T(2) * X + T(3) * Y;
+    return (T(0.5) * inv_dx) * a2 - (inv_dx * T(1.0 / 6.0)) * mol_quot(Np * Dm + Nm * Dp, Dp * Dm);
+  }
+};
+
+// FP64: w_k cleared to the product of the other two (4 (eps + beta_j))^2, so the derivative has
+// one quotient.  48 instructions per derivative (61 with the candidate values and both normalised
+// weight sets formed separately): Burgers right-hand side at 4096^2 103 -> 92 us.
 template <class U>
 __device__ __forceinline__ U mol_weno5_t(U um2, U um1, U u0, U up1, U up2, T eps, T inv_dx) {
-  const U dmm = um1 - um2, dm = u0 - um1, dp = up1 - u0, dpp = up2 - up1;
-  const U D2m = dm - dmm, D20 = dp - dm, D2p = dpp - dp;
-  const U a1 = T(-2) * dp + D2p;
-  const U a2 = dm + dp;
-  const U a3 = T(2) * dm + D2m;
-  const T eps4 = T(4) * eps;
-  const U b1 = (T(13.0 / 3.0) * D2p) * D2p + (a1 * a1 + eps4);
-  const U b2 = (T(13.0 / 3.0) * D20) * D20 + (a2 * a2 + eps4);
-  const U b3 = (T(13.0 / 3.0) * D2m) * D2m + (a3 * a3 + eps4);
-  const U q1 = b1 * b1, q2 = b2 * b2, q3 = b3 * b3;
-  const U P1 = q2 * q3, P2 = q1 * q3, P3 = q1 * q2;
-  const U A1 = T(0.3) * P1, A2 = T(0.6) * P2, A3 = T(0.1) * P3;
-  const U B1 = T(0.1) * P1, B3 = T(0.3) * P3;
-  const U Dp = A1 + A2 + A3;
-  const U Dm = B1 + A2 + B3;
-  const U ep1 = T(4) * dp - dpp, ep2 = T(2) * dp + dm, ep3 = T(5) * dm - T(2) * dmm;
-  const U em1 = T(-5) * dp + T(2) * dpp, em2 = T(-2) * dm - dp, em3 = T(-4) * dm + dmm;
-  const U Np = A1 * ep1 + A2 * ep2 + A3 * ep3;
-  const U Nm = B1 * em1 + A2 * em2 + B3 * em3;
-  return mol_quot(Np * Dm - Nm * Dp, Dp * Dm) * (inv_dx * T(1.0 / 6.0));
+  const MolWeno5<U> s(um2, um1, u0, up1, up2, eps);
+  const U q1 = s.b1 * s.b1, q2 = s.b2 * s.b2, q3 = s.b3 * s.b3;
+  return s.apply(q2 * q3, q1 * q3, q1 * q2, inv_dx);
 }
 
 // Reciprocal and quotient for the FP32 WENO5 weights: the hardware reciprocal (v_rcp_f32,
@@ -198,40 +211,26 @@ __device__ __forceinline__ float mol_rcp(const float x) {
   return fmaf(r, fmaf(-x, r, 1.0f), r);
 }
 __device__ __forceinline__ double mol_rcp(const double x) { return 1.0 / x; }
-__device__ __forceinline__ float mol_div(const float n, const float d) {
+__device__ __forceinline__ float mol_quot(const float n, const float d) {
   const float r = mol_rcp(d);
   const float q = n * r;
   return fmaf(fmaf(-d, q, n), r, q);
 }
-__device__ __forceinline__ double mol_div(const double n, const double d) { return n / d; }
 
-// The same derivative in the reference's normalised-weight form (weno_f_uniform,
-// src/discretization/schemes/WENO/WENO.jl:6-57).  Used in FP32, where the products of four
-// squared smoothness indicators of the cleared form (~eps^8) underflow.
+__device__ __forceinline__ double mol_val(double v) { return v; }
+__device__ __forceinline__ float mol_val(float v) { return v; }
+
+// FP32, where products of four squared smoothness sums (~eps^8) underflow: w_k = (b / b_k)^2 with
+// b the smallest of the three sums, so every weight lies in (0, 1], at least one is 1, and
+// neither the sums nor the quotient leave the FP32 range whatever eps and the state's scale.
+// One quotient instead of two and no cancellation of the two face values (SSPRK3 step of the
+// FP32 + Kahan Burgers system at 1447^2: 67 -> 50 us).
 template <class U>
 __device__ __forceinline__ U mol_weno5_ref_t(U um2, U um1, U u0, U up1, U up2, T eps, T inv_dx) {
-  const U c1 = u0 - T(2) * up1 + up2, c2 = T(3) * u0 - T(4) * up1 + up2;
-  const U c3 = um1 - T(2) * u0 + up1, c4 = um1 - up1;
-  const U c5 = um2 - T(2) * um1 + u0, c6 = um2 - T(4) * um1 + T(3) * u0;
-  const U b1 = T(13) * c1 * c1 / T(12) + c2 * c2 / T(4);
-  const U b2 = T(13) * c3 * c3 / T(12) + c4 * c4 / T(4);
-  const U b3 = T(13) * c5 * c5 / T(12) + c6 * c6 / T(4);
-  const U q1 = (eps + b1) * (eps + b1), q2 = (eps + b2) * (eps + b2), q3 = (eps + b3) * (eps + b3);
-  // the six weights share three reciprocals and each normalisation one division
-  const U r1 = mol_rcp(q1), r2 = mol_rcp(q2), r3 = mol_rcp(q3);
-  const U om1 = T(0.1) * r1, om2 = T(0.6) * r2, om3 = T(0.3) * r3;
-  const U op1 = T(0.3) * r1, op2 = T(0.6) * r2, op3 = T(0.1) * r3;
-  const U wmd = om1 + om2 + om3, wpd = op1 + op2 + op3;
-  // candidate values times 6 (the 1/6 goes into the final scale)
-  const U hm1 = T(11) * u0 - T(7) * up1 + T(2) * up2;
-  const U hm2 = T(5) * u0 - up1 + T(2) * um1;
-  const U hm3 = T(2) * u0 + T(5) * um1 - um2;
-  const U hp1 = T(2) * u0 + T(5) * up1 - up2;
-  const U hp2 = T(5) * u0 + T(2) * up1 - um1;
-  const U hp3 = T(11) * u0 - T(7) * um1 + T(2) * um2;
-  const U hp = mol_div(op1 * hp1 + op2 * hp2 + op3 * hp3, wpd);
-  const U hm = mol_div(om1 * hm1 + om2 * hm2 + om3 * hm3, wmd);
-  return (hp - hm) * (inv_dx * T(1.0 / 6.0));
+  const MolWeno5<U> s(um2, um1, u0, up1, up2, eps);
+  const T b = fmin(fmin(mol_val(s.b1), mol_val(s.b2)), mol_val(s.b3));
+  const U r1 = b * mol_rcp(s.b1), r2 = b * mol_rcp(s.b2), r3 = b * mol_rcp(s.b3);
+  return s.apply(r1 * r1, r2 * r2, r3 * r3, inv_dx);
 }
 
 __device__ __forceinline__ T mol_weno5(T um2, T um1, T u0, T up1, T up2, T eps, T inv_dx) {
@@ -265,8 +264,9 @@ __device__ __forceinline__ MolDual mol_rcp(const MolDual x) {
   const T r = mol_rcp(x.v);
   return {r, -(x.d * r) * r};
 }
-__device__ __forceinline__ MolDual mol_div(const MolDual n, const MolDual d) { return n / d; }
 __device__ __forceinline__ MolDual mol_quot(const MolDual n, const MolDual d) { return n / d; }
+
+__device__ __forceinline__ T mol_val(MolDual v) { return v.v; }
 
 // Gradient of the WENO5 node derivative with respect to its five inputs.
 __device__ __noinline__ void mol_weno5_grad(T um2, T um1, T u0, T up1, T up2, T eps, T inv_dx, T* g, bool cleared) {
@@ -312,10 +312,6 @@ __device__ __forceinline__ void mol_fornberg3(const double a0, const double a1, 
   m1[2] = r2 * (a2m0 - sB2 * a2m1);
   m2[2] = r2 * (2.0 * a2m1 - sB2 * a2m2);
 }
-
-__device__ __forceinline__ double mol_val(double v) { return v; }
-__device__ __forceinline__ float mol_val(float v) { return v; }
-__device__ __forceinline__ T mol_val(MolDual v) { return v.v; }
 
 template <class U>
 __device__ __forceinline__ U mol_dot3(const double* w, U a, U b, U c) {
