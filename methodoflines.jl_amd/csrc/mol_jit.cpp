@@ -342,7 +342,10 @@ class Gen {
   std::string ref(int id) const;
   // row of the nonuniform-WENO coefficient table of the axis of X_WENONU node n at its node
   std::string wrow(const Node& n) const {
-    return "(jp.wtab[" + istr(n.ax) + "] + MOL_NU_NC * (" + n.text + " - 1))";
+    // the stage regions of the fused step reach past the ends of a periodic axis
+    std::string i = n.text;
+    if (fused_ && g_.periodic[n.ax]) i = "mol_wrap(mol_wrap(" + i + ", " + NN(n.ax) + "), " + NN(n.ax) + ")";
+    return "(jp.wtab[" + istr(n.ax) + "] + MOL_NU_NC * (" + i + " - 1))";
   }
   std::string op_expr(const Node& n, int id) const;
   void print_region(std::ostream& o, int r) const;

@@ -179,3 +179,20 @@ def test_generated_reverse_mode_matches_finite_differences(periodic):
     d2 = (F(u + h / 2 * v) - F(u - h / 2 * v)) / h
     fd = (4 * d2 - d1) / 3
     assert abs(g @ v - fd) <= 1e-8 * abs(fd)
+
+
+def test_fused_step_wraps_the_coefficient_rows():
+    """The fused RK4 step of a periodic stretched system evaluates frame nodes past the ends of the
+    ring: they take the coefficient row of the node whose image they are (an unwrapped index
+    reads outside the axis table)."""
+    low = lower(*systems.weno1d_nonuniform(systems.stretched_grid(61, 1.0, 4), 1.0, periodic=True))
+    u = np.random.default_rng(2).uniform(0.5, 1.5, low.n_unknowns)
+    dt = 1e-3
+    f = lambda w: genhost.rhs(low, w)
+    k1 = f(u)
+    k2 = f(u + dt / 2 * k1)
+    k3 = f(u + dt / 2 * k2)
+    k4 = f(u + dt * k3)
+    ref = u + dt / 6 * (k1 + 2 * k2 + 2 * k3 + k4)
+    got, _ = genhost.rk4_fused(low, u, 0.0, dt, tile=(16, 1, 1))
+    assert np.max(np.abs(got - ref)) <= 1e-14 * np.max(np.abs(ref))
