@@ -133,6 +133,7 @@ class Gen {
   bool ok_ = true;
   bool param_ = false;                // parametric (batched) printing
   bool fused_ = false;                // fused RK4 step printing (coordinates from LDS)
+  bool vjp_ = false;                  // reverse-mode kernel printing
   bool stage_noif_ = false;           // printing stage_ni (interface sides read nothing)
   // printing overrides: nodes not printed, and nodes referenced by another expression
   std::vector<char> skip_;
@@ -342,10 +343,23 @@ class Gen {
   std::string ref(int id) const;
   // row of the nonuniform-WENO coefficient table of the axis of X_WENONU node n at its node
   std::string wrow(const Node& n) const {
+    // centred target along x of a forward kernel: the tile's columns in LDS
+    if (nup() > 0 && n.ax == 0 && n.target == 3)
+      return "MolCol<" + istr(nup()) + ">{mol_nux + (I0 - " + istr(g_.ulo[0]) + ") % " + istr(g_.tile[0]) + "}";
     // the stage regions of the fused step reach past the ends of a periodic axis
     std::string i = n.text;
     if (fused_ && g_.periodic[n.ax]) i = "mol_wrap(mol_wrap(" + i + ", " + NN(n.ax) + "), " + NN(n.ax) + ")";
-    return "(jp.wtab[" + istr(n.ax) + "] + MOL_NU_NC * (" + i + " - 1))";
+    return std::string(n.target == 3 && !vjp_ ? "(MolRow)" : "") + "(jp.wtab[" + istr(n.ax) + "] + MOL_NU_NC * (" + i +
+           " - 1))";
+  }
+  // Padded width of the tile's table of WENO5 coefficients along x in LDS; 0: read the rows of
+  // the axis table (no such slot; 1D, where a node's row is used once; tiles wider than 128
+  // nodes, whose table would cost occupancy; the reverse sweep and the fused step).
+  int nup() const {
+    if (param_ || fused_ || vjp_ || d_->ndim < 2 || g_.tile[0] > 128) return 0;
+    for (int k = 0; k < d_->nslots; ++k)
+      if (d_->slots_h[k].kind == MOL_SLOT_WENO_NU && d_->slots_h[k].axis == 0) return g_.tile[0] + 1;
+    return 0;
   }
   std::string op_expr(const Node& n, int id) const;
   void print_region(std::ostream& o, int r) const;
@@ -1117,7 +1131,7 @@ std::string Gen::op_expr(const Node& n, int id) const {
       return e;
     }
     case X_WENONU:
-      return "mol_weno5_nu_tab(" + A(0) + ", " + A(1) + ", " + A(2) + ", " + A(3) + ", " + A(4) + ", " + wrow(n) +
+      return std::string(n.target == 3 ? "mol_weno5_nu3(" : "mol_weno5_nu_tab(") + A(0) + ", " + A(1) + ", " + A(2) + ", " + A(3) + ", " + A(4) + ", " + wrow(n) +
              ", " + pk(n.w[0], d_->ncpool + 2LL * n.imm) + ")";
     case X_WENO:
       // FP64: one-division cleared form; FP32: normalised weights (the cleared form underflows)
@@ -1249,7 +1263,7 @@ void Gen::print_reverse(std::ostream& o, int r, const std::vector<std::pair<int,
           << ", " << (d_->dtype == MOL_F64 ? "true" : "false") << ");\n";
       }
       if (n.op == X_WENONU) {
-        o << "    T wd" << id << "[5];\n    mol_weno5_nu_tab_grad(";
+        o << "    T wd" << id << "[5];\n    " << (n.target == 3 ? "mol_weno5_nu3_grad(" : "mol_weno5_nu_tab_grad(");
         for (int q = 0; q < 5; ++q) o << ref(n.a[q]) << ", ";
         o << wrow(n) << ", " << pk(n.w[0], d_->ncpool + 2LL * n.imm) << ", wd" << id << ");\n";
       }
@@ -1686,6 +1700,8 @@ std::string Gen::geo_variant(const std::string& name, const int* halo, const Usa
     c("FLO" + istr(a), flo);
     c("FHI" + istr(a), fhi);
   }
+  c("NUP", nup());
+  if (nup() > 0) o << "  static __device__ __forceinline__ T* nux() { return mol_nux; }\n";
   // values of the staged arrays at one tile + halo position (p: unwrapped full-grid index),
   // v[slot]; mode 0: plain loads, 1: plain loads after the periodic wrap, 2: through the ghost
   // closures
@@ -1787,6 +1803,7 @@ std::string Gen::geo_variant(const std::string& name, const int* halo, const Usa
 // Forward (vjp = false) or reverse-mode kernel of one system.
 std::string Gen::source_kernel(bool f64, bool vjp) {
   std::ostringstream o;
+  vjp_ = vjp;
   o << "// generated " << (vjp ? "vector-Jacobian product of the " : "") << "right-hand side of one PDE system\n";
   o << "#define MOL_T " << (f64 ? "double" : "float") << "\n";
   o << "#include \"mol_jit_prelude.h\"\n\n";
@@ -1799,6 +1816,7 @@ std::string Gen::source_kernel(bool f64, bool vjp) {
   build_node(false, out_bound, r_bound);
   if (!ok_) return "";
   const Usage us = usage();
+  if (nup() > 0) o << "__shared__ T mol_nux[MOL_NU3 * " << nup() << "];\n\n";
   o << "struct GeoBase {\n" << geo_common() << stage << scatter << "};\n\n";
   int lds = 1, ldsf = 1, ldsa = 1, npf = 1;
   auto sizes = [&](const PrintGeo& pg) {

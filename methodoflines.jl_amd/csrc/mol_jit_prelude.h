@@ -318,14 +318,118 @@ __device__ __forceinline__ U mol_dot3(const double* w, U a, U b, U c) {
   return (T)w[0] * a + (T)w[1] * b + (T)w[2] * c;
 }
 
-// The coordinate-only part of the nonuniform WENO5 derivative at one node (target TG of the
-// stencil x1..x5), MOL_NU_NC values: for each sub-stencil k = 0, 1, 2 the weights of r_k
+// Centred target (node 3 of the stencil: every node but the two next to a non-periodic end).
+// Here the ideal weights d_k are positive on any nodes (the denominators of 1 - d_0 - d_2 add up
+// to sums of products of spacings), so the split weights are 2 d_k and d_k, both normalised sets
+// are equal and the derivative is the single sum  sum_k w_k r_k, w_k ~ d_k / (eps + beta_k)^2.
+// The quadratic p_k has p_k'(x) = pM + (x - xM) pp, so Simpson's rule of the smoothness indicator
+// is exact: beta_k = (dx pM)^2 + 13/12 (dx^2 pp)^2 and r_k = (g_k + gamma c_k) / dx with
+// g_k = dx pM, c_k = sqrt(13/12) dx^2 pp, each a combination of two differences of u.
+// MOL_NU3 coefficients: per k the factors of the differences in g_k and c_k, then gamma, 1/dx,
+// d_0, d_1, d_2.
+constexpr int MOL_NU3 = 17;
+constexpr int MOL_NU_NC = 56;   // row stride of the axis tables
+
+__device__ __forceinline__ void mol_weno5_nu3_coefs(const double* x, double* c) {
+  const double xL = (x[1] + x[2]) / 2, xph = (x[2] + x[3]) / 2, dx = xph - xL, xM = (xL + xph) / 2;
+  const double s = 1.0408329997330663;   // sqrt(13/12)
+  for (int k = 0; k < 3; ++k) {
+    double m0[3], m1[3], m2[3];
+    mol_fornberg3(x[k], x[k + 1], x[k + 2], xM, m0, m1, m2);
+    c[4 * k + 0] = -dx * m1[0];
+    c[4 * k + 1] = dx * m1[2];
+    c[4 * k + 2] = -s * dx * dx * m2[0];
+    c[4 * k + 3] = s * dx * dx * m2[2];
+  }
+  c[12] = (x[2] - xM) / (dx * s);
+  c[13] = 1.0 / dx;
+  c[14] = ((x[2] - x[3]) * (x[2] - x[4])) / ((x[0] - x[3]) * (x[0] - x[4]));
+  c[16] = ((x[2] - x[0]) * (x[2] - x[1])) / ((x[4] - x[0]) * (x[4] - x[1]));
+  c[15] = 1.0 - c[14] - c[16];
+}
+
+// The derivative from the coefficients (C: a row, or a column of the tile's table in LDS).  The
+// weights are cleared to products in FP64 and scaled by the smallest sum in FP32, as on uniform
+// nodes: one quotient.  17 coefficients and 46 operations against 56 and about 140 of the split
+// form: the FP64 Burgers right-hand side on 1024^2 stretched nodes 116 -> 9.7 us, with the
+// coefficients along x read from the tile's columns in LDS and those along y by scalar loads.
+template <class U, class C>
+__device__ __forceinline__ U mol_weno5_nu3_t(U u1, U u2, U u3, U u4, U u5, const C& c, const T eps) {
+  const U d[4] = {u2 - u1, u3 - u2, u4 - u3, u5 - u4};
+  U e[3], r[3], w[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const U g = (T)c[4 * k] * d[k] + (T)c[4 * k + 1] * d[k + 1];
+    const U h = (T)c[4 * k + 2] * d[k] + (T)c[4 * k + 3] * d[k + 1];
+    e[k] = h * h + (g * g + eps);
+    r[k] = g + (T)c[12] * h;
+  }
+  if constexpr (sizeof(T) == 8) {
+    const U q0 = e[0] * e[0], q1 = e[1] * e[1], q2 = e[2] * e[2];
+    w[0] = q1 * q2;
+    w[1] = q0 * q2;
+    w[2] = q0 * q1;
+  } else {
+    const T b = fmin(fmin(mol_val(e[0]), mol_val(e[1])), mol_val(e[2]));
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const U v = b * mol_rcp(e[k]);
+      w[k] = v * v;
+    }
+  }
+  w[0] = (T)c[14] * w[0];
+  w[1] = (T)c[15] * w[1];
+  w[2] = (T)c[16] * w[2];
+  return (T)c[13] * mol_quot(w[0] * r[0] + (w[1] * r[1] + w[2] * r[2]), w[0] + (w[1] + w[2]));
+}
+
+template <class C>
+__device__ __forceinline__ T mol_weno5_nu3(T u1, T u2, T u3, T u4, T u5, const C& c, T eps) {
+  return mol_weno5_nu3_t<T>(u1, u2, u3, u4, u5, c, eps);
+}
+
+// The gradient with respect to the five values.
+__device__ __noinline__ void mol_weno5_nu3_grad(T u1, T u2, T u3, T u4, T u5, const double* c, T eps, T* g) {
+  const T x[5] = {u1, u2, u3, u4, u5};
+  for (int k = 0; k < 5; ++k) {
+    MolDual d[5];
+    for (int j = 0; j < 5; ++j) d[j] = MolDual{x[j], j == k ? T(1) : T(0)};
+    g[k] = mol_weno5_nu3_t<MolDual>(d[0], d[1], d[2], d[3], d[4], c, eps).d;
+  }
+}
+
+// Row of an axis table as constant memory: along y and z a wave's nodes share the row, and its
+// loads are scalar loads (the kernels never write the tables).
+#ifdef __AMDGCN__
+typedef const __attribute__((address_space(4))) double* MolRow;
+#else
+typedef const double* MolRow;
+#endif
+
+// Column of the tile's table of centred-target coefficients along x (G::nux: MOL_NU3 rows of
+// NUP = TX + 1 values, so that both the copy below and the nodes' reads are free of bank
+// conflicts).  The 17 values of a node lie 448 bytes from its neighbour's in the axis table:
+// read per lane they cost the L1 64 lines per load.
+template <int NUP>
+struct MolCol {
+  const T* p;
+  __device__ __forceinline__ T operator[](const int k) const { return p[k * NUP]; }
+};
+template <class G>
+__device__ __forceinline__ void mol_stage_nux(const int o0, const JPtrs& jp) {
+  if constexpr (G::NUP > 0)
+    for (int e = (int)threadIdx.x; e < G::TX * MOL_NU3; e += G::NTHR) {
+      const int x = e / MOL_NU3, k = e - x * MOL_NU3;
+      G::nux()[k * G::NUP + x] = (T)jp.wtab[0][(i64)MOL_NU_NC * (min(o0 + x, (int)G::UHI0) - 1) + k];
+    }
+}
+
+// One-sided targets (TG = 1, 2, 4, 5 of the stencil x1..x5).  The coordinate-only part of the
+// derivative, MOL_NU_NC values: for each sub-stencil k = 0, 1, 2 the weights of r_k
 // (derivative at the target) and of the interval values pL, pM, pR (first derivative at the left
 // end, midpoint and right end) and pp (second derivative), 15 per sub-stencil; then dx/6, dx,
 // dx^3 of the Simpson smoothness indicator, the split ideal weights dp_k/sgp and dm_k/sgm, and
 // sgp, sgm.  mol_weno5_nu_apply turns them and the five values into the derivative.
-constexpr int MOL_NU_NC = 56;
-
 __device__ __forceinline__ void mol_nu_sub(const double a0, const double a1, const double a2, const double xi,
                                            const double xL, const double xM, const double xph, double* c) {
   double m0[3], t2[3];
@@ -342,8 +446,7 @@ __device__ __forceinline__ void mol_weno5_nu_coefs(const double x1, const double
   if (TG == 1) { xi = x1; xL = x1; xph = (x1 + x2) / 2; }
   else if (TG == 2) { xi = x2; xL = (x1 + x2) / 2; xph = (x2 + x3) / 2; }
   else if (TG == 4) { xi = x4; xL = (x3 + x4) / 2; xph = (x4 + x5) / 2; }
-  else if (TG == 5) { xi = x5; xL = (x4 + x5) / 2; xph = x5; }
-  else { xi = x3; xL = (x2 + x3) / 2; xph = (x3 + x4) / 2; }
+  else { xi = x5; xL = (x4 + x5) / 2; xph = x5; }
   if (TG == 1) {
     d0 = ((2 * x1 - x2 - x3) * (x1 - x4) * (x1 - x5) + (x1 - x3) * (x1 - x5) * (x1 - x2) +
           (x1 - x3) * (x1 - x4) * (x1 - x2)) / ((2 * x1 - x2 - x3) * (x1 - x4) * (x1 - x5));
@@ -354,13 +457,10 @@ __device__ __forceinline__ void mol_weno5_nu_coefs(const double x1, const double
   } else if (TG == 4) {
     d0 = ((-x2 + x4) * (-x3 + x4) * (x4 - x5)) / ((x1 - x4) * (x1 - x5) * (-x2 - x3 + 2 * x4));
     d2 = ((-x1 + x4) * (-x2 + x4)) / ((-x1 + x5) * (-x2 + x5));
-  } else if (TG == 5) {
+  } else {
     d0 = ((-x2 + x5) * (-x3 + x5) * (-x4 + x5)) / ((x1 - x4) * (x1 - x5) * (-x2 - x3 + 2 * x5));
     d2 = ((-x1 - x4 + 2 * x5) * (-x2 + x5) * (-x3 + x5) + (-x1 + x5) * (-x2 - x3 + 2 * x5) * (-x4 + x5)) /
          ((-x1 + x5) * (-x2 + x5) * (-x3 - x4 + 2 * x5));
-  } else {
-    d0 = ((x3 - x4) * (x3 - x5)) / ((x1 - x4) * (x1 - x5));
-    d2 = ((x3 - x1) * (x3 - x2)) / ((x5 - x1) * (x5 - x2));
   }
   const double dx = xph - xL, xM = (xL + xph) / 2;
   mol_nu_sub(x1, x2, x3, xi, xL, xM, xph, c + 0);
@@ -411,20 +511,6 @@ __device__ __forceinline__ U mol_weno5_nu_apply(U u1, U u2, U u3, U u4, U u5, co
   return (T)c[54] * Rp - (T)c[55] * Rm;
 }
 
-template <int TG, class U>
-__device__ __forceinline__ U mol_weno5_nu_t(U u1, U u2, U u3, U u4, U u5, const double x1, const double x2,
-                                            const double x3, const double x4, const double x5, const T eps) {
-  double c[MOL_NU_NC];
-  mol_weno5_nu_coefs<TG>(x1, x2, x3, x4, x5, c);
-  return mol_weno5_nu_apply<U>(u1, u2, u3, u4, u5, c, eps);
-}
-
-template <int TG>
-__device__ __forceinline__ T mol_weno5_nu(T u1, T u2, T u3, T u4, T u5, double x1, double x2, double x3, double x4,
-                                          double x5, T eps) {
-  return mol_weno5_nu_t<TG, T>(u1, u2, u3, u4, u5, x1, x2, x3, x4, x5, eps);
-}
-
 // The FP64 derivative from the coefficients with the normalised nonlinear weights cleared, as
 // in the uniform case: alpha_k / sum_j alpha_j = g_k P_k / sum_j g_j P_j with P_k the product of
 // the other two q_j, so sgp Rp - sgm Rm = (sgp Np Dm - sgm Nm Dp) / (Dp Dm) costs one quotient
@@ -460,18 +546,6 @@ __device__ __forceinline__ double mol_pcoord(const double* x, const int k, const
   return x[k - 1];
 }
 
-// Gradient of the nonuniform WENO5 derivative with respect to its five values.
-template <int TG>
-__device__ __noinline__ void mol_weno5_nu_grad(T u1, T u2, T u3, T u4, T u5, double x1, double x2, double x3,
-                                               double x4, double x5, T eps, T* g) {
-  const T x[5] = {u1, u2, u3, u4, u5};
-  for (int k = 0; k < 5; ++k) {
-    MolDual d[5];
-    for (int j = 0; j < 5; ++j) d[j] = MolDual{x[j], j == k ? T(1) : T(0)};
-    g[k] = mol_weno5_nu_t<TG, MolDual>(d[0], d[1], d[2], d[3], d[4], x1, x2, x3, x4, x5, eps).d;
-  }
-}
-
 // The gradient from a node's row of precomputed coefficients.
 __device__ __noinline__ void mol_weno5_nu_tab_grad(T u1, T u2, T u3, T u4, T u5, const double* c, T eps, T* g) {
   const T x[5] = {u1, u2, u3, u4, u5};
@@ -482,7 +556,7 @@ __device__ __noinline__ void mol_weno5_nu_tab_grad(T u1, T u2, T u3, T u4, T u5,
   }
 }
 
-// Row of coefficients (MOL_NU_NC values) of node i = 1..n of an axis with coordinates x: the
+// Row of coefficients (MOL_NU3 or MOL_NU_NC values) of node i = 1..n of an axis with coordinates x: the
 // stencil and target of the generated code (one-sided at nodes 1, 2, n-1, n of a non-periodic
 // axis, centred elsewhere; periodic images through mol_pcoord).
 __device__ __forceinline__ void mol_weno_nu_row(const double* x, const int n, const bool periodic, const int i,
@@ -507,7 +581,7 @@ __device__ __forceinline__ void mol_weno_nu_row(const double* x, const int n, co
     case 2: mol_weno5_nu_coefs<2>(xs[0], xs[1], xs[2], xs[3], xs[4], c); break;
     case 4: mol_weno5_nu_coefs<4>(xs[0], xs[1], xs[2], xs[3], xs[4], c); break;
     case 5: mol_weno5_nu_coefs<5>(xs[0], xs[1], xs[2], xs[3], xs[4], c); break;
-    default: mol_weno5_nu_coefs<3>(xs[0], xs[1], xs[2], xs[3], xs[4], c); break;
+    default: mol_weno5_nu3_coefs(xs, c); break;
   }
 }
 
@@ -597,6 +671,16 @@ __device__ __forceinline__ void mol_stage_tile(T* L, const int o0, const int o1,
   }
 }
 
+// The value of the wave's first lane in every lane (v is the same in all of them): index
+// arithmetic and table reads along rows become scalar.
+__device__ __forceinline__ int mol_uniform(const int v) {
+#ifdef __AMDGCN__
+  return __builtin_amdgcn_readfirstlane(v);
+#else
+  return v;
+#endif
+}
+
 // Node phase of one staged tile in variant G: each thread runs G::RB consecutive nodes along
 // axis G::BA; their node functions see the same LDS tile at offsets that differ by a constant,
 // so shared taps and subexpressions are loaded and computed once.  Nodes of a ragged tile past
@@ -615,10 +699,14 @@ __device__ __forceinline__ void mol_tile_nodes(const T* L, const int tx, const i
   for (int r = 0; r < (PV + G::NTHR - 1) / G::NTHR; ++r) {
     const int q = (int)threadIdx.x + r * G::NTHR;
     if (PV % G::NTHR != 0 && q >= PV) break;
-    const int lz0 = q / PXY;
+    int lz0 = q / PXY;
     const int rr = q - lz0 * PXY;
-    const int ly0 = rr / PX;
+    int ly0 = rr / PX;
     const int lx = rr - ly0 * PX;
+    if constexpr (PX % 64 == 0 && G::NUP > 0) {   // a wave's nodes lie in one row: scalar table reads
+      ly0 = mol_uniform(ly0);
+      lz0 = mol_uniform(lz0);
+    }
     const int ly = G::BA == 1 ? ly0 * RB : ly0, lz = G::BA == 2 ? lz0 * RB : lz0;
     const int base = (lx + G::HX) + G::EX * (ly + G::HY) + G::EX * G::EY * (lz + G::HZ);
     T out[RB][G::NF];
@@ -684,6 +772,7 @@ __device__ __forceinline__ void mol_full_tile(T* L, const int tx, const int ty, 
   if (G::NST > 0) {
     const int o0 = G::ULO0 + tx * G::TX, o1 = G::ULO1 + ty * G::TY, o2 = G::ULO2 + tz * G::TZ;
     mol_stage_tile<G>(L, o0, o1, o2, mol_stage_mode<G>(tx, ty, tz), t, ep.p, u, jp);
+    mol_stage_nux<G>(o0, jp);
     __syncthreads();
   }
   mol_tile_nodes<G>(L, tx, ty, tz, u, ep, jp, t);
@@ -731,6 +820,7 @@ __device__ __forceinline__ void mol_tiles_persistent(T* L, const T* __restrict__
     if (GB::NST > 0) {
       if (HASC && core) mol_put<GC, NPF, NSR>(L, R);
       else mol_put<GB, NPF, NSR>(L, R);
+      mol_stage_nux<GB>(GB::ULO0 + tx * GB::TX, jp);
       __syncthreads();
     }
     const int kn = k + (int)gridDim.x;

@@ -196,3 +196,31 @@ def test_fused_step_wraps_the_coefficient_rows():
     ref = u + dt / 6 * (k1 + 2 * k2 + 2 * k3 + k4)
     got, _ = genhost.rk4_fused(low, u, 0.0, dt, tile=(16, 1, 1))
     assert np.max(np.abs(got - ref)) <= 1e-14 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("tile", [None, (64, 8, 1), (20, 7, 1), (130, 4, 1)])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_generated_rhs_on_stretched_2d_nodes(periodic, tile):
+    """u_t = -u_x - u_y / 2 on stretched nodes along both axes, line by line against the 1D oracle:
+    coefficient columns of the tile (widths with whole waves, odd, ragged at the box's end), and
+    tiles wider than 128 nodes, which read the axis table."""
+    from molgpu.discretization import MOLFiniteDifference, WENOScheme
+    from molgpu.pdesys import Differential, Eq, Interval, PDESystem, parameters, variables
+    t, x, y = parameters("t x y")
+    u = variables("u")
+    nodes = [systems.stretched_grid(151, 1.0, 3), systems.stretched_grid(38, 1.0, 4)]
+    U = u(t, x, y)
+    eq = Eq(Differential(t)(U), -Differential(x)(U) - 0.5 * Differential(y)(U))
+    if periodic:
+        bcs = [Eq(u(0, x, y), 0.5), Eq(u(t, 0, y), u(t, 1, y)), Eq(u(t, x, 0), u(t, x, 1))]
+    else:
+        bcs = [Eq(u(0, x, y), 0.5), Eq(u(t, 0, y), 0.2), Eq(u(t, 1, y), 0.3), Eq(u(t, x, 0), 0.1), Eq(u(t, x, 1), 0.4)]
+    low = lower(PDESystem([eq], bcs, [Interval(v, 0.0, 1.0) for v in (t, x, y)], [t, x, y], [U]),
+                MOLFiniteDifference({x: nodes[0], y: nodes[1]}, t, advection_scheme=WENOScheme(1e-6)))
+    shape = [h - l + 1 for l, h in zip(low.lo[0], low.hi[0])][::-1]
+    v = np.random.default_rng(5).uniform(0.0, 1.0, shape)
+    got = genhost.rhs(low, v.reshape(-1), tile=tile).reshape(shape)
+    ref = np.stack([orc.weno_nu1d_rhs(nodes[0], 1.0, 1e-6, periodic, 0.2, 0.3, row) for row in v])
+    ref = ref + np.stack([orc.weno_nu1d_rhs(nodes[1], 0.5, 1e-6, periodic, 0.1, 0.4, np.ascontiguousarray(col))
+                          for col in v.T]).T
+    assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(ref))
