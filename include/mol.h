@@ -268,9 +268,10 @@ typedef enum { MOL_FLAG_KAHAN = 1, MOL_FLAG_GRAPH = 2, MOL_FLAG_UNFUSED = 4 } mo
  * mol_set_aux, mol_set_tile and mol_destroy, and all of them when more than eight keys are in
  * use (that drop waits for the device).  A 1D system held by one resident tile runs up to 1024
  * steps per launch and is launched directly.
- * Periodic 1D/2D systems of reach 1 run RK4 (without Kahan) as one fused launch per step (the
- * four stages on a tile with a 4-node halo, same arithmetic as the stage launches);
- * MOL_FLAG_UNFUSED runs the four stage launches instead. */
+ * 1D/2D systems of reach 1 (2 on periodic axes) run RK4 as one fused launch per step, with the
+ * arithmetic of the stage launches: on tiles with a 4-reach halo, or swept along y in registers
+ * (2D systems and batches of reach 1; also with MOL_FLAG_KAHAN).  MOL_FLAG_UNFUSED runs the four
+ * stage launches instead. */
 int mol_integrate(mol_handle* h, void* u, const void* p, double t0, double dt, int64_t nsteps,
                   int32_t scheme, int32_t flags, void* stream);
 

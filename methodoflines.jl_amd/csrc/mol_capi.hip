@@ -113,7 +113,7 @@ void free_handle(mol_handle* h) {
                   h->d_prog, h->d_coord[0], h->d_coord[1], h->d_coord[2], h->w_y1,
                   h->w_y2, h->w_acc, h->w_comp, h->d_tnow, h->d_ka64, h->d_ka32, h->d_tiles,
                   h->ck_u, h->ck_t, h->seg_u, h->seg_t, h->adj_y[0], h->adj_y[1], h->adj_y[2], h->adj_y[3],
-                  h->d_insts, h->d_wl, h->d_bdata, h->vjp_bf, h->vjp_ba, h->r_u, h->r_du, h->r_p,
+                  h->d_insts, h->d_wl, h->d_swl, h->d_bdata, h->vjp_bf, h->vjp_ba, h->r_u, h->r_du, h->r_p,
                   h->d_norm_part, h->d_wtab[0], h->d_wtab[1], h->d_wtab[2]};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -793,19 +793,72 @@ int build_wenonu_tables(mol_handle* h, const mol_desc* d, const std::string& src
   return 0;
 }
 
+// Rows per strip of the register sweep over `box`es of (rows, column windows): one box, or the
+// instances of a batch; `bytes` of state per node.  A wave evaluates its strip's rows and the
+// equivalent of three more.  With k waves per SIMD an iteration takes the issue time of k waves
+// and a fixed part (latencies and scalar instructions a wave cannot hide) once per round of the
+// waves that fit at once: cost = (rows + 3) (k + O ceil(k / w)), O and w from the registers and
+// arithmetic per node, which grow with its bytes.  Measured, us per step: Brusselator FP64 1501^2
+// with strips of 41 / 22 / 16 / 8 rows (k = 1, 2, 3, 5) 22.6 / 20.6 / 22.5 / 21.6; diffusion-reaction
+// FP32 + Kahan 3000^2 with 82 / 32 / 16 rows (k = 2, 5, 10) 42.9 / 32.3 / 32.0.
+// MOL_SWEEP_ROWS overrides.
+int sweep_rows(int device, int bytes, const std::vector<std::pair<int, int>>& box) {
+  if (const char* e = std::getenv("MOL_SWEEP_ROWS")) return std::max(4, std::atoi(e));
+  int ncu = 0, top = 4;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0) ncu = 256;
+  for (const auto& b : box) top = std::max(top, b.first);
+  const int64_t w = std::max(1, 32 / bytes);
+  const double fixed = std::min(1.5, 8.0 / bytes);
+  int best = top;
+  double cost = 1e300;
+  for (int rows = 4; rows <= top; ++rows) {
+    int64_t waves = 0;
+    for (const auto& b : box) waves += (int64_t)b.second * ((b.first + rows - 1) / rows);
+    const int64_t k = (waves + 4 * ncu - 1) / (4 * ncu);
+    const double c = (rows + 3) * ((double)k + fixed * (double)((k + w - 1) / w));
+    if (c < cost) {
+      cost = c;
+      best = rows;
+    }
+  }
+  return best;
+}
+
+// The fused step of a 2D system of reach one whose tiles outnumber the compute units is a register
+// sweep where the system has one (jit_sweep_source).  MOL_SWEEP=0 or 1 overrides the size rule.
+bool sweep_source(mol_handle* h, const mol_desc* d, JitGeom& g, std::string& src) {
+  if (d->ndim != 2 || h->tile_req[0] > 0 || std::getenv("MOL_FUSED_TILE") || std::getenv("MOL_FUSED_STEPS")) return false;
+  const char* e = std::getenv("MOL_SWEEP");
+  if (e ? e[0] == '0' : g.fsteps != 1) return false;
+  JitGeom gs = g;
+  const int nw = sweep_windows(d->periodic[0], g.uhi[0] - g.ulo[0] + 1);
+  gs.sweep_h = sweep_rows(h->device, d->nfields * (int)h->esize(), {{g.uhi[1] - g.ulo[1] + 1, nw}});
+  std::string err;
+  src = jit_sweep_source(d, gs, err);
+  if (src.empty()) return false;
+  g = gs;
+  g.nthr = 64;
+  g.fsteps = 1;
+  g.ntile[0] = nw;
+  g.ntile[1] = (g.uhi[1] - g.ulo[1] + 1 + g.sweep_h - 1) / g.sweep_h;
+  return true;
+}
+
 void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, const KCore<double>& kc, int ncore) {
-  h->fused_fn = nullptr;
+  h->fused_fn = h->fused_kahan_fn = nullptr;
   h->fused_tiles = 0;
   h->fused_reason.clear();
   const char* e = std::getenv("MOL_FUSED");
   if (e && e[0] == '0') { h->fused_reason = "disabled (MOL_FUSED=0)"; return; }
   JitGeom g;
   if (!fused_geometry(h, d, ka, kc, ncore, g, h->fused_reason)) return;
-  std::string err;
-  const std::string src = jit_fused_source(d, g, err);
+  std::string err, src;
+  const bool sweep = sweep_source(h, d, g, src);
+  if (!sweep) src = jit_fused_source(d, g, err);
   if (src.empty()) { h->fused_reason = err; return; }
-  if (jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
-    h->fused_fn = nullptr;
+  if (jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err) ||
+      (sweep && jit_kernel(src, "mol_rk4_fused_kahan", h->device, &h->fused_kahan_fn, err))) {
+    h->fused_fn = h->fused_kahan_fn = nullptr;
     h->fused_reason = err;
     return;
   }
@@ -933,15 +986,21 @@ Work handle_work(const mol_handle* h) { return Work{h->w_y1, h->w_y2, h->w_acc, 
 
 // t0v: the start time, passed by value to the first fused launch instead of read from the
 // device clock (which that launch then sets for the next); null: the clock holds it.
+// comp_zero: the first fused launch takes the compensation as zero instead of reading it.
+// RK4 runs as fused launches (the compensated update only where the fused kernel has it).
+bool use_fused(const mol_handle* h, int scheme, bool kahan) {
+  return scheme == MOL_RK4 && (kahan ? h->fused_kahan_fn : h->fused_fn) && !h->no_fuse;
+}
+
 template <typename T>
 int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int64_t nsteps, int scheme,
-                  bool kahan, hipStream_t s, const double* t0v = nullptr) {
+                  bool kahan, hipStream_t s, const double* t0v = nullptr, bool comp_zero = false) {
   const Launch<T> L = launch_of<T>(h);
   T* y1 = (T*)w.y1;
   T* y2 = (T*)w.y2;
   T* acc = (T*)w.acc;
   T* comp = (T*)w.comp;
-  if (scheme == MOL_RK4 && !kahan && h->fused_fn && !h->no_fuse) {
+  if (use_fused(h, scheme, kahan)) {
     // one launch per step (or per chunk of resident steps), the state alternating between u
     // and the workspace
     T* src = u;
@@ -954,6 +1013,11 @@ int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int
       e.tnext = w.tnow + (1 - h->clk);
       e.tadv = dt;
       e.p = p;
+      if (kahan) {
+        e.mode = 2;
+        e.comp = comp;
+        e.subA = comp_zero && step == 0;   // nothing to read yet
+      }
       if (t0v && step == 0 && !h->fused_resident) {
         e.tnow = nullptr;
         e.tofs = *t0v;
@@ -961,8 +1025,12 @@ int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int
       JitPtrs<T> jp = L.jp;
       const T* sp = src;
       int ns = nsub;
-      void* args[] = {(void*)&sp, (void*)&dst, (void*)&e, (void*)&jp, (void*)&ns};
-      if (hipModuleLaunchKernel(h->fused_fn, h->fused_tiles, 1, 1, h->fused_nthr, 1, 1, 0, s, args, nullptr) !=
+      const BInst* insts = L.insts;
+      const int32_t* swl = (const int32_t*)h->d_swl;
+      void* args1[] = {(void*)&sp, (void*)&dst, (void*)&e, (void*)&jp, (void*)&ns};
+      void* argsb[] = {(void*)&sp, (void*)&dst, (void*)&e, (void*)&insts, (void*)&swl};
+      void** args = h->batch ? argsb : args1;
+      if (hipModuleLaunchKernel(kahan ? h->fused_kahan_fn : h->fused_fn, h->fused_tiles, 1, 1, h->fused_nthr, 1, 1, 0, s, args, nullptr) !=
           hipSuccess)
         return fail(h, MOL_ERR_HIP, "fused RK4 launch failed");
       h->clk ^= 1;
@@ -1049,12 +1117,12 @@ int integrate_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int64_
   h->clk = 0;
   // a resident fused kernel already runs up to 1024 steps per launch and flips the clock once
   // per launch, whatever the step count: it is launched directly
-  const bool fused = scheme == MOL_RK4 && !kahan && h->fused_fn && !h->no_fuse;
+  const bool fused = use_fused(h, scheme, kahan);
   const bool resident = fused && h->fused_resident;
   const bool direct = !(flags & MOL_FLAG_GRAPH) || resident || nsteps < kGraphChunks[2];
   // direct fused steps take the start time by value in their first launch: no clock launch
   if (direct && fused && !resident && nsteps > 0)
-    return enqueue_steps<T>(h, handle_work(h), u, p, dt, nsteps, scheme, kahan, s, &t0);
+    return enqueue_steps<T>(h, handle_work(h), u, p, dt, nsteps, scheme, kahan, s, &t0, true);
   if (launch_set_clock(h->d_tnow, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
   if (kahan && launch_fill_zero<T>((T*)h->w_comp, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
   if (direct) return enqueue_steps<T>(h, handle_work(h), u, p, dt, nsteps, scheme, kahan, s);
@@ -1092,11 +1160,11 @@ int integrate_noalloc_impl(mol_handle* h, T* u, const T* p, double t0, double dt
   if (!base) return fail(h, MOL_ERR_HIP, err);
   const bool kahan = (flags & MOL_FLAG_KAHAN) != 0;
   h->no_fuse = (flags & MOL_FLAG_UNFUSED) != 0;
-  const bool fused = scheme == MOL_RK4 && !kahan && h->fused_fn && !h->no_fuse;
+  const bool fused = use_fused(h, scheme, kahan);
   // stage vectors each path touches: fused RK4 y1; RK4 stage launches y1, y2, acc; SSPRK33 y1,
   // y2; Kahan adds the compensation
   const size_t vb = ((size_t)h->nunk * sizeof(T) + 255) / 256 * 256;
-  const int narr = fused ? 1 : (scheme == MOL_RK4 ? 3 : 2) + (kahan ? 1 : 0);
+  const int narr = (fused ? 1 : scheme == MOL_RK4 ? 3 : 2) + (kahan ? 1 : 0);
   const size_t need = 256 + (size_t)narr * vb;
   if (need > (size_t)MOL_NOALLOC_SCRATCH_BYTES)
     return fail(h, MOL_ERR_SHAPE, "mol_integrate_noalloc: this integration needs " + std::to_string(need) +
@@ -1109,8 +1177,8 @@ int integrate_noalloc_impl(mol_handle* h, T* u, const T* p, double t0, double dt
   if (!fused) {
     w.y2 = q + vb;
     if (scheme == MOL_RK4) w.acc = q + 2 * vb;
-    if (kahan) w.comp = q + (size_t)(narr - 1) * vb;
   }
+  if (kahan) w.comp = q + (size_t)(narr - 1) * vb;
   h->clk = 0;
   if (launch_set_clock(w.tnow, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
   if (kahan && launch_fill_zero<T>((T*)w.comp, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
@@ -1474,6 +1542,8 @@ struct BatchPlan {
   int nclasses = 0;
   int tile[3] = {1, 1, 1};
   std::string src;
+  std::vector<int32_t> sweep;   // register sweep of a whole RK4 step: per wave instance, class and
+                                // window, first row, end row; empty when an instance does not qualify
 };
 
 int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t ninst, const int32_t* tile,
@@ -1491,8 +1561,11 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
       return fail(nullptr, MOL_ERR_INVALID, "parameter values of instance " + std::to_string(i) + " missing");
   }
   const size_t esize = ds[0]->dtype == MOL_F64 ? sizeof(double) : sizeof(float);
-  std::map<std::string, int> cls_of;
-  std::vector<std::string> cls_src;
+  std::map<std::string, int> cls_of, sw_of;
+  std::vector<std::string> cls_src, sw_src;
+  std::vector<int> sw_cls(ninst, 0);
+  const char* se = std::getenv("MOL_SWEEP");
+  bool sweep = !(se && se[0] == '0');
   P.hdr.assign(ninst, BInst{});
   P.dofs.assign(ninst, {});
   int ldsn = 1;
@@ -1523,8 +1596,24 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
     } else {
       cls = it->second;
     }
+    if (sweep) {
+      const std::string ss = jit_sweep_class(d, geom_of(ka, th.kc64, ncore), "SwpY", err);
+      sweep = !ss.empty();
+      if (sweep) {
+        const auto sit = sw_of.emplace(ss, (int)sw_src.size());
+        if (sit.second) sw_src.push_back(ss);
+        sw_cls[i] = sit.first->second;
+      }
+    }
     BInst& b = P.hdr[i];
     std::memset(&b, 0, sizeof(b));
+    for (int k = 0; k < d->nclosures; ++k) {
+      const mol_closure& cl = d->closures_h[k];
+      if (cl.axis > 1 || cl.K > 2) continue;
+      double* gv = b.g[cl.field][2 * cl.axis + cl.side];
+      for (int m = 0; m < cl.K; ++m) gv[m] = d->pool_h[cl.wC + m];
+      gv[2] = cl.gprog >= 0 ? d->pool_h[cl.wc] : 0.0;
+    }
     for (int a = 0; a < 3; ++a) {
       b.n[a] = ka.n[a];
       b.ulo[a] = ka.ulo[a];
@@ -1630,6 +1719,59 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
   for (size_t c = 0; c < cls_src.size(); ++c)
     src << "    case " << c << ": mol_batch_tile<Geo" << c << ">(L, hd, tile, u, ep, t); break;\n";
   src << "    default: break;\n    }\n  }\n}\n";
+  if (sweep) {
+    // a whole RK4 step per launch: a wave per window and strip of an instance, longest first
+    const int nf = ds[0]->nfields;
+    std::vector<std::pair<int, int>> box;
+    for (const BInst& b : P.hdr)
+      box.push_back({b.uhi[1] - b.ulo[1] + 1, sweep_windows(ds[0]->periodic[0], b.uhi[0] - b.ulo[0] + 1)});
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const int rows = sweep_rows(dev, nf * (int)esize, box);
+    std::vector<std::array<int32_t, 4>> items;
+    for (int i = 0; i < ninst; ++i) {
+      // strips of an instance as even as whole rows allow, four rows or more
+      const int ny = box[i].first, ns = std::min((ny + rows - 1) / rows, ny / 4);
+      for (int s = 0; s < ns; ++s)
+        for (int w = 0; w < box[i].second; ++w)
+          items.push_back({i, sw_cls[i] + 65536 * w, (int)((int64_t)ny * s / ns), (int)((int64_t)ny * (s + 1) / ns)});
+    }
+    std::stable_sort(items.begin(), items.end(), [](const std::array<int32_t, 4>& a, const std::array<int32_t, 4>& b) {
+      return a[3] - a[2] > b[3] - b[2];
+    });
+    for (const auto& it : items) P.sweep.insert(P.sweep.end(), it.begin(), it.end());
+    for (size_t c = 0; c < sw_src.size(); ++c) {
+      std::string body = sw_src[c];
+      const std::string from = "struct SwpY {";
+      body.replace(body.find(from), from.size(), "struct SwpY" + std::to_string(c) + " {");
+      src << body;
+    }
+    // two kernels: the compensated update's registers would cost the plain one occupancy
+    for (const char* kahan : {"false", "true"}) {
+      src << "extern \"C\" __global__ void __launch_bounds__(64) mol_batch_rk4" << (kahan[0] == 't' ? "_kahan" : "")
+          << "(const T* __restrict__ u, T* __restrict__ unew,\n"
+             "    Epi ep, const BInst* __restrict__ insts, const int* __restrict__ wl) {\n"
+             "  const double t = ep.tnow ? ep.tnow[0] : ep.tofs;\n"
+             "  if (ep.tnext && blockIdx.x == 0 && threadIdx.x == 0) ep.tnext[0] = t + ep.tadv;\n"
+             "  const int* const it = wl + 4 * blockIdx.x;\n"
+             "  const BInst& in = insts[it[0]];\n"
+          << "  constexpr int NF = " << nf << ";\n"
+          << "  MolSHdr<NF> hd;\n  MolSweep<NF> g;\n  JPtrs jp{};\n"
+             "  for (int a = 0; a < 3; ++a) {\n    hd.n[a] = in.n[a];\n    jp.coord[a] = in.coord[a];\n  }\n"
+             "  hd.W = (MolRow)in.W;\n  hd.K = (MolRow)in.K;\n"
+             "  for (int f = 0; f < NF; ++f) {\n    g.fofs[f] = in.fofs[f];\n"
+             "    for (int s = 0; s < 4; ++s)\n      for (int m = 0; m < 3; ++m) hd.g[f][s][m] = (T)in.g[f][s][m];\n  }\n"
+             "  g.nx = in.uhi[0] - in.ulo[0] + 1;\n  g.ny = in.uhi[1] - in.ulo[1] + 1;\n"
+             "  g.lo0 = in.ulo[0];\n  g.lo1 = in.ulo[1];\n  g.lo2 = 1;\n  g.y0 = it[2];\n  g.y1 = it[3];\n"
+             "  const int cls = it[1] & 0xffff, w = it[1] >> 16;\n";
+      for (size_t c = 0; c < sw_src.size(); ++c) {
+        const std::string G = "SwpY" + std::to_string(c);
+        src << "  if (cls == " << c << ") {\n    mol_sweep_window<" << G << "::PER0 != 0, " << G << "::CX>(g, w);\n"
+            << "    mol_rk4_sweep<" << G << ", " << kahan << ">(hd, g, u, unew, ep, jp, t);\n  }\n";
+      }
+      src << "}\n";
+    }
+  }
   P.src = src.str();
   return 0;
 }
@@ -1663,6 +1805,7 @@ int create_batched(const mol_desc* const* ds, const double* const* params, int32
   }
   r |= upload(h, &h->d_insts, P.hdr.data(), P.hdr.size());
   r |= upload(h, &h->d_wl, P.wl.data(), P.wl.size());
+  r |= upload(h, &h->d_swl, P.sweep.data(), P.sweep.size());
   if (r) {
     set_global_error(h->err);
     free_handle(h);
@@ -1673,6 +1816,16 @@ int create_batched(const mol_desc* const* ds, const double* const* params, int32
     set_global_error("batched kernel: " + err);
     free_handle(h);
     return MOL_ERR_HIP;
+  }
+  if (!P.sweep.empty()) {
+    if (jit_kernel(P.src, "mol_batch_rk4", h->device, &h->fused_fn, err) ||
+        jit_kernel(P.src, "mol_batch_rk4_kahan", h->device, &h->fused_kahan_fn, err)) {
+      set_global_error("batched kernel: " + err);
+      free_handle(h);
+      return MOL_ERR_HIP;
+    }
+    h->fused_tiles = (int)(P.sweep.size() / 4);
+    h->fused_nthr = 64;
   }
   h->batch_grid = std::min(h->nwork, 1 << 24);
   *out = h;
@@ -2021,7 +2174,8 @@ int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t b
   std::string src;
   if (flags & MOL_CODEGEN_FUSED) {
     JitGeom g;
-    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err)) src = jit_fused_source(d, g, err);
+    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, g, src))
+      src = jit_fused_source(d, g, err);
   } else {
     src = (flags & MOL_CODEGEN_VJP) ? jit_vjp_source(d, vjp_geometry(&tmp, d, nullptr), err)
                                     : jit_source(d, fwd_geom(tmp, ncore), err);

@@ -19,6 +19,7 @@ struct JitGeom {
   int ct_lo[3], ct_n[3], ncore;                       // core tiles (interior rows only)
   int nthr;                                           // threads per work-group (multiple of 64)
   int fsteps = 1;                                     // fused RK4: steps per launch (1 or 2)
+  int sweep_h = 0;                                    // fused RK4 as a register sweep: rows per strip
 };
 
 // Pointer arguments of the generated kernel (layout identical to JPtrs of mol_jit_prelude.h).
@@ -39,6 +40,14 @@ std::string jit_fused_source(const mol_desc* d, const JitGeom& g, std::string& e
 // kernel: the arrays it stages (and their adjoints); 0 when the system cannot be generated.
 size_t jit_lds_per_pos(const mol_desc* d, const JitGeom& g, size_t esize, bool vjp);
 std::string jit_class_source(const mol_desc* d, const JitGeom& g, const std::string& name, std::string& err);
+// RK4 step swept along y in registers: the kernel of one system, or the class body of batched
+// instances; empty when the system does not qualify.
+std::string jit_sweep_source(const mol_desc* d, const JitGeom& g, std::string& err);
+std::string jit_sweep_class(const mol_desc* d, const JitGeom& g, const std::string& name, std::string& err);
+// Windows of columns over an axis of n unknowns (mol_sweep_windows of mol_jit_prelude.h).
+inline int sweep_windows(bool per, int n) {
+  return per ? (n + 55) / 56 : (n <= 64 ? 1 : (n - 8 + 55) / 56);
+}
 
 // Header of one instance of a batch (layout identical to BInst of mol_jit_prelude.h).
 struct BInst {
@@ -53,6 +62,7 @@ struct BInst {
   const double* coord[3];
   const double* W;
   const double* K;
+  double g[MOL_MAX_FIELDS][4][3];   // ghost next to each side of the first two axes (register sweep)
 };
 int jit_compile(const std::string& src, std::vector<char>& code, std::string& log);
 int jit_kernel(const std::string& src, const char* name, int device, hipFunction_t* fn, std::string& err);
@@ -187,6 +197,7 @@ struct mol_handle {
   int batch_tile[3] = {0, 0, 0};
   void* d_insts = nullptr;
   void* d_wl = nullptr;
+  void* d_swl = nullptr;                  // wave list of the batch's RK4 register sweep
   void* d_bdata = nullptr;                // weights, constants and coordinates of all instances
   std::vector<int64_t> inst_off;          // first unknown of each instance
   int jit_grid = 0;                       // work-groups of the persistent generated RHS kernel
@@ -196,6 +207,7 @@ struct mol_handle {
   int fused_nthr = 256;
   bool fused_resident = false;     // one 1D tile: many steps per fused launch
   int fused_steps = 1;             // steps per fused launch otherwise (1, or 2 with an 8-reach halo)
+  hipFunction_t fused_kahan_fn = nullptr;   // its compensated update (register sweep only)
   std::string fused_reason;               // why there is no fused kernel
   bool no_fuse = false;                   // this integration runs the stage kernels (MOL_FLAG_UNFUSED)
   int vjp_nthr = 256;                     // threads per work-group of the generated VJP kernel

@@ -119,6 +119,13 @@ class Gen {
   // Parametric class body for batched instances: weights, constants, grid sizes and boxes are
   // read from the instance header `hd`; the text is identical for instances of one structure.
   std::string source_class(const std::string& name);
+  // RK4 step swept along y in registers (mol_rk4_sweep): 2D, reach one, cross-shaped taps
+  std::string source_sweep(bool f64);
+  std::string sweep_class(const std::string& name);
+  std::string sweep_class_of(const std::string& name) {   // parametric, for batched instances
+    param_ = true;
+    return sweep_class(name);
+  }
   std::string error;
 
  private:
@@ -134,6 +141,7 @@ class Gen {
   bool param_ = false;                // parametric (batched) printing
   bool fused_ = false;                // fused RK4 step printing (coordinates from LDS)
   bool vjp_ = false;                  // reverse-mode kernel printing
+  bool sweep_ = false;                // register sweep printing (window in registers, constant-memory reads)
   bool stage_noif_ = false;           // printing stage_ni (interface sides read nothing)
   // printing overrides: nodes not printed, and nodes referenced by another expression
   std::vector<char> skip_;
@@ -300,6 +308,7 @@ class Gen {
     // fused step kernel: coordinates of the tile + halo staged in LDS, indexed by the
     // unwrapped node index relative to the first staged position
     if (fused_) return "(T)mol_fc[" + istr(d) + "][I" + istr(d) + " - mol_fo[" + istr(d) + "]]";
+    if (sweep_) return "(T)((MolRow)jp.coord[" + istr(d) + "])[I" + istr(d) + " - 1]";
     return "(T)jp.coord[" + istr(d) + "][I" + istr(d) + " - 1]";
   }
   std::string coord_tap(int d, int off) const {
@@ -547,7 +556,7 @@ int Gen::leaf(uint32_t code, int imm, const Ctx& c) {
     case MOL_OP_PARAM:
       // batched instances carry their parameter values after the constants, eps and 1/dx
       if (param_) return expr("(T)hd.K[" + istr(d_->ncpool + 2LL * d_->nslots + imm) + "]");
-      return expr("P[" + istr(imm) + "]");
+      return expr((sweep_ ? "((MolPar)P)[" : "P[") + istr(imm) + "]");
     default: break;
   }
   if (c.kind == CTX_BOUNDARY) {
@@ -1042,6 +1051,8 @@ std::string Gen::ref(int id) const {
         if (n.arr < d_->nfields) return "u[" + UIDX(n.arr, "I0", "I1", "I2") + "]";
         return "jp.aux[" + istr(n.arr - d_->nfields) + "][gidx(I0, I1, I2)]";
       }
+      if (sweep_)
+        return "L[b + " + istr(sl) + " * VOL + " + istr(n.dv[0]) + " + " + istr(n.dv[1]) + " * EX]";
       const long long o = (long long)sl * pg_.vol + n.dv[0] + (long long)pg_.ext[0] * (n.dv[1] + (long long)pg_.ext[1] * n.dv[2]);
       if (o == 0) return "L[b]";
       return o > 0 ? "L[b + " + istr(o) + "]" : "L[b - " + istr(-o) + "]";
@@ -1602,7 +1613,9 @@ std::vector<int> Gen::invariant_frontier(int r, const std::vector<int>& outs, st
     if (!used[id] || !inv[id]) continue;
     const Node& n = nodes_[id];
     if (n.kind == N_LIT) continue;
-    if (n.kind == N_EXPR && n.text.compare(0, 2, "P[") == 0) continue;
+    if (n.kind == N_EXPR && (n.text.compare(0, 2, "P[") == 0 || n.text.compare(0, 9, "((MolPar)") == 0 ||
+                             n.text.compare(0, 6, "(T)hd.") == 0))
+      continue;
     if (n.kind == N_OP && std::find(regs_[r].nodes.begin(), regs_[r].nodes.end(), (int)id) == regs_[r].nodes.end())
       continue;
     front.push_back((int)id);
@@ -2129,6 +2142,154 @@ std::string Gen::source_class(const std::string& name) {
   return o.str();
 }
 
+// Class body of the register sweep: window geometry, ghosts next to the four sides, node function
+// and its node-invariant part.  Empty when the system does not qualify.
+std::string Gen::sweep_class(const std::string& name) {
+  sweep_ = true;
+  if (d_->ndim != 2) { bad("register sweep: not a 2D system"); return ""; }
+  for (int f = 1; f < d_->nfields; ++f)
+    for (int a = 0; a < 3; ++a)
+      if (d_->lo[f][a] != d_->lo[0][a] || d_->hi[f][a] != d_->hi[0][a]) { bad("register sweep: unequal unknown boxes"); return ""; }
+  for (int a = 0; a < 2; ++a)
+    if (d_->hi[0][a] - d_->lo[0][a] + 1 < 8) { bad("register sweep: box narrower than 8 nodes"); return ""; }
+  for (int c = 0; c < d_->nclosures; ++c) {
+    // the ghost next to a side is combined from the two nodes next to it, which the sweep holds
+    const mol_closure& cl = d_->closures_h[c];
+    if (cl.src >= 0 || cl.K > 2) { bad("register sweep: boundary closure over more than two nodes"); return ""; }
+  }
+  bool allper = true;
+  for (int a = 0; a < d_->ndim; ++a) allper = allper && d_->periodic[a];
+  std::vector<int> outs;
+  int region = -1;
+  build_node(allper, outs, region);
+  if (!ok_) return "";
+  for (size_t id = 0; id < nodes_.size(); ++id) {
+    if (!live_[id]) continue;
+    if (nodes_[id].kind == N_BRANCH) { bad("register sweep: boundary rows"); return ""; }
+    if (nodes_[id].kind == N_OP && (nodes_[id].op == X_WENO || nodes_[id].op == X_WENONU)) { bad("register sweep: WENO5"); return ""; }
+  }
+  Usage us = usage();
+  if (!us.separable || us.reach[0] > 1 || us.reach[1] > 1) { bad("register sweep: reach above one or diagonal taps"); return ""; }
+  for (int k = d_->nfields; k < d_->nfields + d_->naux; ++k)
+    if (us.staged[k]) { bad("register sweep: a grid field read away from the node"); return ""; }
+  for (int f = 0; f < d_->nfields; ++f) us.staged[f] = true;
+  const int halo[3] = {1, 1, 0};
+  pg_ = make_pg(halo, us);
+  std::ostringstream o;
+  o << "struct " << name << (param_ ? " {\n" : " : GeoBase {\n");
+  auto c = [&](const std::string& nm, const std::string& v) { o << "  static constexpr int " << nm << " = " << v << ";\n"; };
+  if (param_) {
+    c("NF", istr(d_->nfields));
+    c("PER0", istr(d_->periodic[0]));
+    c("PER1", istr(d_->periodic[1]));
+    c("CX", "1");
+  } else {
+    // off the GPU one lane holds a whole row
+    c("CX", "MOL_WAVE == 64 ? 1 : " +
+                istr(g_.hi[0][0] - g_.lo[0][0] + 1 + (g_.periodic[0] ? 8 : 0)));
+  }
+  c("EX", "CX + 2");
+  c("VOL", "3 * EX");
+  const std::string hdt = param_ ? "const MolSHdr<NF>& hd" : "const MolNoHdr& hd";
+  // ghosts: sides x low, x high, y low, y high
+  o << "  static __device__ __forceinline__ T ghost(" << hdt << ", const int f, const int side, const T y0, const T y1,\n"
+       "      const int p0, const int p1, const int p2, const double t, const T* __restrict__ P, const JPtrs& jp) {\n"
+       "    (void)hd; (void)y0; (void)y1; (void)p0; (void)p1; (void)p2; (void)t; (void)P; (void)jp;\n"
+       "    switch (f * 4 + side) {\n";
+  for (int k = 0; k < d_->nclosures; ++k) {
+    const mol_closure& cl = d_->closures_h[k];
+    const int side = 2 * cl.axis + cl.side;
+    o << "    case " << cl.field * 4 + side << ": {\n";
+    std::string G;
+    if (cl.gprog >= 0) {
+      const int r = new_region();
+      cur_ = r;
+      Ctx bc;
+      bc.kind = CTX_BOUNDARY;
+      bc.ax = cl.axis;
+      bc.side = cl.side;
+      regs_[r].result = prog(cl.gprog, bc);
+      print_region(o, r);
+      G = ref(regs_[r].result);
+    }
+    std::string e;
+    auto term = [&](int m, double w, const std::string& x) {
+      if (!param_ && w == 0.0) return;
+      const std::string tw = param_ ? "hd.g[f][side][" + istr(m) + "]" : lit(w);
+      e += (e.empty() ? "" : " + ") + tw + " * " + x;
+    };
+    for (int m = 0; m < (param_ ? 2 : cl.K); ++m) term(m, param_ ? 1.0 : d_->pool_h[cl.wC + m], m == 0 ? "y0" : "y1");
+    if (cl.gprog >= 0) term(2, param_ ? 1.0 : d_->pool_h[cl.wc], G);
+    o << "    return " << (e.empty() ? "T(0)" : e) << ";\n    }\n";
+  }
+  o << "    default: return T(0);\n    }\n  }\n";
+  std::vector<char> inv;
+  std::vector<int> front = invariant_frontier(region, outs, inv);
+  // carried for four rows of every column: not worth the registers beyond a few values
+  if (front.size() > 4) front.clear();
+  c("NINV", istr((long long)front.size()));
+  const std::string args = "const int I0, const int I1, const int I2";
+  if (!front.empty()) {
+    o << "  static __device__ __forceinline__ void node_inv(" << hdt << ", " << args << ",\n"
+         "      const T* __restrict__ P, const JPtrs& jp, T* inv) {\n"
+         "    (void)hd; (void)I0; (void)I1; (void)I2; (void)P; (void)jp;\n";
+    for (int id : regs_[region].nodes)
+      if (nodes_[id].kind == N_OP && inv[id]) print_node(o, id);
+    for (size_t k = 0; k < front.size(); ++k) o << "    inv[" << k << "] = " << ref(front[k]) << ";\n";
+    o << "  }\n";
+    skip_.assign(nodes_.size(), 0);
+    for (int id : regs_[region].nodes)
+      if (nodes_[id].kind == N_OP && inv[id]) skip_[id] = 1;
+    for (size_t k = 0; k < front.size(); ++k) subst_[front[k]] = "inv[" + istr((long long)k) + "]";
+  }
+  o << "  static __device__ __forceinline__ void node(" << hdt << ", const T* L, const int b, " << args << ",\n"
+       "      const double t, const T* __restrict__ P, const JPtrs& jp, const T* inv, T* out) {\n"
+       "    (void)hd; (void)I0; (void)I1; (void)I2; (void)t; (void)P; (void)jp; (void)L; (void)b; (void)inv;\n";
+  print_region(o, region);
+  for (int f = 0; f < d_->nfields; ++f) o << "    out[" << f << "] = " << ref(outs[f]) << ";\n";
+  skip_.clear();
+  subst_.clear();
+  o << "  }\n};\n\n";
+  return o.str();
+}
+
+// The register sweep of one system as the fused step kernel: a wave per window and strip.
+std::string Gen::source_sweep(bool f64) {
+  const std::string body = sweep_class("SwpS");
+  if (!ok_ || g_.sweep_h < 1) return "";
+  const int nx = g_.hi[0][0] - g_.lo[0][0] + 1, ny = g_.hi[0][1] - g_.lo[0][1] + 1;
+  const int ns = (ny + g_.sweep_h - 1) / g_.sweep_h, nw = sweep_windows(g_.periodic[0], nx);
+  for (int a = 0; a < 3; ++a) g_.tile[a] = g_.ntile[a] = 1;
+  g_.ntile[0] = nw;
+  g_.ntile[1] = ns;
+  std::ostringstream o;
+  o << "// generated fused RK4 step of one PDE system (register sweep)\n#define MOL_T " << (f64 ? "double" : "float")
+    << "\n#include \"mol_jit_prelude.h\"\n\n" << layout_asserts(f64);
+  g_.nthr = 64;
+  o << "struct GeoBase {\n" << geo_common() << "};\n\n" << body;
+  // two kernels: the compensated update's registers would cost the plain one occupancy
+  for (const char* kahan : {"false", "true"}) {
+    o << "extern \"C\" __global__ void __launch_bounds__(64) mol_rk4_fused" << (kahan[0] == 't' ? "_kahan" : "")
+      << "(const T* __restrict__ u, T* __restrict__ unew,\n"
+         "    Epi ep, JPtrs jp, int nsub) {\n"
+         "  (void)nsub;\n"
+         "  const double t = ep.tnow ? ep.tnow[0] : ep.tofs;\n"
+         "  if (ep.tnext && blockIdx.x == 0 && threadIdx.x == 0) ep.tnext[0] = t + ep.tadv;\n"
+         "  constexpr int NX = " << nx << ", NY = " << ny << ", H = " << g_.sweep_h << ";\n"
+         "  constexpr int NW = mol_sweep_windows<SwpS::PER0 != 0, SwpS::CX>(NX);\n"
+         "  const int b = mol_xcd_tile<SwpS::NBLK>((int)blockIdx.x);\n"
+         "  if (b >= NW * " << ns << ") return;   // (off the GPU: one window)\n"
+         "  MolSweep<SwpS::NF> g;\n"
+         "  g.nx = NX; g.ny = NY; g.lo0 = " << g_.lo[0][0] << "; g.lo1 = " << g_.lo[0][1] << "; g.lo2 = 1;\n";
+    for (int f = 0; f < d_->nfields; ++f) o << "  g.fofs[" << f << "] = " << g_.fofs[f] << "LL;\n";
+    o << "  mol_sweep_window<SwpS::PER0 != 0, SwpS::CX>(g, b % NW);\n"
+         "  g.y0 = (b / NW) * H;\n  g.y1 = min(g.y0 + H, NY);\n"
+         "  mol_rk4_sweep<SwpS, " << kahan << ">(MolNoHdr{}, g, u, unew, ep, jp, t);\n}\n";
+  }
+  o << "// resident steps per launch: 1\n";
+  return o.str();
+}
+
 uint64_t fnv1a(const std::string& s) {
   uint64_t h = 1469598103934665603ull;
   for (unsigned char ch : s) {
@@ -2259,6 +2420,20 @@ std::string jit_class_source(const mol_desc* d, const JitGeom& g, const std::str
 std::string jit_vjp_source(const mol_desc* d, const JitGeom& g, std::string& err) {
   Gen gen(d, g);
   std::string s = gen.source_vjp(d->dtype == MOL_F64);
+  err = gen.error;
+  return s;
+}
+
+std::string jit_sweep_source(const mol_desc* d, const JitGeom& g, std::string& err) {
+  Gen gen(d, g);
+  std::string s = gen.source_sweep(d->dtype == MOL_F64);
+  err = gen.error;
+  return s;
+}
+
+std::string jit_sweep_class(const mol_desc* d, const JitGeom& g, const std::string& name, std::string& err) {
+  Gen gen(d, g);
+  std::string s = gen.sweep_class_of(name);
   err = gen.error;
   return s;
 }

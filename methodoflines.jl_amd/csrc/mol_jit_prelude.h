@@ -33,6 +33,20 @@ __device__ __forceinline__ void mol_advance_clock(const Epi& ep) {
   if (ep.tnext && blockIdx.x == 0 && threadIdx.x == 0) ep.tnext[0] = ep.tnow[0] + ep.tadv;
 }
 
+// Constant memory (tables, coordinates, instance headers: no kernel that reads through this type
+// writes them): loads are hoisted out of loops, and are scalar where the address is uniform.
+#ifdef __AMDGCN__
+typedef const __attribute__((address_space(4))) double* MolRow;
+#else
+typedef const double* MolRow;
+#endif
+
+#ifdef __AMDGCN__
+typedef const __attribute__((address_space(4))) T* MolPar;
+#else
+typedef const T* MolPar;
+#endif
+
 // Node coordinates and auxiliary grid arrays (layout identical to mol::JitPtrs<T>).
 struct JPtrs {
   const double* coord[3];
@@ -397,14 +411,6 @@ __device__ __noinline__ void mol_weno5_nu3_grad(T u1, T u2, T u3, T u4, T u5, co
     g[k] = mol_weno5_nu3_t<MolDual>(d[0], d[1], d[2], d[3], d[4], c, eps).d;
   }
 }
-
-// Row of an axis table as constant memory: along y and z a wave's nodes share the row, and its
-// loads are scalar loads (the kernels never write the tables).
-#ifdef __AMDGCN__
-typedef const __attribute__((address_space(4))) double* MolRow;
-#else
-typedef const double* MolRow;
-#endif
 
 // Column of the tile's table of centred-target coefficients along x (G::nux: MOL_NU3 rows of
 // NUP = TX + 1 values, so that both the copy below and the nodes' reads are free of bank
@@ -1364,6 +1370,321 @@ __device__ __forceinline__ void mol_rk4_ring(T* X, double* fc, int* fo, const T*
   if (ep.tnext && threadIdx.x == 0) ep.tnext[0] = t;
 }
 
+// ---------------------------------------------------------------------------------------
+// One RK4 step of a 2D system of reach one (cross-shaped stencils) swept along y in registers.
+//
+// A wave owns a window of columns, one per lane (CX per lane: off the GPU a lane holds whole rows;
+// on it two or four FP32 columns per lane halve the DPP moves but not the time), and a strip of rows, and walks up the strip a row per iteration: iteration r takes row r of u, and stage s
+// evaluates row r - s from the three newest rows of its input, so the four stages run one row
+// apart and every stage value lives in registers for three iterations.  Neighbours along x come
+// from the adjacent lanes by DPP, ghosts along a non-periodic axis from the two nodes next to the
+// side: no LDS, no barrier, one read and one write of the state per step.  Windows overlap by
+// four columns (none where one window holds whole rows), strips by four rows on either side;
+// what is evaluated past the needed region never reaches an owned node.  A strip starts at row 0
+// of a non-periodic axis or at row 4 or above.
+//
+// What bounds it is VALU issue: the tile kernel above spends 74 instructions per node and stage of
+// the FP64 Brusselator (frame positions, index arithmetic, LDS addresses) where the arithmetic is
+// 23; the sweep spends 33, eight of them DPP moves.  Measured, us per step, tile kernel or stage
+// launches against the sweep: Brusselator FP64 1501^2 33 / 20, 1024^2 16.7 / 12.3, 400^2 6.8 / 5.6;
+// diffusion-reaction FP32 + Kahan 1500^2 57 / 13; 512 FP32 + Kahan instances 266 / 63 (3.2 TB/s).
+template <int V>
+struct MolInt {
+  static constexpr int v = V;
+};
+struct MolNoHdr {};   // header of a specialised system (all numbers are literals)
+
+// What a batched instance's generated code reads, loaded once per wave.
+template <int NF>
+struct MolSHdr {
+  int n[3];
+  MolRow W, K;
+  T g[NF][4][3];   // per side (x low, x high, y low, y high): factors of the two nodes next to it, of G
+};
+
+// Geometry of one sweep: unknowns nx x ny whose first node is (lo0, lo1), variable f at fofs[f];
+// window columns xb .., owned columns [x0, x1) and rows [y0, y1).
+template <int NF>
+struct MolSweep {
+  int nx, ny, lo0, lo1, lo2, xb, x0, x1, y0, y1;
+  i64 fofs[NF];
+};
+
+// Windows along an axis of n columns: their number, and window w's first and owned columns.
+template <bool PER, int CX>
+__device__ __forceinline__ constexpr int mol_sweep_windows(const int n) {
+  constexpr int WC = MOL_WAVE * CX, S = WC - 8;
+  return PER ? (n + S - 1) / S : (n <= WC ? 1 : (n - 8 + S - 1) / S);
+}
+template <bool PER, int CX, class Q>
+__device__ __forceinline__ void mol_sweep_window(Q& g, const int w) {
+  constexpr int WC = MOL_WAVE * CX, S = WC - 8;
+  const int nw = mol_sweep_windows<PER, CX>(g.nx);
+  g.xb = w * S - (PER ? 4 : 0);
+  g.x0 = PER ? w * S : (w == 0 ? 0 : g.xb + 4);
+  g.x1 = PER ? min(g.nx, (w + 1) * S) : (w == nw - 1 ? g.nx : g.xb + WC - 4);
+}
+
+template <class G, bool KAHAN, class HD>
+__device__ __forceinline__ void mol_rk4_sweep(const HD& hd, const MolSweep<G::NF>& g, const T* __restrict__ u,
+                                              T* __restrict__ unew, const Epi& ep, const JPtrs& jp, const double t) {
+  constexpr int NF = G::NF, CX = G::CX, NI = G::NINV > 0 ? G::NINV : 1, PF = 3;
+  constexpr bool PX = G::PER0 != 0, PY = G::PER1 != 0;
+  typedef T Row[CX][NF];
+  const double dt = ep.tadv;
+  const int lane = (int)threadIdx.x % MOL_WAVE, nx = g.nx, ny = g.ny, cb = g.xb + lane * CX;
+  // node index of each slot (its image on a periodic axis; the last node past the end, where the
+  // slot's values are never used)
+  int I0[CX];
+  unsigned co[CX];
+  bool own[CX];
+#pragma unroll
+  for (int c = 0; c < CX; ++c) {
+    int k = cb + c;
+    own[c] = k >= g.x0 && k < g.x1;
+    if (PX) {
+      k = min(k, nx + 3);
+      k = k < 0 ? k + nx : (k >= nx ? k - nx : k);
+    } else {
+      k = min(k, nx - 1);
+    }
+    I0[c] = g.lo0 + k;
+    co[c] = (unsigned)k * (unsigned)sizeof(T);
+  }
+  auto row_of = [&](int r) {
+    if (PY) return r < 0 ? r + ny : (r >= ny ? r - ny : r);
+    return min(max(r, 0), ny - 1);
+  };
+  // row at element offset o of each variable
+  auto load = [&](Row& v, const T* __restrict__ src, const i64 o) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const char* const p = (const char*)(src + g.fofs[f] + o);
+#pragma unroll
+      for (int c = 0; c < CX; ++c) v[c][f] = *(const T*)(p + co[c]);
+    }
+  };
+  auto store = [&](T* __restrict__ dst, const Row& v, const i64 o) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      char* const p = (char*)(dst + g.fofs[f] + o);
+#pragma unroll
+      for (int c = 0; c < CX; ++c)
+        if (own[c]) *(T*)(p + co[c]) = v[c][f];
+    }
+  };
+  // k = f at row q from rows up, ctr, dn of the stage input
+  auto eval = [&](const Row& up, const Row& ctr, const Row& dn, const int q, const double ts, const T (&iv)[CX][NI],
+                  Row& k) {
+    T w[NF * G::VOL];
+    const int I1 = g.lo1 + row_of(q);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      T* const L = w + f * G::VOL;
+#pragma unroll
+      for (int c = 0; c < CX; ++c) {
+        L[1 + c] = up[c][f];
+        L[1 + c + G::EX] = ctr[c][f];
+        L[1 + c + 2 * G::EX] = dn[c][f];
+      }
+      L[G::EX] = mol_lane_below(ctr[CX - 1][f]);
+      L[G::EX + CX + 1] = mol_lane_above(ctr[0][f]);
+      if constexpr (!PX) {
+        // window 0 starts at column 0
+        const T gl = G::ghost(hd, f, 0, L[G::EX + 1], L[G::EX + 2], g.lo0 - 1, I1, g.lo2, ts, ep.p, jp);
+        T gh[CX];
+#pragma unroll
+        for (int c = 0; c < CX; ++c)
+          gh[c] = G::ghost(hd, f, 1, L[G::EX + 1 + c], L[G::EX + c], g.lo0 + nx, I1, g.lo2, ts, ep.p, jp);
+        L[G::EX] = cb == 0 ? gl : L[G::EX];
+#pragma unroll
+        for (int c = 0; c < CX; ++c) L[G::EX + 2 + c] = cb + c == nx - 1 ? gh[c] : L[G::EX + 2 + c];
+      }
+      if constexpr (!PY) {
+        if (q == 0)
+#pragma unroll
+          for (int c = 0; c < CX; ++c)
+            L[1 + c] = G::ghost(hd, f, 2, ctr[c][f], dn[c][f], I0[c], g.lo1 - 1, g.lo2, ts, ep.p, jp);
+        if (q == ny - 1)
+#pragma unroll
+          for (int c = 0; c < CX; ++c)
+            L[1 + c + 2 * G::EX] = G::ghost(hd, f, 3, ctr[c][f], up[c][f], I0[c], g.lo1 + ny, g.lo2, ts, ep.p, jp);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CX; ++c) G::node(hd, w, 1 + c + G::EX, I0[c], I1, g.lo2, ts, ep.p, jp, iv[c], k[c]);
+  };
+  // Rings indexed by the row modulo their length: with six iterations unrolled every index is a
+  // constant and no value moves between registers.
+  constexpr int UN = 6;
+  Row U[UN], Y1[3], Y2[3], Y3[3], A1[2], A2[2], A3[2], pre[PF], cp[UN];
+  T iv[UN][CX][NI];
+#pragma unroll
+  for (int c = 0; c < CX; ++c)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 0; i < UN; ++i) {
+        U[i][c][f] = T(0);
+        Y1[i % 3][c][f] = Y2[i % 3][c][f] = Y3[i % 3][c][f] = T(0);
+        A1[i % 2][c][f] = A2[i % 2][c][f] = A3[i % 2][c][f] = cp[i][c][f] = T(0);
+      }
+#pragma unroll
+  for (int c = 0; c < CX; ++c)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < UN; ++j) iv[j][c][i] = T(0);
+  // r: the row taken by the running iteration; lr: the row being loaded, PF rows ahead (past a
+  // non-periodic end the last row again: its values are not used); offsets advance row by row
+  const bool cut = !PY && g.y0 == 0;   // no rows below the strip
+  int r = cut ? 0 : g.y0 - 4, lr = row_of(r);
+  const int rend = g.y1 + 4;
+  i64 lo = (i64)lr * nx, so = (i64)g.y0 * nx, ko = so;
+  const i64 ke = (i64)g.y1 * nx;
+  auto next = [&]() {
+    if (PY) {
+      if (++lr == ny) {
+        lr = 0;
+        lo = 0;
+      } else {
+        lo += nx;
+      }
+    } else if (lr < ny - 1) {
+      ++lr;
+      lo += nx;
+    }
+  };
+  const bool comp0 = KAHAN && ep.subA == 0;   // the compensation is read (else it is zero)
+  auto load_comp = [&](auto XC) {
+    if (KAHAN && comp0 && ko < ke) {
+      load(cp[decltype(XC)::v % UN], ep.comp, ko);
+      ko += nx;
+    }
+  };
+  // One iteration at ring position X (r modulo 6 from the strip's start) with its first NS stages.
+  auto step = [&](auto XC, auto NC) {
+    constexpr int x = decltype(XC)::v % 6, NS = decltype(NC)::v;
+    Row &u0 = U[x], &u1 = U[(x + 5) % 6], &u2 = U[(x + 4) % 6], &u3 = U[(x + 3) % 6], &u4 = U[(x + 2) % 6];
+#pragma unroll
+    for (int c = 0; c < CX; ++c)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) u0[c][f] = pre[x % PF][c][f];
+    load(pre[x % PF], u, lo);
+    next();
+    Row k;
+    if constexpr (NS >= 1) {
+      auto& iw = iv[(x + 5) % 6];
+      if constexpr (G::NINV > 0)
+#pragma unroll
+        for (int c = 0; c < CX; ++c) G::node_inv(hd, I0[c], g.lo1 + row_of(r - 1), g.lo2, ep.p, jp, iw[c]);
+      // u0 .. u4: rows r .. r - 4; stage s evaluates row r - s
+      eval(u2, u1, u0, r - 1, t, iw, k);
+      Row &a1 = A1[x % 2], &y1 = Y1[x % 3];
+#pragma unroll
+      for (int c = 0; c < CX; ++c)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          T v = (T)(dt / 2) * k[c][f];
+          v += u1[c][f];
+          y1[c][f] = v;
+          a1[c][f] = k[c][f];
+        }
+    }
+    if constexpr (NS >= 2) {
+      eval(Y1[(x + 1) % 3], Y1[(x + 2) % 3], Y1[x % 3], r - 2, t + dt / 2, iv[(x + 4) % 6], k);
+      Row &a2 = A2[x % 2], &b1 = A1[(x + 1) % 2], &y2 = Y2[x % 3];
+#pragma unroll
+      for (int c = 0; c < CX; ++c)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          T v = (T)(dt / 2) * k[c][f];
+          v += u2[c][f];
+          y2[c][f] = v;
+          const T a = T(2) * k[c][f];
+          a2[c][f] = a + b1[c][f];
+        }
+    }
+    if constexpr (NS >= 3) {
+      eval(Y2[(x + 1) % 3], Y2[(x + 2) % 3], Y2[x % 3], r - 3, t + dt / 2, iv[(x + 3) % 6], k);
+      Row &a3 = A3[x % 2], &b2 = A2[(x + 1) % 2], &y3 = Y3[x % 3];
+#pragma unroll
+      for (int c = 0; c < CX; ++c)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          T v = (T)dt * k[c][f];
+          v += u3[c][f];
+          y3[c][f] = v;
+          const T a = T(2) * k[c][f];
+          a3[c][f] = a + b2[c][f];
+        }
+    }
+    if constexpr (NS >= 4) {
+      eval(Y3[(x + 1) % 3], Y3[(x + 2) % 3], Y3[x % 3], r - 4, t + dt, iv[(x + 2) % 6], k);
+      Row out;
+      const Row &cx = cp[(x + 2) % UN], &b3 = A3[(x + 1) % 2];
+#pragma unroll
+      for (int c = 0; c < CX; ++c)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          if (KAHAN) {
+            T incr = (T)(dt / 6) * k[c][f];
+            incr += (T)(dt / 6) * b3[c][f];
+            const T y = incr - cx[c][f];
+            const T sm = u4[c][f] + y;
+            k[c][f] = (sm - u4[c][f]) - y;
+            out[c][f] = sm;
+          } else {
+            T v = (T)(dt / 6) * k[c][f];
+            v += u4[c][f];
+            v += (T)(dt / 6) * b3[c][f];
+            out[c][f] = v;
+          }
+        }
+      store(unew, out, so);
+      if (KAHAN) store(ep.comp, k, so);
+      so += nx;
+    }
+    // row r + 2 of the compensation, wanted six iterations later (its slot held row r - 4's)
+    if constexpr (NS >= 1) load_comp(MolInt<x + 2>{});
+    ++r;
+  };
+  // Rows y0 - 4 .. y0 + 3 start the stages two rows apart (a strip at a non-periodic end starts at
+  // its first row); from row y0 + 4 on every iteration finishes one row.
+#define MOL_STEP(X, N) step(MolInt<X>{}, MolInt<N>{})
+  auto fill = [&](auto XC) {   // the first PF rows, the strip's first one at ring position X
+#pragma unroll
+    for (int i = 0; i < PF; ++i) {
+      load(pre[(decltype(XC)::v + i) % PF], u, lo);
+      next();
+    }
+  };
+  if (!cut) {
+    fill(MolInt<0>{});
+    MOL_STEP(0, 0); MOL_STEP(1, 0); MOL_STEP(2, 1); MOL_STEP(3, 1);
+  } else {
+    fill(MolInt<4>{});
+    load_comp(MolInt<4>{});
+    load_comp(MolInt<5>{});
+  }
+  MOL_STEP(4, 2); MOL_STEP(5, 2); MOL_STEP(6, 3); MOL_STEP(7, 3);
+  while (true) {
+    MOL_STEP(8, 4);
+    if (r >= rend) break;
+    MOL_STEP(9, 4);
+    if (r >= rend) break;
+    MOL_STEP(10, 4);
+    if (r >= rend) break;
+    MOL_STEP(11, 4);
+    if (r >= rend) break;
+    MOL_STEP(12, 4);
+    if (r >= rend) break;
+    MOL_STEP(13, 4);
+    if (r >= rend) break;
+  }
+#undef MOL_STEP
+}
+
 // Arguments of the generated vector-Jacobian product (layout identical to mol::VArgs<T>).
 // The seed is lam = c1*s1 + c2*s2 (s2 may be null); out receives (df/du)^T lam and g_aux the
 // FP64 auxiliary-array gradients (may be null); both are accumulated, not overwritten.  bf and
@@ -1612,6 +1933,8 @@ struct BInst {
   const double* coord[3];
   const double* W;
   const double* K;
+  double g[8][4][3];    // per variable and side of the first two axes (x low, x high, y low, y high): the ghost
+                        // next to the box as factors of the two nodes next to the side and of G
 };
 
 // Index of node (p0, p1, p2) of variable f in the batch state: the instance's offset plus a

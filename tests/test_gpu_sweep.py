@@ -1,0 +1,79 @@
+"""GPU: RK4 steps of 2D systems and of batches swept along y in registers."""
+import numpy as np
+import pytest
+
+import molgpu
+from molgpu import systems
+from molgpu.batch import BatchProblem
+from molgpu.discretization import lower
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(prob, u0, t0, dt, N, **kw):
+    import torch
+    td = prob.torch_dtype()
+    u = torch.tensor(u0, device="cuda").to(td)
+    prob.integrate(u, t0, dt, N, molgpu.RK4, **kw)
+    torch.cuda.synchronize()
+    return u.double().cpu().numpy()
+
+
+# unknowns per axis at the edges of a window: less than one, one exactly, one column more, the
+# last two-window size, the first three-window size
+@pytest.mark.parametrize("n,rows", [(10, 4), (57, 5), (66, 9), (67, 64), (122, 16), (123, 7)])
+@pytest.mark.parametrize("case", ["periodic", (0, 1, 1, 0), (1, 0, 0, 1)])
+def test_swept_steps_equal_stage_launches(case, n, rows, monkeypatch):
+    monkeypatch.setenv("MOL_SWEEP", "1")
+    monkeypatch.setenv("MOL_SWEEP_ROWS", str(rows))
+    if case == "periodic":
+        prob = molgpu.discretize(*systems.brusselator2d(n=n))
+        dt, t0 = 0.01 / (n - 1) ** 2, 1.2
+    else:
+        prob = molgpu.discretize(*systems.diffreact2d(n, 0.1, 2.0, case))
+        dt, t0 = 0.5 / (n - 1) ** 2, 0.0
+    u0 = np.random.default_rng(n).uniform(0.5, 1.5, prob.lowered.n_unknowns)
+    print("  sweep %s n=%d rows=%d" % (case, n, rows), flush=True)
+    ref = _run(prob, u0, t0, dt, 5, fused=False)
+    got = _run(prob, u0, t0, dt, 5)
+    assert np.max(np.abs(got - ref)) <= 1e-13 * (1 + np.max(np.abs(ref)))
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_swept_compensated_fp32_steps(graph):
+    """200 FP32 steps with the compensated update stay within two roundings of the FP64 run, called
+    twice (the compensation starts from zero each time); without it the error is larger."""
+    n, N = 400, 200
+    sy = lambda dtype: systems.diffreact2d(n, 0.05, 1.0, (0, 1, 1, 0), dtype=dtype)
+    u0 = np.random.default_rng(3).uniform(0.1, 0.9, (n - 2) ** 2).astype(np.float32).astype(np.float64)
+    dt = 1.0 / (n - 1) ** 2
+    ref = _run(molgpu.discretize(*sy("f64")), u0, 0.0, dt, N)
+    prob = molgpu.discretize(*sy("f32"))
+    for call in range(2):
+        print("  sweep kahan graph=%s call=%d" % (graph, call), flush=True)
+        got = _run(prob, u0, 0.0, dt, N, kahan=True, graph=graph)
+        stage = _run(prob, u0, 0.0, dt, N, kahan=True, graph=graph, fused=False)
+        assert np.max(np.abs(got - ref)) <= 2 * np.max(np.abs(stage - ref)) + 2 ** -24
+        assert np.max(np.abs(got - ref)) < np.max(np.abs(_run(prob, u0, 0.0, dt, N) - ref))
+
+
+@pytest.mark.parametrize("dtype,kahan", [("f32", True), ("f32", False), ("f64", False)])
+def test_swept_batch_equals_stage_launches(dtype, kahan, monkeypatch):
+    """Instances from 8 to 254 unknowns per side with every mix of boundary kinds; odd and even
+    step counts (the state ends in the caller's array either way)."""
+    rng = np.random.default_rng(11)
+    lows, dts = [], []
+    for n in (10, 11, 33, 65, 66, 67, 100, 122, 123, 180, 256):
+        bc = tuple(int(b) for b in rng.integers(0, 2, 4))
+        lows.append(lower(*systems.diffreact2d(n, 0.05, 1.0 + 0.1 * n, bc, dtype=dtype)))
+        dts.append(2.0 / (n - 1) ** 2)
+    batch = BatchProblem(lows)
+    monkeypatch.setenv("MOL_SWEEP", "0")
+    stage = BatchProblem(lows)
+    u0 = rng.uniform(0.1, 0.9, batch.n_unknowns)
+    tol = 1e-13 if dtype == "f64" else 4 * 2.0 ** -24 * (1 if kahan else 4)
+    for N in (1, 4):
+        print("  sweep batch %s kahan=%s N=%d" % (dtype, kahan, N), flush=True)
+        got = _run(batch, u0, 0.0, min(dts), N, kahan=kahan)
+        ref = _run(stage, u0, 0.0, min(dts), N, kahan=kahan)
+        assert np.max(np.abs(got - ref)) <= tol
