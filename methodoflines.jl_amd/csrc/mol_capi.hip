@@ -1003,8 +1003,9 @@ int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int
   if (use_fused(h, scheme, kahan)) {
     // one launch per step (or per chunk of resident steps), the state alternating between u
     // and the workspace
+    // (a resident system is one work-group that reads the whole state before it writes: in place)
     T* src = u;
-    T* dst = y1;
+    T* dst = h->fused_resident ? u : y1;
     for (int64_t step = 0; step < nsteps;) {
       const int nsub = h->fused_resident ? (int)std::min<int64_t>(nsteps - step, 1024)
                                          : (h->fused_steps == 2 && nsteps - step >= 2 ? 2 : 1);
@@ -1018,7 +1019,7 @@ int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int
         e.comp = comp;
         e.subA = comp_zero && step == 0;   // nothing to read yet
       }
-      if (t0v && step == 0 && !h->fused_resident) {
+      if (t0v && step == 0) {
         e.tnow = nullptr;
         e.tofs = *t0v;
       }
@@ -1121,7 +1122,7 @@ int integrate_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int64_
   const bool resident = fused && h->fused_resident;
   const bool direct = !(flags & MOL_FLAG_GRAPH) || resident || nsteps < kGraphChunks[2];
   // direct fused steps take the start time by value in their first launch: no clock launch
-  if (direct && fused && !resident && nsteps > 0)
+  if (direct && fused && nsteps > 0)
     return enqueue_steps<T>(h, handle_work(h), u, p, dt, nsteps, scheme, kahan, s, &t0, true);
   if (launch_set_clock(h->d_tnow, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
   if (kahan && launch_fill_zero<T>((T*)h->w_comp, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
@@ -1563,7 +1564,7 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
   const size_t esize = ds[0]->dtype == MOL_F64 ? sizeof(double) : sizeof(float);
   std::map<std::string, int> cls_of, sw_of;
   std::vector<std::string> cls_src, sw_src;
-  std::vector<int> sw_cls(ninst, 0);
+  std::vector<int> sw_cls(ninst, 0), sw_of_cls;
   const char* se = std::getenv("MOL_SWEEP");
   bool sweep = !(se && se[0] == '0');
   P.hdr.assign(ninst, BInst{});
@@ -1587,24 +1588,26 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
     std::string err;
     const std::string src = jit_class_source(d, geom_of(ka, th.kc64, ncore), "GeoX", err);
     if (src.empty()) return fail(nullptr, MOL_ERR_UNSUPPORTED, "instance " + std::to_string(i) + ": " + err);
-    auto it = cls_of.find(src);
+    const auto it = cls_of.find(src);
+    const bool fresh = it == cls_of.end();
     int cls;
-    if (it == cls_of.end()) {
+    if (fresh) {
       cls = (int)cls_src.size();
       cls_of.emplace(src, cls);
       cls_src.push_back(src);
     } else {
       cls = it->second;
     }
-    if (sweep) {
+    // instances of one class share the sweep's class too (its body has the same structure)
+    for (int a = 0; a < 2 && sweep; ++a) sweep = a >= d->ndim || ka.uhi[a] - ka.ulo[a] + 1 >= 8;
+    if (sweep && fresh) {
       const std::string ss = jit_sweep_class(d, geom_of(ka, th.kc64, ncore), "SwpY", err);
       sweep = !ss.empty();
-      if (sweep) {
-        const auto sit = sw_of.emplace(ss, (int)sw_src.size());
-        if (sit.second) sw_src.push_back(ss);
-        sw_cls[i] = sit.first->second;
-      }
+      const auto sit = sw_of.emplace(ss, (int)sw_src.size());
+      if (sit.second) sw_src.push_back(ss);
+      sw_of_cls.push_back(sit.first->second);
     }
+    if (sweep) sw_cls[i] = sw_of_cls[cls];
     BInst& b = P.hdr[i];
     std::memset(&b, 0, sizeof(b));
     for (int k = 0; k < d->nclosures; ++k) {

@@ -2045,7 +2045,8 @@ std::string Gen::source_fused(bool f64) {
   o << "  static constexpr int KMAX = " << kmax << ";\n";
   o << close;
   o << "extern \"C\" __global__ void __launch_bounds__(" << g_.nthr
-    << ") mol_rk4_fused(const T* __restrict__ u, T* __restrict__ unew, Epi ep, JPtrs jp, int nsub) {\n";
+    << (resident ? ") mol_rk4_fused(const T* u, T* unew" : ") mol_rk4_fused(const T* __restrict__ u, T* __restrict__ unew")
+    << ", Epi ep, JPtrs jp, int nsub) {\n";
   if (resident) o << "  __shared__ T X[MolRing<GeoF>::XN];\n";
   else o << "  __shared__ T U[GeoF::NST * GeoF::VOL];\n  __shared__ T Ya[GeoF::NST * GeoF::VOL];\n"
             "  __shared__ T Yb[GeoF::NST * GeoF::VOL];\n";

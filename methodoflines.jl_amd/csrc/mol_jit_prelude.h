@@ -1238,9 +1238,9 @@ struct MolRing {
 };
 
 template <class G>
-__device__ __forceinline__ void mol_rk4_ring(T* X, double* fc, int* fo, const T* __restrict__ u,
-                                             T* __restrict__ unew, const Epi& ep, const JPtrs& jp, const double t0,
-                                             const int nsub) {
+__device__ __forceinline__ void mol_rk4_ring(T* X, double* fc, int* fo, const T* u, T* unew, const Epi& ep,
+                                             const JPtrs& jp, const double t0, const int nsub) {
+  // u and unew may be the same array
   using Q = MolRing<G>;
   static_assert(G::NBLK == 1 && G::RY == 0 && G::TY == 1 && (Q::PER || G::RX <= 1), "resident steps: one 1D tile");
   constexpr int R = Q::R, NJ = Q::NJ, NF = G::NF, NI = G::NINV > 0 ? G::NINV : 1;
@@ -1281,6 +1281,7 @@ __device__ __forceinline__ void mol_rk4_ring(T* X, double* fc, int* fo, const T*
     }
     if constexpr (G::NINV > 0) G::node_inv(o0 + at(j), o1, o2, ep.p, jp, Iv[j]);
   }
+  if (!Q::ONE) __syncthreads();   // every wave has read its overlaps before one writes
   // slot of the first and last node (compile time) and the lane holding it in this wave, or -1
   constexpr int QL = Q::HL, QH = Q::HL + Q::SL - 1;
   const bool low = !Q::PER && wv == 0 && lane == QL / NJ, high = !Q::PER && wv == Q::W - 1 && lane == QH / NJ;

@@ -16,7 +16,7 @@ import numpy as np
 
 from . import native
 from .discretization import Lowered
-from .problem import RK4, ODEProblem, _torch
+from .problem import RK4, ODEProblem, _stream, _torch
 
 
 def _descs(lows: Sequence[Lowered]):
@@ -103,7 +103,7 @@ class BatchProblem:
         self._check(u)
         self._check(du)
         rc = self.lib.mol_rhs(self.h, du.data_ptr(), u.data_ptr(), None, float(t),
-                              C.c_void_p(torch.cuda.current_stream().cuda_stream))
+                              _stream(torch))
         native.check(self.lib, rc, self.h)
 
     def integrate(self, u, t0: float, dt: float, nsteps: int, alg=RK4, kahan: bool = False,
@@ -112,5 +112,5 @@ class BatchProblem:
         self._check(u)
         flags = (native.MOL_FLAG_KAHAN if kahan else 0) | (native.MOL_FLAG_GRAPH if graph else 0)
         rc = self.lib.mol_integrate(self.h, u.data_ptr(), None, float(t0), float(dt), int(nsteps), alg.scheme,
-                                    flags, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+                                    flags, _stream(torch))
         native.check(self.lib, rc, self.h)
