@@ -844,6 +844,62 @@ bool sweep_source(mol_handle* h, const mol_desc* d, JitGeom& g, std::string& src
   return true;
 }
 
+// March of a 3D divergence-form system (jit_flux_source), forward or reverse mode: its source, and
+// the work-groups and threads in g; false when the system is not one, a tile was asked for or the
+// size rule is against it.  MOL_FLUX=0 or 1 overrides the size rule, MOL_FLUX_TILE=tx,ty,planes and
+// MOL_FLUX_VJP_TILE ask for other columns and chunks.
+//
+// Size: from 2^17 unknowns, and not where half of the columns or more would be padding.  Fewer leave
+// compute units without a work-group.  Per right-hand side and per reverse step with its gradients
+// (FP64, us, tiles -> march): 46^3 6.5 -> 7.3 and 19.7 -> 13.5, 54^3 8.4 -> 6.9 and 23.1 -> 13.7,
+// 126^3 31 -> 22 and 105 -> 47, 254^3 254 -> 209 and 954 -> 386.
+// Columns per work-group: 32 x 8 forward (a row of 32 is read in whole lines), 16 x 16 in reverse
+// mode, whose halo of seven costs less there.
+// Planes per chunk: a plane takes a compute unit about as long as 2.6 + its resident work-groups
+// (the walk is a serial chain of three barriers; the more of them share a unit, the better it is
+// hidden), and a chunk costs two planes more than it holds.  Measured, 126^3 FP64 reverse mode: 47 us
+// with chunks of 11 (three work-groups on every unit), 52 with 8 (four, three of them at a time),
+// 55 with 16; 73^3: 16.9 with 4, 23.6 with 8, 41 with 16.
+bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool vjp, JitGeom& g, std::string& src) {
+  const char* const force = std::getenv("MOL_FLUX");
+  if ((force && force[0] == '0') || d->ndim != 3) return false;
+  for (int a = 0; a < 3; ++a)
+    if (h->tile_req[a] > 0) return false;
+  g = gt;
+  const bool f64 = d->dtype == MOL_F64;
+  int tile[3] = {vjp ? 16 : 32, vjp ? 16 : 8, 0}, req[3], m[3];
+  const char* const e = std::getenv(vjp ? "MOL_FLUX_VJP_TILE" : "MOL_FLUX_TILE");
+  if (e && std::sscanf(e, "%d,%d,%d", &req[0], &req[1], &req[2]) == 3 && req[0] >= 8 && req[1] >= 8 && req[2] >= 3 &&
+      (req[0] * req[1]) % 64 == 0 && req[0] * req[1] <= 512)
+    for (int a = 0; a < 3; ++a) tile[a] = req[a];
+  for (int a = 0; a < 3; ++a) m[a] = g.n[a] - 2;
+  if (m[0] < 3 || m[1] < 3 || m[2] < 3) return false;
+  const long long nt = (long long)((m[0] + tile[0] - 1) / tile[0]) * ((m[1] + tile[1] - 1) / tile[1]);
+  if (!force && ((long long)m[0] * m[1] * m[2] < (1 << 17) || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
+  if (tile[2] == 0) {
+    const int occ = vjp ? (f64 ? 3 : 4) : (f64 ? 5 : 8);   // resident work-groups per compute unit
+    double best = 0.0;
+    for (int z = vjp ? 4 : 3; z <= 16; ++z) {
+      const long long k = (nt * std::min((m[2] + z - 1) / z, m[2] / 3) + 255) / 256;
+      const double cost = (z + 2) * ((k / occ) * (2.6 + occ) + (k % occ ? 2.6 + k % occ : 0.0));
+      if (tile[2] == 0 || cost < best) {
+        best = cost;
+        tile[2] = z;
+      }
+    }
+  }
+  for (int a = 0; a < 3; ++a) {
+    g.tile[a] = tile[a];
+    g.ntile[a] = (m[a] + tile[a] - 1) / tile[a];
+  }
+  g.ntile[2] = std::min(g.ntile[2], m[2] / 3);   // (chunks of three planes or more)
+  g.nthr = tile[0] * tile[1];
+  if (nt * g.ntile[2] > 0x7fffffffll) return false;
+  std::string err;
+  src = jit_flux_source(d, g, vjp, err);
+  return !src.empty();
+}
+
 void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, const KCore<double>& kc, int ncore) {
   h->fused_fn = h->fused_kahan_fn = nullptr;
   h->fused_tiles = 0;
@@ -899,8 +955,11 @@ int setup_paths(mol_handle* h, const mol_desc* d) {
     std::string err;
     JitGeom jg = geom_of(h->ka64, h->kc64, n64);
     jg.nthr = kernel_threads(jg, false);
-    h->jit_nthr = jg.nthr;
-    const std::string src = jit_source(d, jg, err);
+    JitGeom fg;
+    std::string src;
+    const bool flux = flux_source(h, d, jg, false, fg, src);
+    if (!flux) src = jit_source(d, jg, err);
+    h->jit_nthr = flux ? fg.nthr : jg.nthr;
     if (src.empty()) h->jit_reason = err;
     else if (jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err)) {
       h->jit_fn = nullptr;
@@ -910,7 +969,8 @@ int setup_paths(mol_handle* h, const mol_desc* d) {
       h->jit_fn = nullptr;
       h->jit_reason = err;
     }
-    const int ntl = h->ka64.ntile[0] * h->ka64.ntile[1] * h->ka64.ntile[2];
+    const int* nt = flux ? fg.ntile : h->ka64.ntile;
+    const int ntl = nt[0] * nt[1] * nt[2];
     if (h->jit_fn)
       h->jit_grid =
           src.find("mol_tiles_persistent<") != std::string::npos ? persistent_grid(h->jit_fn, ntl, jg.nthr) : ntl;
@@ -1246,9 +1306,17 @@ int ensure_vjp(mol_handle* h) {
   if (h->vjp_fn) return 0;
   const mol_desc* d = &h->desc.d;
   int ntiles = 0;
-  const JitGeom g = vjp_geometry(h, d, &ntiles);
-  std::string err;
-  const std::string src = jit_vjp_source(d, g, err);
+  JitGeom g = vjp_geometry(h, d, &ntiles), gf;
+  std::string err, src;
+  h->vjp_whole = flux_source(h, d, g, true, gf, src);
+  if (h->vjp_whole) {
+    g = gf;
+    ntiles = g.ntile[0] * g.ntile[1] * g.ntile[2];
+    // (a result over its own seed or state is made here first)
+    if (!h->adj_y[0]) HIPCHK(h, hipMalloc(&h->adj_y[0], (size_t)h->nunk * h->esize()));
+  } else {
+    src = jit_vjp_source(d, g, err);
+  }
   if (src.empty()) return fail(h, MOL_ERR_UNSUPPORTED, "vector-Jacobian product: " + err);
   h->vjp_store = src.find("// adjoint gather stores every unknown") != std::string::npos;
   if (jit_kernel(src, "mol_vjp_tiles", h->device, &h->vjp_fn, err) ||
@@ -1307,7 +1375,7 @@ int launch_vjp(mol_handle* h, const VArgs<T>& va, hipStream_t s, bool tiles = tr
     e = hipModuleLaunchKernel(h->vjp_fn, h->vjp_tiles, 1, 1, h->vjp_nthr, 1, 1, 0, s, args, nullptr);
     if (e != hipSuccess) return fail(h, MOL_ERR_HIP, std::string("vector-Jacobian product launch: ") + hipGetErrorString(e));
   }
-  if (!(v.mode & (VJP_GATHER_F | VJP_GATHER_A))) return 0;
+  if (h->vjp_whole || !(v.mode & (VJP_GATHER_F | VJP_GATHER_A))) return 0;
   // gather: every unknown, then every grid position of every grid field (when g_aux is given)
   const int64_t items = h->nunk + (v.g_aux ? (int64_t)h->desc.d.naux * ka.n[0] * ka.n[1] * ka.n[2] : 0);
   void* gargs[] = {(void*)&v};
@@ -1440,6 +1508,7 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
   }
   for (int k = 0; k < 4; ++k)
     if (!h->adj_y[k]) HIPCHK(h, hipMalloc(&h->adj_y[k], vbytes));
+  T* const lam_user = lam;
   T* S = (T*)h->seg_u;
   auto st = [&](int64_t j, int k) { return S + (size_t)(4 * j + k) * n; };   // state k of step j
   T* Y[4] = {(T*)h->adj_y[0], (T*)h->adj_y[1], (T*)h->adj_y[2], (T*)h->adj_y[3]};
@@ -1486,7 +1555,8 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
         va.tofs = tofs[q];
         va.mode = acc_aux ? (VJP_GATHER_F | VJP_ACC_A) : (VJP_GATHER_F | VJP_GATHER_A);
         if (q == 3 && h->vjp_store) {
-          // the last gather of the step stores lam + Y0 + Y1 + Y2 + its own sum into lam
+          // the last gather of the step stores lam + Y0 + Y1 + Y2 + its own sum into lam (the flux
+          // march, whose work-groups read their neighbours' lam, into Y3, which then is lam)
           va.mode |= VJP_SUM;
           va.lam = lam;
           va.y0 = Y[0];
@@ -1495,6 +1565,7 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
         }
         if ((rc = launch_vjp<T>(h, va, s))) return rc;
       }
+      if (h->vjp_whole) std::swap(lam, Y[3]);
       if (!h->vjp_store && (rc = launch_adjoint_sum<T>(lam, Y[0], Y[1], Y[2], Y[3], n, true, s)))
         return fail(h, rc, "adjoint update launch failed");
     }
@@ -1505,6 +1576,21 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
     va.mode = VJP_GATHER_A;
     if ((rc = launch_vjp<T>(h, va, s, false))) return rc;
   }
+  if (lam != lam_user) HIPCHK(h, hipMemcpyAsync(lam_user, lam, vbytes, hipMemcpyDeviceToDevice, s));
+  return 0;
+}
+
+// lam_dot = (df/du)^T lam at one state (mol_vjp).
+template <typename T>
+int vjp_impl(mol_handle* h, const T* u, const T* p, double t, const T* lam, T* lam_dot, double* g_aux, hipStream_t s) {
+  const size_t bytes = (size_t)h->nunk * sizeof(T);
+  auto meets = [&](const T* a) { return (const char*)a < (const char*)lam_dot + bytes && (const char*)lam_dot < (const char*)a + bytes; };
+  const bool over = h->vjp_whole && (meets(u) || meets(lam));
+  VArgs<T> va{u, lam, nullptr, 1.0, 0.0, over ? (T*)h->adj_y[0] : lam_dot, g_aux, p, nullptr, t};
+  va.mode = VJP_GATHER_F | VJP_GATHER_A;
+  if (!h->vjp_store && launch_fill_zero<T>(lam_dot, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
+  if (int rc = launch_vjp<T>(h, va, s)) return rc;
+  if (over) HIPCHK(h, hipMemcpyAsync(lam_dot, h->adj_y[0], bytes, hipMemcpyDeviceToDevice, s));
   return 0;
 }
 
@@ -2083,18 +2169,9 @@ int mol_vjp(mol_handle* h, const void* u, const void* p, double t, const void* l
   if (g_aux && !h->vjp_aux_ok)
     return fail(h, MOL_ERR_UNSUPPORTED, "auxiliary-array gradient through boundary values that read auxiliary arrays");
   hipStream_t s = (hipStream_t)stream;
-  if (h->dtype == MOL_F64) {
-    VArgs<double> va{(const double*)u, (const double*)lam, nullptr, 1.0, 0.0, (double*)lam_dot, g_aux,
-                     (const double*)p, nullptr, t};
-    va.mode = VJP_GATHER_F | VJP_GATHER_A;
-    if (!h->vjp_store && launch_fill_zero<double>((double*)lam_dot, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
-    return launch_vjp<double>(h, va, s);
-  }
-  VArgs<float> va{(const float*)u, (const float*)lam, nullptr, 1.0, 0.0, (float*)lam_dot, g_aux,
-                  (const float*)p, nullptr, t};
-  va.mode = VJP_GATHER_F | VJP_GATHER_A;
-  if (!h->vjp_store && launch_fill_zero<float>((float*)lam_dot, h->nunk, s)) return fail(h, MOL_ERR_HIP, "zero fill launch failed");
-  return launch_vjp<float>(h, va, s);
+  if (h->dtype == MOL_F64)
+    return vjp_impl<double>(h, (const double*)u, (const double*)p, t, (const double*)lam, (double*)lam_dot, g_aux, s);
+  return vjp_impl<float>(h, (const float*)u, (const float*)p, t, (const float*)lam, (float*)lam_dot, g_aux, s);
 }
 
 int mol_forward_checkpointed(mol_handle* h, void* u, const void* p, double t0, double dt, int64_t nsteps,
@@ -2180,8 +2257,10 @@ int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t b
     if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, g, src))
       src = jit_fused_source(d, g, err);
   } else {
-    src = (flags & MOL_CODEGEN_VJP) ? jit_vjp_source(d, vjp_geometry(&tmp, d, nullptr), err)
-                                    : jit_source(d, fwd_geom(tmp, ncore), err);
+    const bool vjp = (flags & MOL_CODEGEN_VJP) != 0;
+    const JitGeom g = vjp ? vjp_geometry(&tmp, d, nullptr) : fwd_geom(tmp, ncore);
+    JitGeom gf;
+    if (!flux_source(&tmp, d, g, vjp, gf, src)) src = vjp ? jit_vjp_source(d, g, err) : jit_source(d, g, err);
   }
   if (src.empty()) return fail(nullptr, MOL_ERR_UNSUPPORTED, err);
   if (flags & MOL_CODEGEN_COMPILE) {

@@ -49,6 +49,10 @@ inline int sweep_windows(bool per, int n) {
   return per ? (n + 55) / 56 : (n <= 64 ? 1 : (n - 8 + 55) / 56);
 }
 
+// 3D divergence form marched along z, forward or reverse mode (tile: columns along x and y per
+// work-group, planes per chunk); empty when the system does not qualify.
+std::string jit_flux_source(const mol_desc* d, const JitGeom& g, bool vjp, std::string& err);
+
 // Header of one instance of a batch (layout identical to BInst of mol_jit_prelude.h).
 struct BInst {
   int32_t n[3];
@@ -215,6 +219,7 @@ struct mol_handle {
   double* d_wtab[3] = {nullptr, nullptr, nullptr};   // nonuniform WENO5 coefficient rows per axis
   hipFunction_t vjp_fn = nullptr;         // generated vector-Jacobian product kernel
   bool vjp_store = false;                 // its gather stores every unknown (no zeroing of the output)
+  bool vjp_whole = false;                 // the tile kernel stores every sum itself (flux march: no gather)
   hipFunction_t vjp_gather_fn = nullptr;  // its gather of the per-tile adjoint buffers
   void* vjp_bf = nullptr;                 // per-tile adjoint buffers: staged variables (T)
   void* vjp_ba = nullptr;                 //   and staged grid fields (FP64)

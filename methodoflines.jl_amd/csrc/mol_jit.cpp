@@ -97,7 +97,7 @@ struct Var {
 };
 
 // Leaf context of a program.
-enum CtxKind { CTX_NODE, CTX_PLAIN, CTX_HALF, CTX_BOUNDARY };
+enum CtxKind { CTX_NODE, CTX_PLAIN, CTX_HALF, CTX_BOUNDARY, CTX_FLUX };
 struct Ctx {
   CtxKind kind = CTX_NODE;
   int ax = 0;                  // half-point axis, or the closure axis (CTX_BOUNDARY)
@@ -126,6 +126,8 @@ class Gen {
     param_ = true;
     return sweep_class(name);
   }
+  // 3D divergence form marched along z (mol_flux_rhs, mol_flux_vjp)
+  std::string source_flux(bool f64, bool vjp);
   std::string error;
 
  private:
@@ -141,6 +143,7 @@ class Gen {
   bool param_ = false;                // parametric (batched) printing
   bool fused_ = false;                // fused RK4 step printing (coordinates from LDS)
   bool vjp_ = false;                  // reverse-mode kernel printing
+  int flux_ = 0;                      // flux march printing: 1 half point, 2 node
   bool sweep_ = false;                // register sweep printing (window in registers, constant-memory reads)
   bool stage_noif_ = false;           // printing stage_ni (interface sides read nothing)
   // printing overrides: nodes not printed, and nodes referenced by another expression
@@ -322,6 +325,13 @@ class Gen {
     return "(T)jp.coord[" + istr(d) + "][min(max(" + k + ", 1), " + NN(d) + ") - 1]";
   }
 
+  // flux march: leaves of the inner derivative and of a slot along an axis
+  static constexpr int kInner = 900, kSlot = 1000;
+  std::vector<int> half_aux_, node_aux_;   // grid fields that the flux programs interpolate; read at the node
+  static int at(const std::vector<int>& v, int x) { return (int)(std::find(v.begin(), v.end(), x) - v.begin()); }
+  bool flux_rows(const mol_slot& s, double* wi, double* wd, double* wo, double (*ext)[4]);
+  void reverse_sweep(std::ostream& o, int r, const std::vector<std::pair<int, std::string>>& seeds,
+                     std::map<std::array<int, 4>, std::string>& acc) const;
   RowR row(const mol_optab& tb, int ax, const Var& v, int idx_rel);
   int apply(const RowR& r, int arr, int ax) {
     if (!r.valid) return lit_node(0.0);
@@ -570,6 +580,16 @@ int Gen::leaf(uint32_t code, int imm, const Ctx& c) {
         return expr("jp.aux[" + istr(imm) + "][(i64)(" + idx[0] + " - 1) + (i64)" + NN(0) + " * ((" +
                     idx[1] + " - 1) + (i64)" + NN(1) + " * (" + idx[2] + " - 1))]");
       default: return lit_node(0.0);
+    }
+  }
+  if (c.kind == CTX_FLUX) {
+    switch (code) {
+      case MOL_OP_FIELD: return lds(imm, 0, 0, 0);
+      case MOL_OP_AUX:
+        if (std::find(half_aux_.begin(), half_aux_.end(), imm) == half_aux_.end()) half_aux_.push_back(imm);
+        return lds(d_->nfields + imm, 0, 0, 0);
+      case MOL_OP_DINNER: return lds(kInner, 0, 0, 0);
+      default: bad("flux march: coordinates or slots in a coefficient"); return lit_node(0.0);
     }
   }
   if (c.kind == CTX_HALF) {
@@ -855,6 +875,11 @@ int Gen::slot(int k) {
   auto it = slot_node_.find(k);
   if (it != slot_node_.end()) return it->second;
   const mol_slot& s = d_->slots_h[k];
+  if (flux_) {
+    const int r = lds(kSlot + s.axis, 0, 0, 0);
+    slot_node_[k] = r;
+    return r;
+  }
   Var v[3];
   int r;
   if (core_ || s.kind == MOL_SLOT_WENO) {
@@ -1045,6 +1070,14 @@ std::string Gen::ref(int id) const {
   switch (n.kind) {
     case N_LIT: return n.src == 2 ? pk(n.val, n.sidx) : lit(n.val);
     case N_LDS: {
+      if (flux_ == 1) {
+        if (n.arr == kInner) return "d";
+        return n.arr == 0 ? "h[0]" : "h[" + istr(1 + at(half_aux_, n.arr - d_->nfields)) + "]";
+      }
+      if (flux_ == 2) {
+        if (n.arr >= kSlot) return "sv[" + istr(n.arr - kSlot) + "]";
+        return n.arr == 0 ? "u0" : "av[" + istr(at(node_aux_, n.arr - d_->nfields)) + "]";
+      }
       const int sl = pg_.slot.empty() ? n.arr : pg_.slot[n.arr];
       if (sl < 0) {
         // read at the node only: straight from global memory
@@ -1250,8 +1283,39 @@ void Gen::partials(const Node& n, int id, std::vector<std::pair<int, std::string
 // Adjoints of LDS leaves are summed per position and added to the LDS adjoint buffers
 // (Ab for variables, Aa in FP64 for auxiliary arrays) with LDS atomics.
 void Gen::print_reverse(std::ostream& o, int r, const std::vector<std::pair<int, std::string>>& seeds) const {
+  std::map<std::array<int, 4>, std::string> acc;
+  reverse_sweep(o, r, seeds, acc);
+  std::ostringstream aux_adds;
+  for (const auto& kv : acc) {
+    const int arr = kv.first[0];
+    const bool field = arr < d_->nfields;
+    const int sl = field ? pg_.fslot[arr] : pg_.aslot[arr - d_->nfields];
+    if (sl < 0) {
+      // array read at the node only: its adjoint goes straight to global memory (this node is
+      // the only writer of its position in a launch)
+      if (field)
+        o << "    outp[" << UIDX(arr, "I0", "I1", "I2") << "] += " << kv.second << ";\n";
+      else
+        o << "    if (gaux) gaux[" << (arr - d_->nfields) << " * NGRID + gidx(I0, I1, I2)] += (double)(" << kv.second
+          << ");\n";
+      continue;
+    }
+    const long long off = kv.first[1] + (long long)pg_.ext[0] * (kv.first[2] + (long long)pg_.ext[1] * kv.first[3]);
+    const std::string pos = off == 0 ? "b" : (off > 0 ? "b + " + istr(off) : "b - " + istr(-off));
+    if (field)
+      o << "    atomicAdd(&Ab[" << (long long)sl * pg_.vol << " + " << pos << "], (double)(" << kv.second << "));\n";
+    else
+      aux_adds << "      atomicAdd(&Aa[" << (long long)sl * pg_.vol << " + " << pos << "], (double)(" << kv.second
+               << "));\n";
+  }
+  // grid-field adjoints only when the caller asks for them (a uniform branch)
+  if (!aux_adds.str().empty()) o << "    if (gaux) {\n" << aux_adds.str() << "    }\n";
+}
+
+// The sweep itself: acc receives the adjoint terms of the leaves, (array, dx, dy, dz) -> expression.
+void Gen::reverse_sweep(std::ostream& o, int r, const std::vector<std::pair<int, std::string>>& seeds,
+                        std::map<std::array<int, 4>, std::string>& acc) const {
   const Region& R = regs_[r];
-  std::map<std::array<int, 4>, std::string> acc;   // (array, dx, dy, dz) -> adjoint terms
   for (int id : R.nodes) o << "    T g" << id << " = T(0);\n";
   auto add_adj = [&](int target, const std::string& e) {
     const Node& t = nodes_[target];
@@ -1297,31 +1361,6 @@ void Gen::print_reverse(std::ostream& o, int r, const std::vector<std::pair<int,
     }
     o << "\n";
   }
-  std::ostringstream aux_adds;
-  for (const auto& kv : acc) {
-    const int arr = kv.first[0];
-    const bool field = arr < d_->nfields;
-    const int sl = field ? pg_.fslot[arr] : pg_.aslot[arr - d_->nfields];
-    if (sl < 0) {
-      // array read at the node only: its adjoint goes straight to global memory (this node is
-      // the only writer of its position in a launch)
-      if (field)
-        o << "    outp[" << UIDX(arr, "I0", "I1", "I2") << "] += " << kv.second << ";\n";
-      else
-        o << "    if (gaux) gaux[" << (arr - d_->nfields) << " * NGRID + gidx(I0, I1, I2)] += (double)(" << kv.second
-          << ");\n";
-      continue;
-    }
-    const long long off = kv.first[1] + (long long)pg_.ext[0] * (kv.first[2] + (long long)pg_.ext[1] * kv.first[3]);
-    const std::string pos = off == 0 ? "b" : (off > 0 ? "b + " + istr(off) : "b - " + istr(-off));
-    if (field)
-      o << "    atomicAdd(&Ab[" << (long long)sl * pg_.vol << " + " << pos << "], (double)(" << kv.second << "));\n";
-    else
-      aux_adds << "      atomicAdd(&Aa[" << (long long)sl * pg_.vol << " + " << pos << "], (double)(" << kv.second
-               << "));\n";
-  }
-  // grid-field adjoints only when the caller asks for them (a uniform branch)
-  if (!aux_adds.str().empty()) o << "    if (gaux) {\n" << aux_adds.str() << "    }\n";
 }
 
 // Slow staging of one position: ring wrap, zero outside the grid and at corners, the unknown
@@ -2291,6 +2330,287 @@ std::string Gen::source_sweep(bool f64) {
   return o.str();
 }
 
+// Rows of a nonlinear-Laplacian slot as the flux march takes them: the interior interpolation (four
+// nodes h-1 .. h+2 around half point h), inner difference (h, h+1) and outer difference (half
+// points i-1, i), the same for every node; next to a side the interpolation may be one-sided, which
+// is the interior row with a node extrapolated past the boundary node, ext[side][m] its factors
+// of the nodes m = 0 .. 3 from the boundary inwards.  false: other rows.
+bool Gen::flux_rows(const mol_slot& s, double* wi, double* wd, double* wo, double (*ext)[4]) {
+  const int ax = s.axis, n = g_.n[ax];
+  for (int t = 0; t < 3; ++t)
+    if (d_->tabs_h[s.tab[t]].pn_hi > 0) return false;
+  // dense weights over rel = lo .. hi; false when a nonzero weight lies outside
+  auto dense = [](const RowR& r, int lo, int cnt, double* w) {
+    double top = 0.0;
+    for (double v : r.w) top = std::max(top, std::fabs(v));
+    for (int k = 0; k < cnt; ++k) w[k] = 0.0;
+    for (size_t k = 0; k < r.w.size(); ++k) {
+      if (std::fabs(r.w[k]) <= 1e-13 * top) continue;
+      const int p = r.rel[k] - lo;
+      if (p < 0 || p >= cnt) return false;
+      w[p] = r.w[k];
+    }
+    return r.valid;
+  };
+  auto same = [](const double* a, const double* b, int cnt) {
+    for (int k = 0; k < cnt; ++k)
+      if (std::fabs(a[k] - b[k]) > 1e-13 * (std::fabs(a[k]) + std::fabs(b[k]))) return false;
+    return true;
+  };
+  const Var in{true, 0};
+  double w[4];
+  const mol_optab &to = d_->tabs_h[s.tab[0]], &ti = d_->tabs_h[s.tab[1]], &tp = d_->tabs_h[s.tab[2]];
+  if (!dense(row(to, ax, in, -1), -1, 2, wo) || !dense(row(ti, ax, in, 0), 0, 2, wd) ||
+      !dense(row(tp, ax, in, 0), -1, 4, wi) || wi[0] == 0.0 || wi[3] == 0.0)
+    return false;
+  for (int i = 2; i <= n - 1; ++i)
+    if (!dense(row(to, ax, Var{false, i}, -1), -1, 2, w) || !same(w, wo, 2)) return false;
+  for (int h = 1; h <= n - 1; ++h) {
+    if (!dense(row(ti, ax, Var{false, h}, 0), 0, 2, w) || !same(w, wd, 2)) return false;
+    if (h > 1 && h < n - 1 && (!dense(row(tp, ax, Var{false, h}, 0), -1, 4, w) || !same(w, wi, 4))) return false;
+  }
+  if (!dense(row(tp, ax, Var{false, 1}, 0), 0, 4, w)) return false;
+  for (int m = 0; m < 4; ++m) ext[0][m] = (w[m] - (m < 3 ? wi[m + 1] : 0.0)) / wi[0];
+  if (!dense(row(tp, ax, Var{false, n - 1}, 0), -2, 4, w)) return false;
+  for (int m = 0; m < 4; ++m) ext[1][m] = (w[3 - m] - (m < 3 ? wi[2 - m] : 0.0)) / wi[3];
+  return true;
+}
+
+// The flux march of one system (forward kernel mol_rhs_tiles or reverse mode mol_vjp_tiles): one
+// variable in 3D on non-periodic axes, one nonlinear Laplacian per axis entering the right-hand
+// side linearly, everything else read at the node.  Empty (with error) otherwise.
+std::string Gen::source_flux(bool f64, bool vjp) {
+  auto no = [&](const char* m) {
+    bad(std::string("flux march: ") + m);
+    return std::string();
+  };
+  if (d_->ndim != 3 || d_->nfields != 1) return no("not one variable in 3D");
+  if ((long long)g_.n[0] * g_.n[1] * 8 >= (1ll << 31)) return no("planes of 2 GiB");   // (32-bit offsets)
+  int slot_of[3] = {-1, -1, -1};
+  const int rst = d_->prog_h[2 * d_->rhs_prog[0]], rln = d_->prog_h[2 * d_->rhs_prog[0] + 1];
+  for (int pc = rst; pc < rst + rln; ++pc) {
+    if ((d_->code_h[pc] & 0xffu) != MOL_OP_SLOT) continue;
+    const int k = (int)(d_->code_h[pc] >> 21);
+    const mol_slot& s = d_->slots_h[k];
+    if (slot_of[s.axis] == k) continue;
+    if (s.kind != MOL_SLOT_NONLINLAP || s.field != 0 || slot_of[s.axis] >= 0) return no("other operators");
+    slot_of[s.axis] = k;
+  }
+  double wi[3][4], wd[3][2], wo[3][2], ext[3][2][4], ws[3] = {0, 0, 0}, cl[3][2][2][4] = {};
+  int gprog[3][2] = {{-1, -1}, {-1, -1}, {-1, -1}};
+  for (int a = 0; a < 3; ++a) {
+    if (slot_of[a] < 0) return no("an axis without an operator");
+    if (g_.periodic[a] || g_.lo[0][a] != 2 || g_.hi[0][a] != g_.n[a] - 1 || g_.n[a] < 12)
+      return no("periodic, clipped or short axes");
+    if (!flux_rows(d_->slots_h[slot_of[a]], wi[a], wd[a], wo[a], ext[a])) return no("other operator rows");
+  }
+  for (int k = 0; k < d_->nclosures; ++k) {
+    const mol_closure& c = d_->closures_h[k];
+    if (c.src >= 0 || c.nghost != 1 || c.K > 3) return no("other boundary closures");
+    double(*w)[4] = cl[c.axis][c.side];
+    for (int m = 0; m < c.K; ++m) w[0][m] = d_->pool_h[c.wC + m];
+    if (c.gprog >= 0) {
+      const int st = d_->prog_h[2 * c.gprog], ln = d_->prog_h[2 * c.gprog + 1];
+      for (int pc = st; pc < st + ln; ++pc)
+        if ((d_->code_h[pc] & 0xffu) == MOL_OP_AUX) return no("boundary values that read a grid field");
+      w[0][3] = d_->pool_h[c.wc];
+      gprog[c.axis][c.side] = c.gprog;
+    }
+  }
+  for (int a = 0; a < 3; ++a)
+    for (int sd = 0; sd < 2; ++sd)
+      for (int m = 0; m < 4; ++m) cl[a][sd][1][m] = ext[a][sd][0] * cl[a][sd][0][m] + (m < 3 ? ext[a][sd][m + 1] : 0.0);
+  // the node's program with the slots as leaves: a linear combination in which each appears once
+  flux_ = 2;
+  std::vector<int> outs;
+  int rn;
+  build_node(true, outs, rn);
+  if (!ok_) return "";
+  {
+    const Node& on = nodes_[outs[0]];
+    if (on.kind != N_OP || on.op != X_LINCOMB || !on.wx.empty()) return no("slots do not enter linearly");
+    for (size_t k = 0; k < on.a.size(); ++k) {
+      const Node& a = nodes_[on.a[k]];
+      if (a.kind == N_LDS && a.arr >= kSlot) ws[a.arr - kSlot] += on.w[k];
+    }
+    for (int id : regs_[rn].nodes)
+      for (int a : nodes_[id].a)
+        if (id != outs[0] && nodes_[a].kind == N_LDS && nodes_[a].arr >= kSlot) return no("slots do not enter linearly");
+  }
+  // the flux programs
+  int rf[3];
+  std::vector<int> res(3);
+  for (int a = 0; a < 3; ++a) {
+    const mol_slot& s = d_->slots_h[slot_of[a]];
+    rf[a] = new_region();
+    cur_ = rf[a];
+    Ctx c;
+    c.kind = CTX_FLUX;
+    const int first = (int)regs_.size() - 1;
+    const int di = leaf(MOL_OP_DINNER, 0, c);
+    res[a] = op(MOL_OP_MUL, {s.prog >= 0 ? prog(s.prog, c) : lit_node(1.0), di});
+    if (!ok_) return "";
+    fold_linear(first, {res[a]});
+  }
+  auto note_aux = [&](int id) {
+    const Node& n = nodes_[id];
+    if (n.kind == N_LDS && n.arr >= d_->nfields && n.arr < kInner && at(node_aux_, n.arr - d_->nfields) == (int)node_aux_.size())
+      node_aux_.push_back(n.arr - d_->nfields);
+  };
+  if (half_aux_.size() > 2) return no("more than two grid fields in the coefficients");
+  std::ostringstream o;
+  o << "// generated " << (vjp ? "vector-Jacobian product of the " : "") << "right-hand side of one PDE system (flux march)\n";
+  o << "#define MOL_T " << (f64 ? "double" : "float") << "\n#include \"mol_jit_prelude.h\"\n\n" << layout_asserts(f64);
+  o << "struct GeoB {\n";
+  auto c = [&](const std::string& nm, long long v) { o << "  static constexpr int " << nm << " = " << v << ";\n"; };
+  const int TX = g_.tile[0], TY = g_.tile[1];
+  int m[3], nt[3];
+  for (int a = 0; a < 3; ++a) {
+    m[a] = g_.n[a] - 2;
+    nt[a] = g_.ntile[a];
+    c("N" + istr(a), g_.n[a]);
+    c("M" + istr(a), m[a]);
+    c("NT" + istr(a), nt[a]);
+  }
+  c("TX", TX); c("TY", TY);
+  c("NBLK", nt[0] * nt[1] * nt[2]);
+  c("NTHR", TX * TY);
+  c("NSTF", 0); c("NSTA", 0);   // (no per-tile adjoint buffers)
+  bool bv = false;
+  for (int a = 0; a < 3; ++a) bv = bv || gprog[a][0] >= 0 || gprog[a][1] >= 0;
+  o << "  static constexpr bool BV = " << (bv ? "true" : "false") << ";   // boundary programs\n";
+  c("NAH", (long long)half_aux_.size());
+  for (int id : regs_[rn].nodes)
+    for (int a : nodes_[id].a) note_aux(a);
+  note_aux(outs[0]);
+  std::vector<int> grad_aux = half_aux_, half_at, node_at;   // fields that get a gradient
+  for (int a : node_aux_)
+    if (at(grad_aux, a) == (int)grad_aux.size()) grad_aux.push_back(a);
+  for (int a : half_aux_) half_at.push_back(at(grad_aux, a));
+  for (int a : node_aux_) node_at.push_back(at(grad_aux, a));
+  auto list = [&](const char* nm, const std::vector<int>& v) {
+    o << "  static constexpr int " << nm << "[" << std::max<size_t>(1, v.size()) << "] = {";
+    for (size_t k = 0; k < v.size(); ++k) o << (k ? ", " : "") << v[k];
+    o << (v.empty() ? "0};\n" : "};\n");
+  };
+  c("NAU", (long long)node_aux_.size());
+  c("NAG", (long long)grad_aux.size());
+  list("AH", half_aux_);   // fields interpolated, read at the node, with a gradient; places in the last
+  list("AN", node_aux_);
+  list("AG", grad_aux);
+  list("HG", half_at);
+  o << "  static constexpr i64 NGRID = " << (long long)g_.n[0] * g_.n[1] * g_.n[2] << ";\n";
+  auto table = [&](const char* name, const char* args, const char* idx, const std::vector<double>& v) {
+    o << "  static __device__ __forceinline__ T " << name << "(" << args << ") {\n    const T tab[" << v.size() << "] = {";
+    for (size_t k = 0; k < v.size(); ++k) o << (k ? ", " : "") << lit(v[k]);
+    o << "};\n    return tab[" << idx << "];\n  }\n";
+  };
+  std::vector<double> vi, vd, vo, ve, vc, vs;
+  for (int a = 0; a < 3; ++a) {
+    vi.insert(vi.end(), wi[a], wi[a] + 4);
+    vd.insert(vd.end(), wd[a], wd[a] + 2);
+    vo.insert(vo.end(), wo[a], wo[a] + 2);
+    vs.push_back(ws[a]);
+    for (int sd = 0; sd < 2; ++sd) {
+      ve.insert(ve.end(), ext[a][sd], ext[a][sd] + 4);
+      for (int g = 0; g < 2; ++g) vc.insert(vc.end(), cl[a][sd][g], cl[a][sd][g] + 4);
+    }
+  }
+  table("wi", "const int ax, const int i", "4 * ax + i", vi);
+  table("wd", "const int ax, const int i", "2 * ax + i", vd);
+  table("wo", "const int ax, const int i", "2 * ax + i", vo);
+  table("ws", "const int ax", "ax", vs);
+  table("ext", "const int ax, const int side, const int m", "8 * ax + 4 * side + m", ve);
+  table("closure", "const int ax, const int side, const int g, const int m", "16 * ax + 8 * side + 4 * g + m", vc);
+  // boundary programs
+  flux_ = 2;
+  o << "  static __device__ __forceinline__ T bval(const int ax, const int side, const int p0, const int p1, const int p2,\n"
+       "      const double t, const T* __restrict__ P, const JPtrs& jp) {\n"
+       "    (void)p0; (void)p1; (void)p2; (void)t; (void)P; (void)jp;\n    switch (2 * ax + side) {\n";
+  for (int a = 0; a < 3; ++a)
+    for (int sd = 0; sd < 2; ++sd) {
+      if (gprog[a][sd] < 0) continue;
+      const int r = new_region();
+      cur_ = r;
+      Ctx bc;
+      bc.kind = CTX_BOUNDARY;
+      bc.ax = a;
+      bc.side = sd;
+      regs_[r].result = prog(gprog[a][sd], bc);
+      o << "    case " << 2 * a + sd << ": {\n";
+      print_region(o, r);
+      o << "    return " << ref(regs_[r].result) << ";\n    }\n";
+    }
+  o << "    default: return T(0);\n    }\n  }\n";
+  // half points
+  flux_ = 1;
+  o << "  template <int AX>\n  static __device__ __forceinline__ T flux(const T* h, const T d, const double t,\n"
+       "      const T* __restrict__ P) {\n    (void)h; (void)d; (void)t; (void)P;\n";
+  for (int a = 0; a < 3; ++a) {
+    o << "    if constexpr (AX == " << a << ") {\n";
+    print_region(o, rf[a]);
+    o << "    return " << ref(res[a]) << ";\n    }\n";
+  }
+  o << "  }\n";
+  if (vjp) {
+    o << "  template <int AX>\n  static __device__ __forceinline__ void dflux(const T* h, const T d, const T phi, const double t,\n"
+         "      const T* __restrict__ P, T& p, T* r, T& q) {\n    (void)h; (void)d; (void)t; (void)P;\n    p = q = T(0);\n"
+         "    for (int a = 0; a < (NAH > 0 ? NAH : 1); ++a) r[a] = T(0);\n";
+    for (int a = 0; a < 3; ++a) {
+      o << "    if constexpr (AX == " << a << ") {\n";
+      print_region(o, rf[a]);
+      std::map<std::array<int, 4>, std::string> acc;
+      reverse_sweep(o, rf[a], {{res[a], "phi"}}, acc);
+      for (const auto& kv : acc) {
+        const int arr = kv.first[0];
+        o << "    " << (arr == kInner ? "q" : arr == 0 ? "p" : "r[" + istr(at(half_aux_, arr - 1)) + "]") << " += " << kv.second << ";\n";
+      }
+      o << "    }\n";
+    }
+    o << "  }\n";
+  }
+  // node
+  flux_ = 2;
+  o << "  static __device__ __forceinline__ void node(const T u0, const T* sv, const T* av, const int I0, const int I1,\n"
+       "      const int I2, const double t, const T* __restrict__ P, const JPtrs& jp, T& out) {\n"
+       "    (void)u0; (void)sv; (void)av; (void)I0; (void)I1; (void)I2; (void)t; (void)P; (void)jp;\n";
+  print_region(o, rn);
+  o << "    out = " << ref(outs[0]) << ";\n  }\n";
+  if (vjp) {
+    o << "  static __device__ __forceinline__ void dnode(const T u0, const T lam, const T* av, const int I0, const int I1,\n"
+         "      const int I2, const double t, const T* __restrict__ P, const JPtrs& jp, double& ub, double* dg) {\n"
+         "    (void)u0; (void)lam; (void)av; (void)I0; (void)I1; (void)I2; (void)t; (void)P; (void)jp; (void)ub; (void)dg;\n"
+         "    const T sv[3] = {T(0), T(0), T(0)};\n    (void)sv;\n";
+    print_region(o, rn);
+    std::map<std::array<int, 4>, std::string> acc;
+    reverse_sweep(o, rn, {{outs[0], "lam"}}, acc);
+    for (const auto& kv : acc) {
+      const int arr = kv.first[0];
+      if (arr >= kSlot) continue;
+      if (arr == 0) o << "    ub += (double)(" << kv.second << ");\n";
+      else o << "    dg[" << node_at[at(node_aux_, arr - 1)] << "] += (double)(" << kv.second << ");\n";
+    }
+    o << "  }\n";
+  }
+  o << "};\n\n";
+  if (!vjp) {
+    o << "extern \"C\" __global__ void __launch_bounds__(" << TX * TY << ") mol_rhs_tiles(const T* __restrict__ u, Epi ep, JPtrs jp) {\n"
+         "  __shared__ MolFluxLds<GeoB> S;\n"
+         "  const double t = (ep.tnow ? ep.tnow[0] : 0.0) + ep.tofs;\n"
+         "  mol_advance_clock(ep);\n"
+         "  mol_flux_rhs<GeoB>(S, u, ep, jp, t);\n}\n";
+  } else {
+    o << "constexpr int VOLX = 1;\n"
+         "extern \"C\" __global__ void MOL_BOUNDS(" << TX * TY << (f64 ? ", 3" : ", 4") << ") mol_vjp_tiles(VArgs va, JPtrs jp) {\n"
+         "  __shared__ MolFluxVLds<GeoB> S;\n"
+         "  const double t = (va.tnow ? va.tnow[0] : 0.0) + va.tofs;\n"
+         "  mol_flux_vjp<GeoB>(S, va, jp, t);\n}\n"
+         "// adjoint gather stores every unknown; nothing is left to gather\n"
+         "extern \"C\" __global__ void __launch_bounds__(256) mol_vjp_gather(VArgs va) { (void)va; }\n";
+  }
+  return o.str();
+}
+
 uint64_t fnv1a(const std::string& s) {
   uint64_t h = 1469598103934665603ull;
   for (unsigned char ch : s) {
@@ -2435,6 +2755,13 @@ std::string jit_sweep_source(const mol_desc* d, const JitGeom& g, std::string& e
 std::string jit_sweep_class(const mol_desc* d, const JitGeom& g, const std::string& name, std::string& err) {
   Gen gen(d, g);
   std::string s = gen.sweep_class_of(name);
+  err = gen.error;
+  return s;
+}
+
+std::string jit_flux_source(const mol_desc* d, const JitGeom& g, bool vjp, std::string& err) {
+  Gen gen(d, g);
+  std::string s = gen.source_flux(d->dtype == MOL_F64, vjp);
   err = gen.error;
   return s;
 }

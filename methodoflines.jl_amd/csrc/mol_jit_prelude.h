@@ -1916,6 +1916,745 @@ __device__ __forceinline__ void mol_vjp_tile(T* L, double* Ab, double* Aa, const
 }
 
 // ---------------------------------------------------------------------------------------
+// 3D divergence form  u_t = r(u, aux) + sum over the axes of  d/dx (a(u, aux) du/dx)  marched
+// along z: the right-hand side (or one Runge-Kutta stage) and its reverse mode.
+//
+// The reference evaluates the half-point flux a(...) du/dx on either side of a node; the flux on
+// a node's upper side is the one on the lower side of its neighbour.  A work-group owns TX x TY
+// columns and walks up ZC planes: along z a thread keeps the last planes and the last flux in
+// registers, along x and y the plane lies in LDS with its halo, every thread evaluates the fluxes
+// on its upper sides and leaves them in LDS for the neighbours.  So a node costs three fluxes
+// instead of six, and the state is read once per plane and tile (with the halo columns) instead
+// of 2.25 times.  The one-sided interpolation next to a side equals the interior row with one
+// more node past the boundary node, extrapolated from the four nodes next to it (G::ext): with
+// that node all half points have one formula.  Every load of a plane is without a branch (columns
+// outside are clamped) and one plane ahead; boundary and extrapolated nodes are made from the
+// staged plane, along z from the planes in registers.
+// Bound: forward FP64 by memory (126^3: 22 us per stage for about 105 MB, 31 us with tiles that stage
+// 2.25 positions per node), FP32 and small grids by the serial chain of a plane (LDS, fluxes, LDS:
+// 0.9 us).  Reverse mode 47 us instead of 105 (tile kernel and gather) at 126^3, 15 instead of 33
+// at 73^3 FP32: about 620 instructions and three barriers per plane.
+//
+// Positions are counted from the first unknown: 0 .. M-1 unknowns, -1 and M boundary nodes, -2 and
+// M + 1 the extrapolated ones.  Staged arrays: 0 the state, 1 .. NAH the grid fields of a().
+
+// Launch bounds with a number of waves per SIMD unit that the registers have to allow.
+#ifdef __AMDGCN__
+#define MOL_BOUNDS(threads, waves) __launch_bounds__(threads, waves)
+#else
+#define MOL_BOUNDS(threads, waves)
+#endif
+
+// Offsets in bytes of a column in a plane of the state and of a grid field; columns outside give the
+// nearest one.  (The plane is added to the pointer, which is the same for all threads.)
+template <class G>
+struct MolFluxCol {
+  unsigned u, a;
+  __device__ __forceinline__ void at(const int x, const int y) {
+    u = (unsigned)(min(max(x, 0), G::M0 - 1) + G::M0 * min(max(y, 0), G::M1 - 1)) * (unsigned)sizeof(T);
+    a = (unsigned)((min(max(x, -1), (int)G::M0) + 1) + G::N0 * (min(max(y, -1), (int)G::M1) + 1)) * (unsigned)sizeof(T);
+  }
+};
+template <typename V>
+__device__ __forceinline__ V& mol_at(V* const p, const unsigned bytes) {
+  return *(V*)((char*)p + bytes);
+}
+template <typename V>
+__device__ __forceinline__ const V& mol_at(const V* const p, const unsigned bytes) {
+  return *(const V*)((const char*)p + bytes);
+}
+
+// The same with the pointer kept in scalar registers.  Left to itself the compiler holds pointer +
+// offset of every array over the loop, two vector registers each: the reverse mode takes 166
+// registers instead of 141 (FP64) and 1.1 to 1.4 times as long in FP32, the right-hand side, which
+// has registers to spare, gets slower by a few per cent.
+#ifdef __AMDGCN__
+template <typename V>
+using MolGlobal = __attribute__((address_space(1))) V;
+__device__ __forceinline__ MolGlobal<char>* mol_scalar(const void* const p) {
+  const unsigned long long v = (unsigned long long)p;   // (an "s" operand has to be in scalar registers)
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+  return (MolGlobal<char>*)(((unsigned long long)hi << 32) | lo);
+}
+template <typename V>
+__device__ __forceinline__ MolGlobal<V>& mol_at_s(V* const p, unsigned bytes) {
+  MolGlobal<char>* q = mol_scalar(p);
+  asm("" : "+s"(q), "+v"(bytes));
+  return *(MolGlobal<V>*)(q + bytes);
+}
+template <typename V>
+__device__ __forceinline__ const MolGlobal<V>& mol_at_s(const V* const p, unsigned bytes) {
+  MolGlobal<char>* q = mol_scalar(p);
+  asm("" : "+s"(q), "+v"(bytes));
+  return *(const MolGlobal<V>*)(q + bytes);
+}
+#else
+template <typename V>
+inline V& mol_at_s(V* const p, const unsigned bytes) {
+  return mol_at(p, bytes);
+}
+#endif
+
+// Staged arrays of a column at plane z (state at the nearest unknown); SC: scalar pointers.
+template <class G, bool SC>
+__device__ __forceinline__ void mol_flux_load(T (&v)[1 + G::NAH], const MolFluxCol<G>& c, const T* __restrict__ u,
+                                              const JPtrs& jp, const int z) {
+  int zu = min(max(z, 0), G::M2 - 1), za = min(max(z, -1), (int)G::M2) + 1;
+  if constexpr (SC) {
+    zu = mol_uniform(zu);
+    za = mol_uniform(za);
+  }
+  const T* const p = u + (i64)G::M0 * G::M1 * zu;
+  v[0] = SC ? mol_at_s(p, c.u) : mol_at(p, c.u);
+#pragma unroll
+  for (int a = 0; a < G::NAH; ++a) {
+    const T* const q = jp.aux[G::AH[a]] + (i64)G::N0 * G::N1 * za;
+    v[1 + a] = SC ? mol_at_s(q, c.a) : mol_at(q, c.a);
+  }
+}
+
+// State at the boundary (g = 0) or extrapolated (g = 1) node of a side from the three unknowns
+// next to it.
+template <class G>
+__device__ __forceinline__ T mol_flux_ghost(const int ax, const int side, const int g, const T n0, const T n1, const T n2,
+                                            const T bv) {
+  T s = G::closure(ax, side, g, 0) * n0;
+  s += G::closure(ax, side, g, 1) * n1;
+  s += G::closure(ax, side, g, 2) * n2;
+  if constexpr (G::BV) s += G::closure(ax, side, g, 3) * bv;
+  return s;
+}
+
+// Plane M2 (g = 0) or M2 + 1 (g = 1) of a column from the four planes before it, the last in r3;
+// v holds the loaded grid fields.
+template <class G>
+__device__ __forceinline__ void mol_flux_above(T (&v)[1 + G::NAH], const T (&r0)[1 + G::NAH], const T (&r1)[1 + G::NAH],
+                                               const T (&r2)[1 + G::NAH], const T (&r3)[1 + G::NAH], const int g,
+                                               const T bv) {
+  if (g == 0) {
+    v[0] = mol_flux_ghost<G>(2, 1, 0, r3[0], r2[0], r1[0], bv);
+  } else {
+    v[0] = mol_flux_ghost<G>(2, 1, 1, r2[0], r1[0], r0[0], bv);
+#pragma unroll
+    for (int a = 1; a <= G::NAH; ++a)
+      v[a] = G::ext(2, 1, 0) * r3[a] + G::ext(2, 1, 1) * r2[a] + G::ext(2, 1, 2) * r1[a] + G::ext(2, 1, 3) * r0[a];
+  }
+}
+
+// Value of the boundary program of a side at a position (coordinates outside the grid: the nearest).
+template <class G>
+__device__ __forceinline__ T mol_flux_bval(const int ax, const int side, const int x, const int y, const int z,
+                                           const double t, const T* __restrict__ P, const JPtrs& jp) {
+  if constexpr (!G::BV) return T(0);
+  else
+    return G::bval(ax, side, min(max(x, -1), (int)G::M0) + 2, min(max(y, -1), (int)G::M1) + 2,
+                   min(max(z, -1), (int)G::M2) + 2, t, P, jp);
+}
+
+// NP planes z0 - B .. of a column: loaded, then those past a side along z.
+template <class G, int NP, int B, bool SC>
+__device__ __forceinline__ void mol_flux_planes(T (&q)[NP][1 + G::NAH], const MolFluxCol<G>& col, const int x, const int y,
+                                                const int z0, const T* __restrict__ u, const JPtrs& jp, const double t,
+                                                const T* __restrict__ P) {
+#pragma unroll
+  for (int i = 0; i < NP; ++i) mol_flux_load<G, SC>(q[i], col, u, jp, z0 - B + i);
+  if (z0 == 0) {
+    const T bv = mol_flux_bval<G>(2, 0, x, y, -1, t, P, jp);
+    q[B - 1][0] = mol_flux_ghost<G>(2, 0, 0, q[B][0], q[B + 1][0], q[B + 2][0], bv);
+    q[B - 2][0] = mol_flux_ghost<G>(2, 0, 1, q[B][0], q[B + 1][0], q[B + 2][0], bv);
+#pragma unroll
+    for (int a = 1; a <= G::NAH; ++a)
+      q[B - 2][a] = G::ext(2, 0, 0) * q[B - 1][a] + G::ext(2, 0, 1) * q[B][a] + G::ext(2, 0, 2) * q[B + 1][a] +
+                    G::ext(2, 0, 3) * q[B + 2][a];
+  }
+  if (z0 - B + NP > G::M2)   // (the last chunk has three planes or more: plane M2 only, the last)
+    mol_flux_above<G>(q[NP - 1], q[0], q[NP - 4], q[NP - 3], q[NP - 2], 0, mol_flux_bval<G>(2, 1, x, y, G::M2, t, P, jp));
+}
+
+// First plane of chunk i: NT2 chunks that differ by one plane at most (three planes or more).
+template <class G>
+__device__ __forceinline__ int mol_flux_chunk(const int i) {
+  return (int)((i64)G::M2 * i / G::NT2);
+}
+
+// Halo position q of a TX x TY tile with HL positions before and HH past it along either axis
+// (no corners), relative to the tile.
+template <class G, int HL, int HH>
+__device__ __forceinline__ void mol_flux_halo(const int q, int& x, int& y) {
+  constexpr int H = HL + HH;
+  const int r = q - H * G::TY;
+  const bool ax = r < 0;
+  const int y0 = q / H, x0 = q - y0 * H, y1 = r / G::TX, x1 = r - y1 * G::TX;
+  x = ax ? (x0 < HL ? x0 - HL : G::TX + (x0 - HL)) : x1;
+  y = ax ? y0 : (y1 < HL ? y1 - HL : G::TY + (y1 - HL));
+}
+
+// Boundary and extrapolated nodes of one side in the staged plane (halo HL, HH, rows of LX).
+template <class G, int AX, int SIDE, int HL, int HH, int LX>
+__device__ __forceinline__ void mol_flux_side(T* const L, const int LN, const int X0, const int Y0, const int c,
+                                              const double t, const T* __restrict__ P, const JPtrs& jp) {
+  constexpr int M = AX == 0 ? G::M0 : G::M1, TA = AX == 0 ? G::TX : G::TY, TB = AX == 0 ? G::TY : G::TX;
+  const int b = (SIDE == 0 ? -1 : M) - (AX == 0 ? X0 : Y0);   // the boundary node, relative to the tile
+  if (SIDE == 0 ? b != -1 : b >= TA + HH) return;
+  const bool two = SIDE == 0 || b + 1 < TA + HH;
+  constexpr int st = AX == 0 ? 1 : LX, d = SIDE == 0 ? st : -st;
+  for (int r = (int)threadIdx.x; r < TB; r += G::NTHR) {
+    const int o = AX == 0 ? (b + HL) + LX * (r + HL) : (r + HL) + LX * (b + HL);
+    const T bv = AX == 0 ? mol_flux_bval<G>(0, SIDE, X0 + b, Y0 + r, c, t, P, jp)
+                         : mol_flux_bval<G>(1, SIDE, X0 + r, Y0 + b, c, t, P, jp);
+    const T n0 = L[o + d], n1 = L[o + 2 * d], n2 = L[o + 3 * d];
+    L[o] = mol_flux_ghost<G>(AX, SIDE, 0, n0, n1, n2, bv);
+    if (two) {
+      L[o - d] = mol_flux_ghost<G>(AX, SIDE, 1, n0, n1, n2, bv);
+#pragma unroll
+      for (int a = 1; a <= G::NAH; ++a) {
+        const T* const A = L + a * LN + o;
+        L[a * LN + o - d] = G::ext(AX, SIDE, 0) * A[0] + G::ext(AX, SIDE, 1) * A[d] + G::ext(AX, SIDE, 2) * A[2 * d] +
+                            G::ext(AX, SIDE, 3) * A[3 * d];
+      }
+    }
+  }
+}
+
+// All four sides of a staged plane, and the barrier after it (a tile that touches no side has none).
+template <class G, int HL, int HH, int LX>
+__device__ __forceinline__ void mol_flux_sides(T* const L, const int LN, const int X0, const int Y0, const int c,
+                                               const double t, const T* __restrict__ P, const JPtrs& jp) {
+  if (X0 > 0 && Y0 > 0 && X0 + G::TX + HH <= G::M0 && Y0 + G::TY + HH <= G::M1) return;
+  mol_flux_side<G, 0, 0, HL, HH, LX>(L, LN, X0, Y0, c, t, P, jp);
+  mol_flux_side<G, 0, 1, HL, HH, LX>(L, LN, X0, Y0, c, t, P, jp);
+  mol_flux_side<G, 1, 0, HL, HH, LX>(L, LN, X0, Y0, c, t, P, jp);
+  mol_flux_side<G, 1, 1, HL, HH, LX>(L, LN, X0, Y0, c, t, P, jp);
+  __syncthreads();
+}
+
+// Interpolated values and inner derivative at a half point from four consecutive positions.
+template <class G>
+__device__ __forceinline__ void mol_flux_half(const int ax, const T (&w)[4][1 + G::NAH], T (&h)[1 + G::NAH], T& d) {
+#pragma unroll
+  for (int a = 0; a <= G::NAH; ++a) {
+    T s = G::wi(ax, 0) * w[0][a];
+    s += G::wi(ax, 1) * w[1][a];
+    s += G::wi(ax, 2) * w[2][a];
+    s += G::wi(ax, 3) * w[3][a];
+    h[a] = s;
+  }
+  d = G::wd(ax, 0) * w[1][0];
+  d += G::wd(ax, 1) * w[2][0];
+}
+
+template <class G, int AX>
+__device__ __forceinline__ T mol_flux_at(const T (&w)[4][1 + G::NAH], const double t, const T* __restrict__ P) {
+  T h[1 + G::NAH], d;
+  mol_flux_half<G>(AX, w, h, d);
+  return G::template flux<AX>(h, d, t, P);
+}
+
+// Right-hand side or one stage.  L: plane with a halo of two, FX, FY: fluxes on the upper sides of
+// columns -1 .. and rows -1 ..
+template <class G>
+struct MolFluxLds {
+  static constexpr int LX = G::TX + 4, LY = G::TY + 4, NA = 1 + G::NAH, NC = G::TX * G::TY;
+  T L[NA][LX * LY];
+  T FX[(G::TX + 1) * G::TY], FY[G::TX * (G::TY + 1)];
+};
+
+template <class G>
+__device__ __forceinline__ void mol_flux_rhs(MolFluxLds<G>& S, const T* __restrict__ u, const Epi& ep, const JPtrs& jp,
+                                             const double t) {
+  typedef MolFluxLds<G> Q;
+  constexpr int TX = G::TX, TY = G::TY, NA = Q::NA, NI = Q::NC / G::NTHR, NH = 4 * (TX + TY);
+  constexpr int NHI = (NH + G::NTHR - 1) / G::NTHR, NQ = G::NAU > 0 ? G::NAU : 1;
+  constexpr i64 PU = (i64)G::M0 * G::M1, PA = (i64)G::N0 * G::N1;
+  const int b = mol_xcd_tile<G::NBLK>((int)blockIdx.x);
+  const int X0 = (b % G::NT0) * TX, Y0 = (b / G::NT0 % G::NT1) * TY, zc = b / (G::NT0 * G::NT1);
+  const int z0 = mol_flux_chunk<G>(zc), z1 = mol_flux_chunk<G>(zc + 1);
+  const T* const P = ep.p;
+  T R[NI][4][NA], Fz[NI], hv[NHI][NA];   // planes c-1 .. c+2 of a column, flux below plane c, halo of plane c
+  int cx[NI], cy[NI], ho[NHI];           // ho: the halo position's place in L
+  MolFluxCol<G> col[NI], hc[NHI];
+#pragma unroll
+  for (int i = 0; i < NHI; ++i) {
+    int x, y;
+    mol_flux_halo<G, 2, 2>(min((int)threadIdx.x + i * G::NTHR, NH - 1), x, y);   // (past the last: it again)
+    hc[i].at(X0 + x, Y0 + y);
+    ho[i] = (x + 2) + Q::LX * (y + 2);
+    mol_flux_load<G, false>(hv[i], hc[i], u, jp, z0);
+  }
+#pragma unroll
+  for (int k = 0; k < NI; ++k) {
+    const int q = (int)threadIdx.x + k * G::NTHR;
+    cy[k] = q / TX;
+    cx[k] = q - cy[k] * TX;
+    col[k].at(X0 + cx[k], Y0 + cy[k]);
+    T v[5][NA], w[4][NA];
+    mol_flux_planes<G, 5, 2, false>(v, col[k], X0 + cx[k], Y0 + cy[k], z0, u, jp, t, P);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        w[i][a] = v[i][a];
+        R[k][i][a] = v[i + 1][a];
+      }
+    Fz[k] = mol_flux_at<G, 2>(w, t, P);
+  }
+  for (int c = z0; c < z1; ++c) {
+    // the plane into LDS
+#pragma unroll
+    for (int k = 0; k < NI; ++k)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) S.L[a][(cx[k] + 2) + Q::LX * (cy[k] + 2)] = R[k][1][a];
+#pragma unroll
+    for (int i = 0; i < NHI; ++i)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) S.L[a][ho[i]] = hv[i][a];
+    // what the next plane and this plane's node program and update read, in flight during the fluxes
+    T nxt[NI][NA], av[NI][NQ], ea[NI], eb[NI], ec[NI];
+#pragma unroll
+    for (int i = 0; i < NHI; ++i) mol_flux_load<G, false>(hv[i], hc[i], u, jp, c + 1);
+    const i64 pu = PU * c, pa = PA * (c + 1);
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      mol_flux_load<G, false>(nxt[k], col[k], u, jp, c + 3);
+#pragma unroll
+      for (int a = 0; a < G::NAU; ++a) av[k][a] = mol_at(jp.aux[G::AN[a]] + pa, col[k].a);
+      ea[k] = eb[k] = ec[k] = T(0);
+      if (ep.mode != 0) {
+        if (ep.A) ea[k] = mol_at(ep.A + pu, col[k].u);
+        if (ep.B) eb[k] = mol_at(ep.B + pu, col[k].u);
+        if (ep.mode == 2) ec[k] = mol_at(ep.comp + pu, col[k].u);
+        else if (ep.acc && ep.acc_keep != 0.0) ec[k] = mol_at(ep.acc + pu, col[k].u);
+      }
+    }
+    __syncthreads();
+    mol_flux_sides<G, 2, 2, Q::LX>(&S.L[0][0], Q::LX * Q::LY, X0, Y0, c, t, P, jp);
+    T fx[NI], fy[NI], fz[NI];
+    auto face = [&](const int ax, const int x, const int y) {
+      const int o = (x + 2) + Q::LX * (y + 2), st = ax == 0 ? 1 : Q::LX;
+      T w[4][NA];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) w[i][a] = S.L[a][o + (i - 1) * st];
+      return ax == 0 ? mol_flux_at<G, 0>(w, t, P) : mol_flux_at<G, 1>(w, t, P);
+    };
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      fx[k] = face(0, cx[k], cy[k]);
+      fy[k] = face(1, cx[k], cy[k]);
+      fz[k] = mol_flux_at<G, 2>(R[k], t, P);
+      S.FX[(cx[k] + 1) + (TX + 1) * cy[k]] = fx[k];
+      S.FY[cx[k] + TX * (cy[k] + 1)] = fy[k];
+    }
+    for (int q = (int)threadIdx.x; q < TX + TY; q += G::NTHR) {   // the lower sides of the tile
+      if (q < TY) S.FX[(TX + 1) * q] = face(0, -1, q);
+      else S.FY[q - TY] = face(1, q - TY, -1);
+    }
+    __syncthreads();
+    const int g = c + 3 - G::M2;
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      const int x = X0 + cx[k], y = Y0 + cy[k];
+      T sv[3], out;
+      sv[0] = G::wo(0, 0) * S.FX[cx[k] + (TX + 1) * cy[k]] + G::wo(0, 1) * fx[k];
+      sv[1] = G::wo(1, 0) * S.FY[cx[k] + TX * cy[k]] + G::wo(1, 1) * fy[k];
+      sv[2] = G::wo(2, 0) * Fz[k] + G::wo(2, 1) * fz[k];
+      Fz[k] = fz[k];
+      if (x < G::M0 && y < G::M1) {
+        G::node(R[k][1][0], sv, av[k], x + 2, y + 2, c + 2, t, P, jp, out);
+        const unsigned i = col[k].u;
+        if (ep.mode == 0) {
+          mol_at(ep.out + pu, i) = out;
+        } else if (ep.mode == 1) {
+          T v = (T)ep.cf * out;
+          if (ep.A) v += (T)ep.ca * ea[k];
+          if (ep.B) v += (T)ep.cb * eb[k];
+          if (ep.acc) {
+            T a = (T)ep.acc_f * out;
+            if (ep.acc_keep != 0.0) a += (T)ep.acc_keep * ec[k];
+            mol_at(ep.acc + pu, i) = a;
+          }
+          mol_at(ep.out + pu, i) = v;
+        } else {
+          T incr = (T)ep.cf * out;
+          if (ep.B) incr += (T)ep.cb * (ep.subA ? (eb[k] - ea[k]) : eb[k]);
+          const T yk = incr - ec[k];
+          const T s = ea[k] + yk;
+          mol_at(ep.comp + pu, i) = (s - ea[k]) - yk;
+          mol_at(ep.out + pu, i) = s;
+        }
+      }
+      if (g == 0 || g == 1) {
+        const T bv = mol_flux_bval<G>(2, 1, x, y, G::M2, t, P, jp);
+        mol_flux_above<G>(nxt[k], R[k][0], R[k][1], R[k][2], R[k][3], g, bv);
+      }
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        R[k][0][a] = R[k][1][a];
+        R[k][1][a] = R[k][2][a];
+        R[k][2][a] = R[k][3][a];
+        R[k][3][a] = nxt[k][a];
+      }
+    }
+  }
+}
+
+// Reverse mode of the march: lam_dot = (df/du)^T lam and the gradients of the grid fields, each
+// node's sum complete in one thread (no atomics, no per-tile buffers, no gather).  With
+// phi = wo1 lam(h) + wo0 lam(h+1) the adjoint of the flux at half point h (lam = 0 outside the
+// unknowns), a half point leaves p = phi dF/d(u_h), q = phi dF/d(inner derivative) and
+// r_a = phi dF/d(aux_h); a position's adjoint is the transposed interpolation and difference of the
+// half points around it, and what the boundary and extrapolated positions get goes back to the
+// nodes they are made of.  Columns within three of a side see its half points: faces -2 .. TX + 1
+// of the tile are evaluated, from a halo of three positions below and four above.  Along z a half
+// point adds to the sums of its four planes, which a thread holds open: plane c is finished when
+// half point c + 1 is in.  Sums in FP64.
+template <class G>
+struct MolFluxAdj {   // what a half point leaves
+  T p, q, r[G::NAH > 0 ? G::NAH : 1];
+};
+template <class G>
+struct MolFluxVLds {
+  static constexpr int LX = G::TX + 7, LY = G::TY + 7, NA = 1 + G::NAH, NC = G::TX * G::TY;
+  static constexpr int FXN = (G::TX + 4) * G::TY, FYN = G::TX * (G::TY + 4), NR = 2 + G::NAH;
+  T L[NA + 1][LX * LY];   // staged arrays, then the seed
+  T FX[NR][FXN], FY[NR][FYN];
+};
+
+template <class G, int AX>
+__device__ __forceinline__ MolFluxAdj<G> mol_flux_rev(const T (&w)[4][1 + G::NAH], const T l0, const T l1,
+                                                      const double t, const T* __restrict__ P) {
+  T h[1 + G::NAH], d;
+  mol_flux_half<G>(AX, w, h, d);
+  T phi = G::wo(AX, 1) * l0;
+  phi += G::wo(AX, 0) * l1;
+  MolFluxAdj<G> o;
+  G::template dflux<AX>(h, d, phi * G::ws(AX), t, P, o.p, o.r, o.q);
+  return o;
+}
+
+// Adjoint of position j along an axis from the half points j - 2 .. j + 1 (f[0] .. f[3]): of the
+// state (R < 0) or of grid field R.
+template <class G, int R>
+__device__ __forceinline__ double mol_flux_tr(const int ax, const MolFluxAdj<G> (&f)[4]) {
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s += (double)G::wi(ax, 3 - i) * (double)(R < 0 ? f[i].p : f[i].r[R < 0 ? 0 : R]);
+  if (R < 0) {
+    s += (double)G::wd(ax, 0) * (double)f[2].q;
+    s += (double)G::wd(ax, 1) * (double)f[1].q;
+  }
+  return s;
+}
+
+// One side's part of a node at distance m (0 .. 2) from it: e0, e1 the side's own half point and the
+// next one inside; edge(a, value): the gradient of a grid field at the boundary node.
+template <class G, int AX, int SIDE, class EDGE>
+__device__ __forceinline__ void mol_flux_back(const int m, const MolFluxAdj<G>& e0, const MolFluxAdj<G>& e1, double& ub,
+                                              double (&da)[G::NAH > 0 ? G::NAH : 1], const bool ga, const EDGE& edge) {
+  MolFluxAdj<G> f[4] = {};
+  f[SIDE == 0 ? 2 : 1] = e0;
+  f[SIDE == 0 ? 3 : 0] = e1;
+  const double we = (double)G::wi(AX, SIDE == 0 ? 0 : 3);
+  auto pick = [&](const T a, const T b, const T c) { return (double)(m == 0 ? a : (m == 1 ? b : c)); };
+  ub += pick(G::closure(AX, SIDE, 0, 0), G::closure(AX, SIDE, 0, 1), G::closure(AX, SIDE, 0, 2)) * mol_flux_tr<G, -1>(AX, f) +
+        pick(G::closure(AX, SIDE, 1, 0), G::closure(AX, SIDE, 1, 1), G::closure(AX, SIDE, 1, 2)) * (we * (double)e0.p);
+  if (ga) {
+    const double ex = pick(G::ext(AX, SIDE, 1), G::ext(AX, SIDE, 2), G::ext(AX, SIDE, 3));
+    if constexpr (G::NAH > 0) {
+      const double v = we * (double)e0.r[0];
+      da[0] += ex * v;
+      if (m == 0) edge(0, mol_flux_tr<G, 0>(AX, f) + (double)G::ext(AX, SIDE, 0) * v);
+    }
+    if constexpr (G::NAH > 1) {
+      const double v = we * (double)e0.r[1];
+      da[1] += ex * v;
+      if (m == 0) edge(1, mol_flux_tr<G, 1>(AX, f) + (double)G::ext(AX, SIDE, 0) * v);
+    }
+  }
+}
+
+// The part of the x or y axis of a node at coordinate v of M: at(i) returns half point v + i, -2 <= i <= 2
+// (zero outside -1 .. M-1); edge(side, a, value): the gradient of a grid field at a boundary node.
+template <class G, int AX, class AT, class EDGE>
+__device__ __forceinline__ void mol_flux_axis(const int v, const AT& at, double& ub,
+                                              double (&da)[G::NAH > 0 ? G::NAH : 1], const bool ga, const EDGE& edge) {
+  constexpr int M = AX == 0 ? G::M0 : G::M1;
+  {
+    const MolFluxAdj<G> f[4] = {at(-2), at(-1), at(0), at(1)};
+    ub += mol_flux_tr<G, -1>(AX, f);
+    if (ga) {
+      if constexpr (G::NAH > 0) da[0] += mol_flux_tr<G, 0>(AX, f);
+      if constexpr (G::NAH > 1) da[1] += mol_flux_tr<G, 1>(AX, f);
+    }
+  }
+  if (v <= 2)
+    mol_flux_back<G, AX, 0>(v, at(-1 - v), at(-v), ub, da, ga, [&](const int a, const double x) { edge(0, a, x); });
+  if (M - 1 - v <= 2)
+    mol_flux_back<G, AX, 1>(M - 1 - v, at(M - 1 - v), at(M - 2 - v), ub, da, ga,
+                            [&](const int a, const double x) { edge(1, a, x); });
+}
+
+template <class G>
+__device__ __forceinline__ void mol_flux_vjp(MolFluxVLds<G>& S, const VArgs& va, const JPtrs& jp, const double t) {
+  typedef MolFluxVLds<G> Q;
+  typedef MolFluxAdj<G> F;
+  constexpr int TX = G::TX, TY = G::TY, NA = Q::NA, NI = Q::NC / G::NTHR, NH = 7 * (TX + TY);
+  constexpr int NHI = (NH + G::NTHR - 1) / G::NTHR, NAD = G::NAH > 0 ? G::NAH : 1, NQ = G::NAU > 0 ? G::NAU : 1;
+  constexpr int NAG = G::NAG > 0 ? G::NAG : 1;
+  constexpr i64 PU = (i64)G::M0 * G::M1, PA = (i64)G::N0 * G::N1;
+  const int b = mol_xcd_tile<G::NBLK>((int)blockIdx.x);
+  const int X0 = (b % G::NT0) * TX, Y0 = (b / G::NT0 % G::NT1) * TY, zc = b / (G::NT0 * G::NT1);
+  const int z0 = mol_flux_chunk<G>(zc), z1 = mol_flux_chunk<G>(zc + 1);
+  const T* const P = va.p;
+  const T* const u = va.u;
+  const bool ga = va.g_aux != nullptr, sum = (va.mode & 8) != 0;
+  // seed at plane z: its two parts as loaded, then put together (0 outside)
+  const T* const s2 = va.s2 ? va.s2 : va.s1;
+  auto raw = [&](T (&v)[2], const MolFluxCol<G>& c, const int z) {
+    const i64 o = PU * mol_uniform(min(max(z, 0), G::M2 - 1));
+    v[0] = mol_at_s(va.s1 + o, c.u);
+    v[1] = mol_at_s(s2 + o, c.u);
+  };
+  auto seed = [&](const T (&v)[2], const bool in, const int z) {
+    const T a = (T)va.c1 * v[0], b = a + (T)va.c2 * v[1];
+    return in && z >= 0 && z < G::M2 ? (va.s2 ? b : a) : T(0);
+  };
+  // a column's planes c .. c+3, seeds and open sums c .. c+2 (and c+3 with half point c+1); the halo
+  // of plane c
+  T R[NI][4][NA], Ls[NI][3], hv[NHI][NA], hs[NHI][2];
+  double ub[NI][4], da[NI][4][NAD];
+  int cx[NI], cy[NI], ho[NHI];
+  MolFluxCol<G> col[NI], hc[NHI];
+  bool in[NI], hin[NHI];
+  auto halo = [&](const int c) {
+#pragma unroll
+    for (int i = 0; i < NHI; ++i) {
+      mol_flux_load<G, true>(hv[i], hc[i], u, jp, c);
+      raw(hs[i], hc[i], c);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NHI; ++i) {
+    int x, y;
+    mol_flux_halo<G, 3, 4>(min((int)threadIdx.x + i * G::NTHR, NH - 1), x, y);
+    hc[i].at(X0 + x, Y0 + y);
+    ho[i] = (x + 3) + Q::LX * (y + 3);
+    hin[i] = X0 + x >= 0 && X0 + x < G::M0 && Y0 + y >= 0 && Y0 + y < G::M1;
+  }
+  halo(z0);
+  // adds to the gradient of the a-th interpolated field at a boundary node
+  auto edge = [&](const int a, const int px, const int py, const int pz, const double v) {
+    va.g_aux[G::AH[a] * G::NGRID + (i64)(px + 1) + (i64)G::N0 * ((py + 1) + (i64)G::N1 * (pz + 1))] += v;
+  };
+  // half point between open planes J + 1 and J + 2 along z into the sums J .. J + 3 (those there are)
+  auto push = [&](const int k, const F& f, const int J) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (J + i < 0) continue;
+      ub[k][J + i] += (double)G::wi(2, i) * (double)f.p;
+      if (i == 1 || i == 2) ub[k][J + i] += (double)G::wd(2, i - 1) * (double)f.q;
+#pragma unroll
+      for (int a = 0; a < G::NAH; ++a) da[k][J + i][a] += (double)G::wi(2, i) * (double)f.r[a];
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < NI; ++k) {
+    const int q = (int)threadIdx.x + k * G::NTHR;
+    cy[k] = q / TX;
+    cx[k] = q - cy[k] * TX;
+    const int x = X0 + cx[k], y = Y0 + cy[k];
+    in[k] = x < G::M0 && y < G::M1;
+    col[k].at(x, y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ub[k][i] = 0.0;
+#pragma unroll
+      for (int a = 0; a < NAD; ++a) da[k][i][a] = 0.0;
+    }
+    // planes z0-3 .. z0+3, half points z0-2 .. z0
+    T v[7][NA], lr[5][2], l[5];
+    F f[3];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) raw(lr[i], col[k], z0 - 2 + i);
+    mol_flux_planes<G, 7, 3, true>(v, col[k], x, y, z0, u, jp, t, P);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) l[i] = seed(lr[i], in[k], z0 - 2 + i);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      T w[4][NA];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) w[j][a] = v[i + j][a];
+      f[i] = mol_flux_rev<G, 2>(w, l[i], l[i + 1], t, P);
+      if (i == 0 && z0 == 0) f[i] = F{};   // (outside)
+      push(k, f[i], i - 3);
+      Ls[k][i] = l[2 + i];
+    }
+    if (z0 == 0 && in[k])
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+        mol_flux_back<G, 2, 0>(m, f[1], f[2], ub[k][m], da[k][m], ga,
+                               [&](const int a, const double e) { edge(a, x, y, -1, e); });
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) R[k][i][a] = v[3 + i][a];
+  }
+  // plane c into LDS: the columns' plane R[.][I] and the halo that was loaded
+  auto stage = [&](const int I, const int c) {
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      const int o = (cx[k] + 3) + Q::LX * (cy[k] + 3);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) S.L[a][o] = R[k][I][a];
+      S.L[NA][o] = Ls[k][I];
+    }
+#pragma unroll
+    for (int i = 0; i < NHI; ++i) {
+#pragma unroll
+      for (int a = 0; a < NA; ++a) S.L[a][ho[i]] = hv[i][a];
+      S.L[NA][ho[i]] = seed(hs[i], hin[i], c);
+    }
+  };
+  auto ag = [&](const int k) { return col[k].a * (unsigned)(sizeof(double) / sizeof(T)); };
+  stage(0, z0);
+  for (int c = z0; c < z1; ++c) {
+    // in flight during the half points: the next plane, the node's fields, the sums to add to
+    T nxt[NI][NA], nl[NI][2], av[NI][NQ], ys[NI][4];
+    double gv[NI][NAG];
+    const i64 pu = PU * mol_uniform(c), pa = PA * mol_uniform(c + 1);
+    halo(c + 1);
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      mol_flux_load<G, true>(nxt[k], col[k], u, jp, c + 4);
+      raw(nl[k], col[k], c + 3);
+#pragma unroll
+      for (int a = 0; a < G::NAU; ++a) av[k][a] = mol_at_s(jp.aux[G::AN[a]] + pa, col[k].a);
+      if (sum) {
+        ys[k][0] = mol_at_s((const T*)va.lam + pu, col[k].u);
+        ys[k][1] = mol_at_s(va.y0 + pu, col[k].u);
+        ys[k][2] = mol_at_s(va.y1 + pu, col[k].u);
+        ys[k][3] = mol_at_s(va.y2 + pu, col[k].u);
+      }
+      if (ga) {
+#pragma unroll
+        for (int a = 0; a < G::NAG; ++a) gv[k][a] = mol_at_s((const double*)va.g_aux + G::AG[a] * G::NGRID + pa, ag(k));
+      }
+    }
+    __syncthreads();
+    mol_flux_sides<G, 3, 4, Q::LX>(&S.L[0][0], Q::LX * Q::LY, X0, Y0, c, t, P, jp);
+    // half points of the plane along x and y: every column's upper sides, and faces -2, -1, TX,
+    // TX + 1 of the tile's rows and columns
+    auto face = [&](const int ax, const int x, const int y) {
+      const int o = (x + 3) + Q::LX * (y + 3), st = ax == 0 ? 1 : Q::LX;
+      const int h = ax == 0 ? X0 + x : Y0 + y;
+      T w[4][NA];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) w[i][a] = S.L[a][o + (i - 1) * st];
+      F f = ax == 0 ? mol_flux_rev<G, 0>(w, S.L[NA][o], S.L[NA][o + st], t, P)
+                    : mol_flux_rev<G, 1>(w, S.L[NA][o], S.L[NA][o + st], t, P);
+      if (h < -1 || h >= (ax == 0 ? G::M0 : G::M1)) f = F{};
+      T* const B = ax == 0 ? &S.FX[0][(x + 2) + (TX + 4) * y] : &S.FY[0][x + TX * (y + 2)];
+      const int N = ax == 0 ? Q::FXN : Q::FYN;
+      B[0] = f.p;
+      B[N] = f.q;
+#pragma unroll
+      for (int a = 0; a < G::NAH; ++a) B[(2 + a) * N] = f.r[a];
+    };
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      face(0, cx[k], cy[k]);
+      face(1, cx[k], cy[k]);
+    }
+    for (int q = (int)threadIdx.x; q < 4 * (TX + TY); q += G::NTHR) {
+      int x, y;
+      mol_flux_halo<G, 2, 2>(q, x, y);
+      if (q < 4 * TY) face(0, x, y);
+      else face(1, x, y);
+    }
+    __syncthreads();
+    stage(1, c + 1);   // (before this plane's stores: the wait for its halo is not one for them)
+    const int g = c + 4 - G::M2;
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {
+      const int x = X0 + cx[k], y = Y0 + cy[k];
+      if (g == 0 || g == 1) {
+        const T bv = mol_flux_bval<G>(2, 1, x, y, G::M2, t, P, jp);
+        mol_flux_above<G>(nxt[k], R[k][0], R[k][1], R[k][2], R[k][3], g, bv);
+      }
+      // along z: half point c + 1; before plane M2 - 3 is finished what its side gives back
+      if (c + 1 < G::M2) {
+        const F f = mol_flux_rev<G, 2>(R[k], Ls[k][1], Ls[k][2], t, P);
+        push(k, f, 0);
+        if (c == G::M2 - 3 && in[k]) {
+          T w[4][NA];
+#pragma unroll
+          for (int a = 0; a < NA; ++a) {
+            w[0][a] = R[k][1][a];
+            w[1][a] = R[k][2][a];
+            w[2][a] = R[k][3][a];
+            w[3][a] = nxt[k][a];
+          }
+          const F e = mol_flux_rev<G, 2>(w, Ls[k][2], T(0), t, P);
+#pragma unroll
+          for (int m = 0; m < 3; ++m)
+            mol_flux_back<G, 2, 1>(m, e, f, ub[k][2 - m], da[k][2 - m], ga,
+                                   [&](const int a, const double v) { edge(a, x, y, G::M2, v); });
+        }
+      }
+      if (in[k]) {
+        double dg[NAG] = {};
+        auto from = [&](const T* const B, const int N) {
+          F f;
+          f.p = B[0];
+          f.q = B[N];
+#pragma unroll
+          for (int a = 0; a < NAD; ++a) f.r[a] = a < G::NAH ? B[(2 + a) * N] : T(0);
+          return f;
+        };
+        mol_flux_axis<G, 0>(x, [&](const int i) { return from(&S.FX[0][cx[k] + 2 + i + (TX + 4) * cy[k]], Q::FXN); },
+                            ub[k][0], da[k][0], ga,
+                            [&](const int side, const int a, const double v) { edge(a, side ? G::M0 : -1, y, c, v); });
+        mol_flux_axis<G, 1>(y, [&](const int i) { return from(&S.FY[0][cx[k] + TX * (cy[k] + 2 + i)], Q::FYN); },
+                            ub[k][0], da[k][0], ga,
+                            [&](const int side, const int a, const double v) { edge(a, x, side ? G::M1 : -1, c, v); });
+        // the node's own terms
+        G::dnode(R[k][0][0], Ls[k][0], av[k], x + 2, y + 2, c + 2, t, P, jp, ub[k][0], dg);
+        if (ga) {
+#pragma unroll
+          for (int a = 0; a < G::NAH; ++a) dg[G::HG[a]] += da[k][0][a];
+#pragma unroll
+          for (int a = 0; a < G::NAG; ++a)
+            mol_at_s(va.g_aux + G::AG[a] * G::NGRID + pa, ag(k)) = gv[k][a] + dg[a];
+        }
+        mol_at_s(va.out + pu, col[k].u) = sum ? (((ys[k][0] + ys[k][1]) + ys[k][2]) + ys[k][3]) + (T)ub[k][0] : (T)ub[k][0];
+      }
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        R[k][0][a] = R[k][1][a];
+        R[k][1][a] = R[k][2][a];
+        R[k][2][a] = R[k][3][a];
+        R[k][3][a] = nxt[k][a];
+      }
+      Ls[k][0] = Ls[k][1];
+      Ls[k][1] = Ls[k][2];
+      Ls[k][2] = seed(nl[k], in[k], c + 3);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ub[k][i] = i < 3 ? ub[k][i < 3 ? i + 1 : 0] : 0.0;
+#pragma unroll
+        for (int a = 0; a < NAD; ++a) da[k][i][a] = i < 3 ? da[k][i < 3 ? i + 1 : 0][a] : 0.0;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Batched instances.  Each instance of a batch has a header with its grid sizes, unknown
 // boxes (offsets into the batch state vector), tile counts and tile classes, and pointers to
 // its weight pool W (the descriptor's pool), constants K (the constant pool, then eps and
