@@ -302,7 +302,8 @@ int mol_integrate_noalloc(mol_handle* h, void* u, const void* p, double t0, doub
  * (g_aux may be NULL).  u, lam, lam_dot: unknown vectors; g_aux: naux full-grid FP64 arrays.
  * Each tile writes its tile + halo adjoints to its own buffer and a gather kernel adds the
  * buffers of the tiles covering each node in a fixed order; only adjoints of ghost nodes reach
- * the unknowns with atomics (through the transposed closures). */
+ * the unknowns with atomics (through the transposed closures).  Large 3D systems in divergence
+ * form finish every sum in one thread instead (no buffers, no atomics). */
 int mol_vjp(mol_handle* h, const void* u, const void* p, double t, const void* lam, void* lam_dot,
             double* g_aux, void* stream);
 
@@ -315,8 +316,9 @@ int mol_forward_checkpointed(mol_handle* h, void* u, const void* p, double t0, d
 
 /* mol_adjoint: discrete adjoint of the last checkpointed RK4 run.  On entry lam = dL/du(T);
  * on exit lam = dL/du(t0) and g_aux += dL/daux (FP64).  Each segment between checkpoints is
- * recomputed forward once (stage states kept on the device), then swept backwards with four
- * VJPs per step; after a ckpt_every = 0 run the sweep uses the stored stage states. */
+ * recomputed forward once (stage states kept on the device; those of the last segment are
+ * there from the run where its steps were not fused), then swept backwards with four VJPs per
+ * step; after a ckpt_every = 0 run the sweep uses the stored stage states. */
 int mol_adjoint(mol_handle* h, const void* p, void* lam, double* g_aux, void* stream);
 
 /* FP64 error norms of a state against a reference, the counterpart of the final-time error checks

@@ -1411,6 +1411,44 @@ int rk4_step_store(mol_handle* h, const T* p, const T* uin, T* y1, T* y2, T* y3,
   return 0;
 }
 
+// Device memory for u and the three stage states of nsteps steps; nonzero when it does not fit
+// (what was there is gone then).
+int segment_memory(mol_handle* h, int64_t nsteps) {
+  const size_t need = (size_t)(4 * nsteps + 1);
+  if (h->seg_cap >= need) return 0;
+  if (h->seg_u) (void)hipFree(h->seg_u);
+  if (h->seg_t) (void)hipFree(h->seg_t);
+  h->seg_u = nullptr;
+  h->seg_t = nullptr;
+  h->seg_cap = 0;
+  if (hipMalloc(&h->seg_u, need * h->nunk * h->esize()) != hipSuccess ||
+      hipMalloc((void**)&h->seg_t, (size_t)(nsteps + 1) * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
+    if (h->seg_u) (void)hipFree(h->seg_u);
+    h->seg_u = nullptr;
+    h->seg_t = nullptr;
+    return 1;
+  }
+  h->seg_cap = need;
+  return 0;
+}
+
+// len steps from u0 (time from the device clock) keeping every stage state and step time in the
+// segment's memory; the state after the last goes to uout.
+template <typename T>
+int segment_steps(mol_handle* h, const T* p, const T* u0, int64_t len, double dt, T* uout, hipStream_t s) {
+  const int64_t n = h->nunk;
+  T* S = (T*)h->seg_u;
+  auto st = [&](int64_t j, int k) { return S + (size_t)(4 * j + k) * n; };
+  HIPCHK(h, hipMemcpyAsync(st(0, 0), u0, (size_t)n * sizeof(T), hipMemcpyDeviceToDevice, s));
+  for (int64_t j = 0; j < len; ++j) {
+    HIPCHK(h, hipMemcpyAsync(h->seg_t + j, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
+    if (int rc = rk4_step_store<T>(h, p, st(j, 0), st(j, 1), st(j, 2), st(j, 3), j + 1 < len ? st(j + 1, 0) : uout, dt, s))
+      return rc;
+  }
+  return 0;
+}
+
 template <typename T>
 int forward_ckpt_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int64_t nsteps, int32_t every,
                       hipStream_t s) {
@@ -1421,31 +1459,11 @@ int forward_ckpt_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int
   if (every == 0) {
     // keep u and the three stage states of every step: the adjoint then runs no forward
     // recomputation (4 * nsteps state vectors of device memory)
-    const size_t need = (size_t)(4 * nsteps + 1);
-    if (h->seg_cap < need) {
-      if (h->seg_u) (void)hipFree(h->seg_u);
-      if (h->seg_t) (void)hipFree(h->seg_t);
-      h->seg_u = nullptr;
-      h->seg_t = nullptr;
-      h->seg_cap = 0;
-      if (hipMalloc(&h->seg_u, need * vbytes) != hipSuccess) {
-        (void)hipGetLastError();
-        h->seg_u = nullptr;
-        return fail(h, MOL_ERR_HIP, "not enough device memory to keep every stage state (use ckpt_every >= 1)");
-      }
-      HIPCHK(h, hipMalloc((void**)&h->seg_t, (size_t)(nsteps + 1) * sizeof(double)));
-      h->seg_cap = need;
-    }
-    const int64_t n = h->nunk;
-    T* S = (T*)h->seg_u;
-    auto st = [&](int64_t j, int k) { return S + (size_t)(4 * j + k) * n; };
+    if (segment_memory(h, nsteps))
+      return fail(h, MOL_ERR_HIP, "not enough device memory to keep every stage state (use ckpt_every >= 1)");
+    h->ck_last = false;
     if (launch_set_clock(h->d_tnow + h->clk, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
-    HIPCHK(h, hipMemcpyAsync(st(0, 0), u, vbytes, hipMemcpyDeviceToDevice, s));
-    for (int64_t j = 0; j < nsteps; ++j) {
-      HIPCHK(h, hipMemcpyAsync(h->seg_t + j, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
-      rc = rk4_step_store<T>(h, p, st(j, 0), st(j, 1), st(j, 2), st(j, 3), j + 1 < nsteps ? st(j + 1, 0) : u, dt, s);
-      if (rc) return rc;
-    }
+    if ((rc = segment_steps<T>(h, p, u, nsteps, dt, u, s))) return rc;
     h->ck_nsteps = nsteps;
     h->ck_every = (int32_t)std::min<int64_t>(nsteps, INT32_MAX);
     h->ck_dt = dt;
@@ -1465,12 +1483,17 @@ int forward_ckpt_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int
     h->ck_cap = (size_t)nseg;
   }
   h->ck_valid = false;
+  // The last segment keeps its stage states for the sweep that starts there (the adjoint needs their
+  // memory in any case), where the steps are stage launches anyway: 32 of 192 right-hand sides of a
+  // gradient over 24 steps with checkpoints every 8.  Systems with fused steps run those instead.
+  h->ck_last = !h->fused_fn && segment_memory(h, std::min<int64_t>(every, nsteps)) == 0;
   if (launch_set_clock(h->d_tnow + h->clk, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
   for (int64_t g = 0; g < nseg; ++g) {
     const int64_t len = std::min<int64_t>(every, nsteps - g * every);
     HIPCHK(h, hipMemcpyAsync((char*)h->ck_u + g * vbytes, u, vbytes, hipMemcpyDeviceToDevice, s));
     HIPCHK(h, hipMemcpyAsync(h->ck_t + g, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
-    rc = enqueue_steps<T>(h, handle_work(h), u, p, dt, len, MOL_RK4, false, s);
+    if (g == nseg - 1 && h->ck_last) rc = segment_steps<T>(h, p, u, len, dt, u, s);
+    else rc = enqueue_steps<T>(h, handle_work(h), u, p, dt, len, MOL_RK4, false, s);
     if (rc) return rc;
   }
   h->ck_nsteps = nsteps;
@@ -1494,18 +1517,8 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
   const double dt = h->ck_dt;
   const int64_t n = h->nunk;
   const size_t vbytes = (size_t)n * h->esize();
-  const size_t need = (size_t)(4 * every + 1);
-  if (h->ck_stored && h->seg_cap < need) return fail(h, MOL_ERR_INVALID, "stored stage states were released");
-  if (h->seg_cap < need) {
-    if (h->seg_u) (void)hipFree(h->seg_u);
-    if (h->seg_t) (void)hipFree(h->seg_t);
-    h->seg_u = nullptr;
-    h->seg_t = nullptr;
-    h->seg_cap = 0;
-    HIPCHK(h, hipMalloc(&h->seg_u, need * vbytes));
-    HIPCHK(h, hipMalloc((void**)&h->seg_t, (size_t)(every + 1) * sizeof(double)));
-    h->seg_cap = need;
-  }
+  if (h->ck_stored && h->seg_cap < (size_t)(4 * every + 1)) return fail(h, MOL_ERR_INVALID, "stored stage states were released");
+  if (segment_memory(h, std::min<int64_t>(every, nsteps))) return fail(h, MOL_ERR_HIP, "not enough device memory for the stage states of a segment");
   for (int k = 0; k < 4; ++k)
     if (!h->adj_y[k]) HIPCHK(h, hipMalloc(&h->adj_y[k], vbytes));
   T* const lam_user = lam;
@@ -1523,16 +1536,13 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
   for (int64_t g = nseg - 1; g >= 0; --g) {
     const int64_t len = std::min<int64_t>(every, nsteps - g * every);
     // recompute the segment from its checkpoint, keeping every stage state and step time
-    // (a run that kept them all is one segment with nothing to recompute)
-    if (!h->ck_stored) {
-      HIPCHK(h, hipMemcpyAsync(st(0, 0), (char*)h->ck_u + g * vbytes, vbytes, hipMemcpyDeviceToDevice, s));
+    // (a run that kept them all is one segment with nothing to recompute, and the last segment's are
+    // there on the first sweep of a run)
+    if (!h->ck_stored && !(h->ck_last && g == nseg - 1)) {
+      h->ck_last = false;   // its memory is taken
       HIPCHK(h, hipMemcpyAsync(h->d_tnow + h->clk, h->ck_t + g, sizeof(double), hipMemcpyDeviceToDevice, s));
-    }
-    for (int64_t j = 0; !h->ck_stored && j < len; ++j) {
-      HIPCHK(h, hipMemcpyAsync(h->seg_t + j, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
       // the state after the segment is not needed: it goes to the integrator's scratch
-      rc = rk4_step_store<T>(h, p, st(j, 0), st(j, 1), st(j, 2), st(j, 3), j + 1 < len ? st(j + 1, 0) : (T*)h->w_y2,
-                             dt, s);
+      rc = segment_steps<T>(h, p, (const T*)((char*)h->ck_u + g * vbytes), len, dt, (T*)h->w_y2, s);
       if (rc) return rc;
     }
     // backward sweep: k4 = f(y3, t+dt), k3 = f(y2, t+dt/2), k2 = f(y1, t+dt/2), k1 = f(u, t)

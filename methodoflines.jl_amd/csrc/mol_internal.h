@@ -234,6 +234,7 @@ struct mol_handle {
   double ck_dt = 0.0;
   bool ck_valid = false;
   bool ck_stored = false;                 // the run kept every stage state (no recomputation)
+  bool ck_last = false;                   // the stage states of the last segment are in seg_u
   void* seg_u = nullptr;                  // stage states of one recomputed segment (or the whole run)
   double* seg_t = nullptr;                // device clock at each step of the segment
   size_t seg_cap = 0;

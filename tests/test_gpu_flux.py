@@ -113,3 +113,28 @@ def test_result_over_its_own_seed(monkeypatch):
         assert rc == 0
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("n,steps,every", [(12, 5, 2), (12, 4, 9), (19, 6, 3)])
+def test_second_adjoint_of_a_run(n, steps, every, monkeypatch):
+    """The first sweep of a run uses the stage states of its last segment, later ones recompute
+    them: same bits, and those of a run that kept every state."""
+    import torch
+    prob = _problem(systems.nonlindiff3d(n), 1, monkeypatch)
+    N = prob.lowered.n_unknowns
+    rng = np.random.default_rng(4)
+    u0, lam0 = _dev(rng.uniform(-1, 1, N), torch.float64), _dev(rng.standard_normal(N), torch.float64)
+    res = []
+    for ev in (0, every):
+        u = u0.clone()
+        print("  flux second adjoint n=%d every=%d" % (n, ev), flush=True)
+        prob.forward_checkpointed(u, 0.0, 1e-5, steps, ev)
+        for rep in range(1 if ev == 0 else 3):
+            lam = lam0.clone()
+            g = torch.zeros(2 * n ** 3, dtype=torch.float64, device="cuda")
+            prob.adjoint(lam, g_aux=g)
+            res.append((u, lam, g))
+    torch.cuda.synchronize()
+    for r in res[1:]:
+        for a, b in zip(r, res[0]):
+            assert torch.equal(a, b)
