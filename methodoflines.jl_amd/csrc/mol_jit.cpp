@@ -431,10 +431,19 @@ class Gen {
     // 3D tiles: no blocking (128^3 nonlinear diffusion, 16x8x8 tile, 512 threads: 31.3 us with
     // two nodes per thread in turn, 37.7 us with two z-neighbours blocked in registers)
     if (!e && d_->ndim == 3) return;
-    // 2D work-groups of 512 threads (64x32 tiles under reach-two stencils): two nodes per
+    // 2D work-groups of 512 threads (64x32 tiles under reach-two stencils): FP64 two nodes per
     // thread in registers, two node groups in turn (four in registers: 10.3 against 9.1 us for
-    // the Burgers WENO5 right-hand side at 1024^2)
-    const int want = e ? std::max(1, std::atoi(e)) : (g_.nthr >= 512 ? 2 : 4);
+    // the Burgers WENO5 right-hand side at 1024^2).  WENO5 in FP32 with tiles that the box cuts: one,
+    // four groups in turn (4100^2 80.3 -> 73.6 us, 2900^2 43.1 -> 39.8; whole tiles, 4096^2: 73.2
+    // against 70.9 with two; FP64 46.3 -> 47.5 at 2900^2; fourth-order diffusion 18.8 -> 22.3).  One
+    // also for its tiles of 28, 20 or 12 rows.
+    bool weno = false;
+    for (int k = 0; k < d_->nslots; ++k) weno = weno || d_->slots_h[k].kind == MOL_SLOT_WENO;
+    weno = weno && d_->ndim == 2 && g_.halo[0] >= 2 && g_.halo[1] >= 2;
+    bool cut = false;
+    for (int a = 0; a < 2; ++a) cut = cut || (g_.uhi[a] - g_.ulo[a] + 1) % g_.tile[a] != 0;
+    const bool one = weno && ((g_.nthr >= 512 && d_->dtype != MOL_F64 && cut) || (g_.tile[0] == 64 && g_.tile[1] % 8 == 4));
+    const int want = e ? std::max(1, std::atoi(e)) : (one ? 1 : g_.nthr >= 512 ? 2 : 4);
     for (int r = want; r > 1; r /= 2)
       if (g_.tile[ba] % r == 0 && (e || vol / r >= g_.nthr)) {
         rb = r;
