@@ -868,9 +868,10 @@ bool sweep_source(mol_handle* h, const mol_desc* d, JitGeom& g, std::string& src
 // size rule is against it.  MOL_FLUX=0 or 1 overrides the size rule, MOL_FLUX_TILE=tx,ty,planes and
 // MOL_FLUX_VJP_TILE ask for other columns and chunks.
 //
-// Size: from 2^17 unknowns, and not where half of the columns or more would be padding.  Fewer leave
-// compute units without a work-group.  Per right-hand side and per reverse step with its gradients
-// (FP64, us, tiles -> march): 46^3 6.5 -> 7.3 and 19.7 -> 13.5, 54^3 8.4 -> 6.9 and 23.1 -> 13.7,
+// Size: forward from 48^3 unknowns, reverse from 2^16, and not where half of the columns or more
+// would be padding.  Fewer leave compute units without a work-group.  Per right-hand side and per
+// reverse step with its gradients (FP64, us, tiles -> march): 28^3 5.7 -> 6.9 and 13.4 -> 13.6, 44^3
+// 6.7 -> 7.3 and 16.6 -> 13.6, 48^3 6.8 -> 6.4 and 16.4 -> 14.2, 52^3 7.9 -> 7.1 and 21.1 -> 13.8,
 // 126^3 31 -> 22 and 105 -> 47, 254^3 254 -> 209 and 954 -> 386.
 // Columns per work-group: 32 x 8 forward (a row of 32 is read in whole lines), 16 x 16 in reverse
 // mode, whose halo of seven costs less there.
@@ -894,7 +895,7 @@ bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool
   for (int a = 0; a < 3; ++a) m[a] = g.n[a] - 2;
   if (m[0] < 3 || m[1] < 3 || m[2] < 3) return false;
   const long long nt = (long long)((m[0] + tile[0] - 1) / tile[0]) * ((m[1] + tile[1] - 1) / tile[1]);
-  if (!force && ((long long)m[0] * m[1] * m[2] < (1 << 17) || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
+  if (!force && ((long long)m[0] * m[1] * m[2] < (vjp ? 1 << 16 : 48 * 48 * 48) || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
   if (tile[2] == 0) {
     const int occ = vjp ? (f64 ? 3 : 4) : (f64 ? 5 : 8);   // resident work-groups per compute unit
     double best = 0.0;

@@ -138,3 +138,30 @@ def test_second_adjoint_of_a_run(n, steps, every, monkeypatch):
     for r in res[1:]:
         for a, b in zip(r, res[0]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [42, 43, 49, 50])
+def test_sizes_at_the_lines_of_the_rule(n, monkeypatch):
+    """Tiles in both directions, march in the reverse direction only, march in both."""
+    import torch
+    steps, dt = 3, 1e-6
+    res = []
+    for flux in ("0", None):
+        if flux is None:
+            monkeypatch.delenv("MOL_FLUX", raising=False)
+        else:
+            monkeypatch.setenv("MOL_FLUX", flux)
+        prob = molgpu.discretize(*systems.nonlindiff3d(n))
+        rng = np.random.default_rng(n)
+        for a in prob.lowered.aux:
+            prob.set_grid_field(a, rng.uniform(0.5, 1.5, prob.lowered.n))
+        N = prob.lowered.n_unknowns
+        u, lam = _dev(rng.uniform(-0.5, 0.5, N), torch.float64), _dev(rng.standard_normal(N), torch.float64)
+        g = torch.zeros(2 * n ** 3, dtype=torch.float64, device="cuda")
+        print("  flux rule n=%d flux=%s" % (n, flux), flush=True)
+        prob.forward_checkpointed(u, 0.0, dt, steps, 2)
+        prob.adjoint(lam, g_aux=g)
+        torch.cuda.synchronize()
+        res.append([v.cpu().numpy() for v in (u, lam, g)])
+    for a, b in zip(*res):
+        assert np.max(np.abs(b - a)) <= 1e-12 * np.max(np.abs(a))
