@@ -1404,14 +1404,13 @@ int launch_vjp(mol_handle* h, const VArgs<T>& va, hipStream_t s, bool tiles = tr
   return 0;
 }
 
-// One RK4 step from uin that keeps the stage states y1, y2, y3 and writes u_{n+1} to uout;
-// the same arithmetic as the stage loop of enqueue_steps (time from the device clock).
+// One RK4 step from uin at time *tcur that keeps the stage states y1, y2, y3, writes u_{n+1} to uout
+// and the time after it to *tnxt; the same arithmetic as the stage loop of enqueue_steps.
 template <typename T>
 int rk4_step_store(mol_handle* h, const T* p, const T* uin, T* y1, T* y2, T* y3, T* uout, double dt,
-                   hipStream_t s) {
+                   const double* tcur, double* tnxt, hipStream_t s) {
   const Launch<T> L = launch_of<T>(h);
   T* acc = (T*)h->w_acc;
-  double* tcur = h->d_tnow + h->clk;
   Epi<T> e{};
   e.tnow = tcur;
   e.p = p;
@@ -1424,9 +1423,8 @@ int rk4_step_store(mol_handle* h, const T* p, const T* uin, T* y1, T* y2, T* y3,
   rc |= launch_rhs<T>(L, y2, e, s);
   Epi<T> l{};
   l.tnow = tcur; l.p = p; l.tofs = dt; l.mode = 1; l.out = uout; l.A = uin; l.ca = 1.0; l.B = acc;
-  l.cb = dt / 6; l.cf = dt / 6; l.tnext = h->d_tnow + (1 - h->clk); l.tadv = dt;
+  l.cb = dt / 6; l.cf = dt / 6; l.tnext = tnxt; l.tadv = dt;
   rc |= launch_rhs<T>(L, y3, l, s);
-  h->clk ^= 1;
   if (rc) return fail(h, MOL_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(hipGetLastError()));
   return 0;
 }
@@ -1453,19 +1451,19 @@ int segment_memory(mol_handle* h, int64_t nsteps) {
   return 0;
 }
 
-// len steps from u0 (time from the device clock) keeping every stage state and step time in the
-// segment's memory; the state after the last goes to uout.
+// len steps from u0 at time *t0 keeping every stage state and step time in the segment's memory
+// (u0 and t0 stay where they are: they stand for its first state and time); the state after the
+// last goes to uout.  The step times are the clock, so no step copies it.
 template <typename T>
-int segment_steps(mol_handle* h, const T* p, const T* u0, int64_t len, double dt, T* uout, hipStream_t s) {
+int segment_steps(mol_handle* h, const T* p, const T* u0, const double* t0, int64_t len, double dt, T* uout,
+                  hipStream_t s) {
   const int64_t n = h->nunk;
   T* S = (T*)h->seg_u;
   auto st = [&](int64_t j, int k) { return S + (size_t)(4 * j + k) * n; };
-  HIPCHK(h, hipMemcpyAsync(st(0, 0), u0, (size_t)n * sizeof(T), hipMemcpyDeviceToDevice, s));
-  for (int64_t j = 0; j < len; ++j) {
-    HIPCHK(h, hipMemcpyAsync(h->seg_t + j, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
-    if (int rc = rk4_step_store<T>(h, p, st(j, 0), st(j, 1), st(j, 2), st(j, 3), j + 1 < len ? st(j + 1, 0) : uout, dt, s))
+  for (int64_t j = 0; j < len; ++j)
+    if (int rc = rk4_step_store<T>(h, p, j ? st(j, 0) : u0, st(j, 1), st(j, 2), st(j, 3), j + 1 < len ? st(j + 1, 0) : uout,
+                                   dt, j ? h->seg_t + j : t0, h->seg_t + j + 1, s))
       return rc;
-  }
   return 0;
 }
 
@@ -1482,8 +1480,9 @@ int forward_ckpt_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int
     if (segment_memory(h, nsteps))
       return fail(h, MOL_ERR_HIP, "not enough device memory to keep every stage state (use ckpt_every >= 1)");
     h->ck_last = false;
-    if (launch_set_clock(h->d_tnow + h->clk, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
-    if ((rc = segment_steps<T>(h, p, u, nsteps, dt, u, s))) return rc;
+    if (launch_set_clock(h->seg_t, t0, s)) return fail(h, MOL_ERR_HIP, "clock launch failed");
+    HIPCHK(h, hipMemcpyAsync(h->seg_u, u, vbytes, hipMemcpyDeviceToDevice, s));
+    if ((rc = segment_steps<T>(h, p, (const T*)h->seg_u, h->seg_t, nsteps, dt, u, s))) return rc;
     h->ck_nsteps = nsteps;
     h->ck_every = (int32_t)std::min<int64_t>(nsteps, INT32_MAX);
     h->ck_dt = dt;
@@ -1512,7 +1511,8 @@ int forward_ckpt_impl(mol_handle* h, T* u, const T* p, double t0, double dt, int
     const int64_t len = std::min<int64_t>(every, nsteps - g * every);
     HIPCHK(h, hipMemcpyAsync((char*)h->ck_u + g * vbytes, u, vbytes, hipMemcpyDeviceToDevice, s));
     HIPCHK(h, hipMemcpyAsync(h->ck_t + g, h->d_tnow + h->clk, sizeof(double), hipMemcpyDeviceToDevice, s));
-    if (g == nseg - 1 && h->ck_last) rc = segment_steps<T>(h, p, u, len, dt, u, s);
+    if (g == nseg - 1 && h->ck_last)
+      rc = segment_steps<T>(h, p, (const T*)((char*)h->ck_u + g * vbytes), h->ck_t + g, len, dt, u, s);
     else rc = enqueue_steps<T>(h, handle_work(h), u, p, dt, len, MOL_RK4, false, s);
     if (rc) return rc;
   }
@@ -1558,11 +1558,12 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
     // recompute the segment from its checkpoint, keeping every stage state and step time
     // (a run that kept them all is one segment with nothing to recompute, and the last segment's are
     // there on the first sweep of a run)
+    const T* const u0 = h->ck_stored ? S : (const T*)((char*)h->ck_u + g * vbytes);
+    const double* const t0 = h->ck_stored ? h->seg_t : h->ck_t + g;
     if (!h->ck_stored && !(h->ck_last && g == nseg - 1)) {
       h->ck_last = false;   // its memory is taken
-      HIPCHK(h, hipMemcpyAsync(h->d_tnow + h->clk, h->ck_t + g, sizeof(double), hipMemcpyDeviceToDevice, s));
       // the state after the segment is not needed: it goes to the integrator's scratch
-      rc = segment_steps<T>(h, p, (const T*)((char*)h->ck_u + g * vbytes), len, dt, (T*)h->w_y2, s);
+      rc = segment_steps<T>(h, p, u0, t0, len, dt, (T*)h->w_y2, s);
       if (rc) return rc;
     }
     // backward sweep: k4 = f(y3, t+dt), k3 = f(y2, t+dt/2), k2 = f(y1, t+dt/2), k1 = f(u, t)
@@ -1573,7 +1574,7 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
       const double c2[4] = {0.0, dt, dt / 2, dt / 2};
       for (int q = 0; q < 4; ++q) {
         VArgs<T> va{};
-        va.u = st(j, stage_state[q]);
+        va.u = j == 0 && q == 3 ? u0 : st(j, stage_state[q]);
         va.s1 = lam;
         va.c1 = c1[q];
         va.s2 = q > 0 ? Y[q - 1] : nullptr;
@@ -1581,7 +1582,7 @@ int adjoint_impl(mol_handle* h, const T* p, T* lam, double* g_aux, hipStream_t s
         va.out = Y[q];
         va.g_aux = g_aux;
         va.p = p;
-        va.tnow = h->seg_t + j;
+        va.tnow = j ? h->seg_t + j : t0;
         va.tofs = tofs[q];
         va.mode = acc_aux ? (VJP_GATHER_F | VJP_ACC_A) : (VJP_GATHER_F | VJP_GATHER_A);
         if (q == 3 && h->vjp_store) {
