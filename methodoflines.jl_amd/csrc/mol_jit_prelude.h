@@ -1921,7 +1921,7 @@ __device__ __forceinline__ void mol_vjp_tile(T* L, double* Ab, double* Aa, const
 //
 // The reference evaluates the half-point flux a(...) du/dx on either side of a node; the flux on
 // a node's upper side is the one on the lower side of its neighbour.  A work-group owns TX x TY
-// columns and walks up ZC planes: along z a thread keeps the last planes and the last flux in
+// columns and walks up a chunk of planes: along z a thread keeps the last planes and the last flux in
 // registers, along x and y the plane lies in LDS with its halo, every thread evaluates the fluxes
 // on its upper sides and leaves them in LDS for the neighbours.  So a node costs three fluxes
 // instead of six, and the state is read once per plane and tile (with the halo columns) instead
