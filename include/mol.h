@@ -234,7 +234,10 @@ int mol_expand(mol_handle* h, void* full, const void* u, const void* p, double t
 int mol_create_batched(const mol_desc* const* ds, const double* const* params, int32_t ninst, const int32_t* tile,
                        mol_handle** out);
 
-/* Generated source of the kernel of a batch (no GPU needed); flags as mol_codegen. */
+/* Generated source of the kernel of a batch (no GPU needed); flags as mol_codegen, or
+ * MOL_CODEGEN_WAVES for the waves of its RK4 step instead: a line each of instance, class, first
+ * column of the window, first and end of the owned columns, first and end row, 0 (counted from the
+ * instance's first unknown); empty when the batch steps by stage launches. */
 int64_t mol_codegen_batched(const mol_desc* const* ds, const double* const* params, int32_t ninst, const int32_t* tile,
                             char* buf, int64_t buflen, int32_t flags);
 
@@ -345,7 +348,7 @@ void mol_destroy(mol_handle* h);
  * flags: MOL_CODEGEN_COMPILE also compiles it with hiprtc for gfx950 and fails when that does;
  * MOL_CODEGEN_VJP returns the reverse-mode (vector-Jacobian product) kernel instead,
  * MOL_CODEGEN_FUSED the fused RK4 step kernel (MOL_ERR_UNSUPPORTED when the system has none). */
-enum { MOL_CODEGEN_COMPILE = 1, MOL_CODEGEN_VJP = 2, MOL_CODEGEN_FUSED = 4 };
+enum { MOL_CODEGEN_COMPILE = 1, MOL_CODEGEN_VJP = 2, MOL_CODEGEN_FUSED = 4, MOL_CODEGEN_WAVES = 8 };
 int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t buflen, int32_t flags);
 
 /* Library / device information (for test harnesses). */

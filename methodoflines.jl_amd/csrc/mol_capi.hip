@@ -1660,8 +1660,9 @@ struct BatchPlan {
   int nclasses = 0;
   int tile[3] = {1, 1, 1};
   std::string src;
-  std::vector<int32_t> sweep;   // register sweep of a whole RK4 step: per wave instance, class and
-                                // window, first row, end row; empty when an instance does not qualify
+  // register sweep of a whole RK4 step: per wave instance, class, first column of its window, first
+  // and end of the columns it owns and of its rows, 0; empty when an instance does not qualify
+  std::vector<int32_t> sweep;
 };
 
 int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t ninst, const int32_t* tile,
@@ -1841,23 +1842,29 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
   src << "    default: break;\n    }\n  }\n}\n";
   if (sweep) {
     // a whole RK4 step per launch: a wave per window and strip of an instance, longest first
+    // (the windows of each instance follow its own x axis: a batch may mix periodic and other axes)
     const int nf = ds[0]->nfields;
     std::vector<std::pair<int, int>> box;
-    for (const BInst& b : P.hdr)
-      box.push_back({b.uhi[1] - b.ulo[1] + 1, sweep_windows(ds[0]->periodic[0], b.uhi[0] - b.ulo[0] + 1)});
+    for (int i = 0; i < ninst; ++i) {
+      const BInst& b = P.hdr[i];
+      box.push_back({b.uhi[1] - b.ulo[1] + 1, sweep_windows(ds[i]->periodic[0], b.uhi[0] - b.ulo[0] + 1)});
+    }
     int dev = 0;
     (void)hipGetDevice(&dev);
     const int rows = sweep_rows(dev, nf * (int)esize, box);
-    std::vector<std::array<int32_t, 4>> items;
+    std::vector<std::array<int32_t, 8>> items;
     for (int i = 0; i < ninst; ++i) {
       // strips of an instance as even as whole rows allow, four rows or more
       const int ny = box[i].first, ns = std::min((ny + rows - 1) / rows, ny / 4);
       for (int s = 0; s < ns; ++s)
-        for (int w = 0; w < box[i].second; ++w)
-          items.push_back({i, sw_cls[i] + 65536 * w, (int)((int64_t)ny * s / ns), (int)((int64_t)ny * (s + 1) / ns)});
+        for (int w = 0; w < box[i].second; ++w) {
+          std::array<int32_t, 8> it = {i, sw_cls[i], 0, 0, 0, (int)((int64_t)ny * s / ns), (int)((int64_t)ny * (s + 1) / ns), 0};
+          sweep_window(ds[i]->periodic[0], P.hdr[i].uhi[0] - P.hdr[i].ulo[0] + 1, w, it[2], it[3], it[4]);
+          items.push_back(it);
+        }
     }
-    std::stable_sort(items.begin(), items.end(), [](const std::array<int32_t, 4>& a, const std::array<int32_t, 4>& b) {
-      return a[3] - a[2] > b[3] - b[2];
+    std::stable_sort(items.begin(), items.end(), [](const std::array<int32_t, 8>& a, const std::array<int32_t, 8>& b) {
+      return a[6] - a[5] > b[6] - b[5];
     });
     for (const auto& it : items) P.sweep.insert(P.sweep.end(), it.begin(), it.end());
     for (size_t c = 0; c < sw_src.size(); ++c) {
@@ -1873,7 +1880,7 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
              "    Epi ep, const BInst* __restrict__ insts, const int* __restrict__ wl) {\n"
              "  const double t = ep.tnow ? ep.tnow[0] : ep.tofs;\n"
              "  if (ep.tnext && blockIdx.x == 0 && threadIdx.x == 0) ep.tnext[0] = t + ep.tadv;\n"
-             "  const int* const it = wl + 4 * blockIdx.x;\n"
+             "  const int* const it = wl + 8 * blockIdx.x;\n"
              "  const BInst& in = insts[it[0]];\n"
           << "  constexpr int NF = " << nf << ";\n"
           << "  MolSHdr<NF> hd;\n  MolSweep<NF> g;\n  JPtrs jp{};\n"
@@ -1882,12 +1889,11 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
              "  for (int f = 0; f < NF; ++f) {\n    g.fofs[f] = in.fofs[f];\n"
              "    for (int s = 0; s < 4; ++s)\n      for (int m = 0; m < 3; ++m) hd.g[f][s][m] = (T)in.g[f][s][m];\n  }\n"
              "  g.nx = in.uhi[0] - in.ulo[0] + 1;\n  g.ny = in.uhi[1] - in.ulo[1] + 1;\n"
-             "  g.lo0 = in.ulo[0];\n  g.lo1 = in.ulo[1];\n  g.lo2 = 1;\n  g.y0 = it[2];\n  g.y1 = it[3];\n"
-             "  const int cls = it[1] & 0xffff, w = it[1] >> 16;\n";
+             "  g.lo0 = in.ulo[0];\n  g.lo1 = in.ulo[1];\n  g.lo2 = 1;\n  g.xb = it[2];\n  g.x0 = it[3];\n  g.x1 = it[4];\n  g.y0 = it[5];\n  g.y1 = it[6];\n"
+             "  const int cls = it[1];\n";
       for (size_t c = 0; c < sw_src.size(); ++c) {
         const std::string G = "SwpY" + std::to_string(c);
-        src << "  if (cls == " << c << ") {\n    mol_sweep_window<" << G << "::PER0 != 0, " << G << "::CX>(g, w);\n"
-            << "    mol_rk4_sweep<" << G << ", " << kahan << ">(hd, g, u, unew, ep, jp, t);\n  }\n";
+        src << "  if (cls == " << c << ") mol_rk4_sweep<" << G << ", " << kahan << ">(hd, g, u, unew, ep, jp, t);\n";
       }
       src << "}\n";
     }
@@ -1944,7 +1950,7 @@ int create_batched(const mol_desc* const* ds, const double* const* params, int32
       free_handle(h);
       return MOL_ERR_HIP;
     }
-    h->fused_tiles = (int)(P.sweep.size() / 4);
+    h->fused_tiles = (int)(P.sweep.size() / 8);
     h->fused_nthr = 64;
   }
   h->batch_grid = std::min(h->nwork, 1 << 24);
@@ -2022,12 +2028,18 @@ int64_t mol_codegen_batched(const mol_desc* const* ds, const double* const* para
     std::string log;
     if (jit_compile(P.src, code, log)) return fail(nullptr, MOL_ERR_HIP, "hiprtc: " + log);
   }
+  std::string& text = P.src;
+  if (flags & MOL_CODEGEN_WAVES) {
+    std::ostringstream o;
+    for (size_t k = 0; k < P.sweep.size(); ++k) o << P.sweep[k] << (k % 8 == 7 ? "\n" : " ");
+    text = o.str();
+  }
   if (buf && buflen > 0) {
-    const size_t n = std::min<size_t>(P.src.size(), (size_t)buflen - 1);
-    std::memcpy(buf, P.src.data(), n);
+    const size_t n = std::min<size_t>(text.size(), (size_t)buflen - 1);
+    std::memcpy(buf, text.data(), n);
     buf[n] = '\0';
   }
-  return (int64_t)P.src.size();
+  return (int64_t)text.size();
 }
 
 int mol_batch_offsets(const mol_handle* h, int64_t* offs, int32_t n) {

@@ -1,6 +1,7 @@
 // Host-side internals shared by the C-ABI translation units.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <string>
 #include <vector>
 #include "mol.h"
@@ -44,9 +45,15 @@ std::string jit_class_source(const mol_desc* d, const JitGeom& g, const std::str
 // instances; empty when the system does not qualify.
 std::string jit_sweep_source(const mol_desc* d, const JitGeom& g, std::string& err);
 std::string jit_sweep_class(const mol_desc* d, const JitGeom& g, const std::string& name, std::string& err);
-// Windows of columns over an axis of n unknowns (mol_sweep_windows of mol_jit_prelude.h).
+// Windows of columns over an axis of n unknowns, and window w's first and owned columns
+// (mol_sweep_windows and mol_sweep_window of mol_jit_prelude.h).
 inline int sweep_windows(bool per, int n) {
   return per ? (n + 55) / 56 : (n <= 64 ? 1 : (n - 8 + 55) / 56);
+}
+inline void sweep_window(bool per, int n, int w, int32_t& xb, int32_t& x0, int32_t& x1) {
+  xb = w * 56 - (per ? 4 : 0);
+  x0 = per ? w * 56 : (w == 0 ? 0 : xb + 4);
+  x1 = per || w < sweep_windows(per, n) - 1 ? std::min(n, xb + 60) : n;
 }
 
 // 3D divergence form marched along z, forward or reverse mode (tile: columns along x and y per

@@ -35,15 +35,17 @@ def _descs(lows: Sequence[Lowered]):
     return ds, ps, keep
 
 
-def codegen_batched(lows: Sequence[Lowered], compile: bool = False, tile=None) -> str:
-    """Source of the kernel of a batch (no GPU needed)."""
+def codegen_batched(lows: Sequence[Lowered], compile: bool = False, tile=None, waves: bool = False) -> str:
+    """Source of the kernel of a batch (no GPU needed), or with ``waves=True`` the waves of its RK4
+    step (``MOL_CODEGEN_WAVES`` in include/mol.h)."""
     lib = native.load_library()
     ds, ps, keep = _descs(lows)
     tl = (C.c_int32 * 3)(*tile) if tile is not None else None
-    n = lib.mol_codegen_batched(ds, ps, len(lows), tl, None, 0, 0)
+    what = 8 if waves else 0
+    n = lib.mol_codegen_batched(ds, ps, len(lows), tl, None, 0, what)
     native.check(lib, n if n < 0 else 0, None)
     buf = C.create_string_buffer(int(n) + 1)
-    n = lib.mol_codegen_batched(ds, ps, len(lows), tl, buf, len(buf), 1 if compile else 0)
+    n = lib.mol_codegen_batched(ds, ps, len(lows), tl, buf, len(buf), what | (1 if compile else 0))
     native.check(lib, n if n < 0 else 0, None)
     return buf.value.decode()
 

@@ -6,6 +6,7 @@ import molgpu
 from molgpu import systems
 from molgpu.batch import BatchProblem
 from molgpu.discretization import lower
+from test_sweep import axis_system
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +78,41 @@ def test_swept_batch_equals_stage_launches(dtype, kahan, monkeypatch):
         got = _run(batch, u0, 0.0, min(dts), N, kahan=kahan)
         ref = _run(stage, u0, 0.0, min(dts), N, kahan=kahan)
         assert np.max(np.abs(got - ref)) <= tol
+
+
+@pytest.mark.parametrize("dtype,kahan", [("f32", True), ("f32", False), ("f64", True), ("f64", False)])
+@pytest.mark.parametrize("first", [0, 1, 2])
+def test_mixed_periodic_batch_equals_stage_launches(first, dtype, kahan, monkeypatch):
+    """Periodic, non-periodic and one-axis-periodic instances in one batch, each kind first, at the
+    column counts where the two kinds differ in windows; the workspace holds NaN before the run."""
+    rng = np.random.default_rng(5)
+    kinds = [(True, True), (False, False), (True, False), (False, True)]
+    sizes = [(c, 12 + c // 4, *kinds[(j + first) % 4]) for c in (57, 64, 112, 120) for j in range(4)]
+    lows = [lower(*axis_system(c + (1 if xp else 2), r + (1 if yp else 2), xp, yp, dtype)) for c, r, xp, yp in sizes]
+    batch = BatchProblem(lows)
+    monkeypatch.setenv("MOL_SWEEP", "0")
+    stage = BatchProblem(lows)
+    # a run from NaN leaves NaN in every vector of the batch's workspace that a step writes
+    _run(batch, np.full(batch.n_unknowns, np.nan), 0.0, 1e-5, 3, kahan=kahan)
+    u0 = rng.uniform(0.1, 0.9, batch.n_unknowns)
+    tol = 1e-13 if dtype == "f64" else 4 * 2.0 ** -24 * (1 if kahan else 4)
+    for N in (1, 4):
+        print("  mixed batch first=%d %s kahan=%s N=%d" % (first, dtype, kahan, N), flush=True)
+        got = _run(batch, u0, 0.0, 1e-4, N, kahan=kahan)
+        ref = _run(stage, u0, 0.0, 1e-4, N, kahan=kahan)
+        assert np.all(np.isfinite(got))
+        assert np.max(np.abs(got - ref)) <= tol
+
+
+@pytest.mark.parametrize("kahan", [False, True])
+@pytest.mark.parametrize("nx,ny,rows", [(9, 30, 4), (57, 33, 7), (64, 20, 5), (120, 64, 64), (121, 40, 9)])
+@pytest.mark.parametrize("xper,yper", [(True, False), (False, True)])
+def test_swept_steps_with_one_periodic_axis(xper, yper, nx, ny, rows, kahan, monkeypatch):
+    monkeypatch.setenv("MOL_SWEEP", "1")
+    monkeypatch.setenv("MOL_SWEEP_ROWS", str(rows))
+    prob = molgpu.ODEProblem(lower(*axis_system(nx + (1 if xper else 2), ny + (1 if yper else 2), xper, yper)))
+    u0 = np.random.default_rng(nx).uniform(0.1, 0.9, prob.lowered.n_unknowns)
+    print("  sweep per=(%s, %s) %dx%d rows=%d kahan=%s" % (xper, yper, nx, ny, rows, kahan), flush=True)
+    ref = _run(prob, u0, 0.0, 1e-5, 5, kahan=kahan, fused=False)
+    got = _run(prob, u0, 0.0, 1e-5, 5, kahan=kahan)
+    assert np.max(np.abs(got - ref)) <= 1e-13 * (1 + np.max(np.abs(ref)))

@@ -73,3 +73,58 @@ def test_systems_that_the_sweep_does_not_hold_keep_the_tile_step(monkeypatch):
     monkeypatch.setenv("MOL_SWEEP", "1")
     assert "mol_rk4_sweep<" not in molgpu.codegen(lower(*systems.brusselator2d(n=65, approx_order=4)), fused=True)
     assert "mol_rk4_sweep<" not in molgpu.codegen(lower(*systems.mixed2d(41, 0.3)), fused=True)
+
+
+def axis_system(nx, ny, xper, yper, dtype="f64", k=1.0):
+    """u_t = 0.05 (u_xx + u_yy) + k u (1 - u), each axis periodic or from a value to a flux."""
+    t, x, y = parameters("t x y")
+    u = variables("u")
+    Dx, Dy = Differential(x), Differential(y)
+    U = u(t, x, y)
+    eq = Eq(Differential(t)(U), 0.05 * ((Dx ** 2)(U) + (Dy ** 2)(U)) + k * U * (1 - U))
+    bcs = [Eq(u(0, x, y), 0.5)]
+    bcs += [Eq(u(t, 0, y), u(t, 1, y))] if xper else [Eq(u(t, 0, y), 0.2), Eq(Dx(u(t, 1, y)), 0.1)]
+    bcs += [Eq(u(t, x, 0), u(t, x, 1))] if yper else [Eq(Dy(u(t, x, 0)), 0.3), Eq(u(t, x, 1), 0.4)]
+    return PDESystem([eq], bcs, [Interval(v, 0.0, 1.0) for v in (t, x, y)], [t, x, y], [U]), \
+        MOLFiniteDifference({x: nx, y: ny}, t, dtype=dtype)
+
+
+@pytest.mark.parametrize("xper,yper", [(True, False), (False, True)])
+@pytest.mark.parametrize("rows", [4, 9, 64])
+def test_swept_step_with_one_periodic_axis(xper, yper, rows, monkeypatch):
+    import molgpu
+    monkeypatch.setenv("MOL_SWEEP", "1")
+    monkeypatch.setenv("MOL_SWEEP_ROWS", str(rows))
+    low = lower(*axis_system(23, 31, xper, yper))
+    assert "mol_rk4_sweep<" in molgpu.codegen(low, fused=True)
+    w = np.random.default_rng(rows).uniform(0.1, 0.9, low.n_unknowns)
+    got, _ = genhost.rk4_fused(low, w, 0.0, 1e-3)
+    ref = _rk4(lambda v, s: genhost.rhs(low, v, t=s), w, 0.0, 1e-3)
+    assert np.max(np.abs(got - ref)) <= 1e-14 * (1 + np.max(np.abs(ref)))
+
+
+# columns around the edges of one and two windows, periodic and not
+MIXED = [(n, 20, xper, yper) for n in (9, 56, 57, 63, 64, 65, 112, 113, 119, 120, 121) for xper, yper in
+         ((True, True), (False, False), (True, False), (False, True))]
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_waves_of_a_mixed_batch_own_every_node_once(first, monkeypatch):
+    """Periodic and non-periodic instances in one batch, either kind first: the columns and rows
+    that the waves of an instance own tile it, each inside the part of its window that four
+    stages leave valid."""
+    from molgpu.batch import codegen_batched
+    monkeypatch.setenv("MOL_SWEEP_ROWS", "7")
+    order = MIXED[first:] + MIXED[:first]
+    lows = [lower(*axis_system(c + (1 if xp else 2), r + (1 if yp else 2), xp, yp, "f32")) for c, r, xp, yp in order]
+    waves = [[int(v) for v in ln.split()] for ln in codegen_batched(lows, waves=True).splitlines()]
+    own = [np.zeros((c, r), dtype=int) for c, r, _, _ in order]
+    for i, _, xb, x0, x1, y0, y1, _ in waves:
+        c, r, xper, yper = order[i]
+        assert 0 <= x0 < x1 <= c and 0 <= y0 < y1 <= r and (y0 == 0 or yper or y0 >= 4), (order[i], xb, x0, x1, y0, y1)
+        assert xper or xb >= 0, (order[i], xb)
+        assert x0 >= xb + 4 or (not xper and x0 == xb == 0), (order[i], xb, x0, x1)
+        assert x1 <= xb + 60 or (not xper and x1 == c <= xb + 64), (order[i], xb, x0, x1)
+        own[i][x0:x1, y0:y1] += 1
+    for i, m in enumerate(own):
+        assert np.all(m == 1), (order[i], m.min(), m.max())
