@@ -1322,6 +1322,19 @@ JitGeom vjp_geometry(mol_handle* h, const mol_desc* d, int* ntiles) {
   return g;
 }
 
+// Source of the reverse-mode tile kernel that `build` (its status, 0 when built) takes: where the
+// registers leave no room for the work-group, half the threads, each with twice the nodes.
+template <typename BUILD>
+std::string vjp_tiles_source(const mol_desc* d, JitGeom& g, std::string& err, const BUILD& build) {
+  for (;; g.nthr = (g.nthr / 2 + 63) / 64 * 64) {
+    const std::string src = jit_vjp_source(d, g, err);
+    if (src.empty()) return src;
+    const int rc = build(src, err);
+    if (rc == 0) return src;
+    if (rc != JIT_REGISTERS || g.nthr < 512) return std::string();
+  }
+}
+
 int ensure_vjp(mol_handle* h) {
   if (h->vjp_fn) return 0;
   const mol_desc* d = &h->desc.d;
@@ -1334,16 +1347,21 @@ int ensure_vjp(mol_handle* h) {
     ntiles = g.ntile[0] * g.ntile[1] * g.ntile[2];
     // (a result over its own seed or state is made here first)
     if (!h->adj_y[0]) HIPCHK(h, hipMalloc(&h->adj_y[0], (size_t)h->nunk * h->esize()));
+  }
+  int built = 0;
+  auto build = [&](const std::string& text, std::string& why) {
+    built = jit_kernel(text, "mol_vjp_tiles", h->device, &h->vjp_fn, why);
+    if (!built) built = jit_kernel(text, "mol_vjp_gather", h->device, &h->vjp_gather_fn, why);
+    if (built) h->vjp_fn = nullptr;
+    return built;
+  };
+  if (h->vjp_whole) {
+    if (build(src, err)) src.clear();
   } else {
-    src = jit_vjp_source(d, g, err);
+    src = vjp_tiles_source(d, g, err, build);
   }
-  if (src.empty()) return fail(h, MOL_ERR_UNSUPPORTED, "vector-Jacobian product: " + err);
+  if (src.empty()) return fail(h, built ? MOL_ERR_HIP : MOL_ERR_UNSUPPORTED, "vector-Jacobian product: " + err);
   h->vjp_store = src.find("// adjoint gather stores every unknown") != std::string::npos;
-  if (jit_kernel(src, "mol_vjp_tiles", h->device, &h->vjp_fn, err) ||
-      jit_kernel(src, "mol_vjp_gather", h->device, &h->vjp_gather_fn, err)) {
-    h->vjp_fn = nullptr;
-    return fail(h, MOL_ERR_HIP, "vector-Jacobian product: " + err);
-  }
   // per-tile buffers: VOLX positions per staged array and tile (numbers of the generated code)
   auto num_after = [&](const std::string& key, size_t from) -> long long {
     const size_t k = src.find(key, from);
@@ -2294,23 +2312,32 @@ int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t b
     build_core<double>(&tmp, d, tmp.ka64, tmp.kc64, gen, ncore);
   }
   std::string err;
-  std::string src;
+  std::string src, done;
+  auto compiled = [&](const std::string& text, std::string& why) {
+    std::vector<char> code;
+    std::string log;
+    const int r = text == done ? 0 : jit_compile(text, code, log);
+    if (r) why = "hiprtc: " + log;
+    else done = text;
+    return r;
+  };
   if (flags & MOL_CODEGEN_FUSED) {
     JitGeom g;
     if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, g, src))
       src = jit_fused_source(d, g, err);
   } else {
     const bool vjp = (flags & MOL_CODEGEN_VJP) != 0;
-    const JitGeom g = vjp ? vjp_geometry(&tmp, d, nullptr) : fwd_geom(tmp, ncore);
-    JitGeom gf;
-    if (!flux_source(&tmp, d, g, vjp, gf, src)) src = vjp ? jit_vjp_source(d, g, err) : jit_source(d, g, err);
+    JitGeom g = vjp ? vjp_geometry(&tmp, d, nullptr) : fwd_geom(tmp, ncore), gf;
+    if (!flux_source(&tmp, d, g, vjp, gf, src) && !vjp) src = jit_source(d, g, err);
+    if (vjp && src.empty()) {
+      src = vjp_tiles_source(d, g, err, [&](const std::string& text, std::string& why) {
+        return flags & MOL_CODEGEN_COMPILE ? (rc = compiled(text, why)) : 0;
+      });
+      if (src.empty()) return fail(nullptr, rc ? MOL_ERR_HIP : MOL_ERR_UNSUPPORTED, err);
+    }
   }
   if (src.empty()) return fail(nullptr, MOL_ERR_UNSUPPORTED, err);
-  if (flags & MOL_CODEGEN_COMPILE) {
-    std::vector<char> code;
-    std::string log;
-    if (jit_compile(src, code, log)) return fail(nullptr, MOL_ERR_HIP, "hiprtc: " + log);
-  }
+  if ((flags & MOL_CODEGEN_COMPILE) && compiled(src, err)) return fail(nullptr, MOL_ERR_HIP, err);
   if (buf && buflen > 0) {
     const size_t n = std::min<size_t>(src.size(), (size_t)buflen - 1);
     std::memcpy(buf, src.data(), n);

@@ -75,6 +75,9 @@ struct BInst {
   const double* K;
   double g[MOL_MAX_FIELDS][4][3];   // ghost next to each side of the first two axes (register sweep)
 };
+// 0, MOL_ERR_HIP, or JIT_REGISTERS where a kernel takes more registers than its work-group leaves it
+// (fewer threads may do).
+constexpr int JIT_REGISTERS = 1;
 int jit_compile(const std::string& src, std::vector<char>& code, std::string& log);
 int jit_kernel(const std::string& src, const char* name, int device, hipFunction_t* fn, std::string& err);
 

@@ -2713,6 +2713,39 @@ void disk_cache_store(const std::string& src, const std::vector<char>& code) {
   if (!ok || std::rename(tmp.c_str(), path.c_str()) != 0) (void)std::remove(tmp.c_str());
 }
 
+// Value of the integer that follows a key of the code object's metadata (MessagePack), from `at` on;
+// at: past it; -1: no such key.
+long long meta_int(const std::vector<char>& code, const char* key, size_t& at) {
+  const auto it = std::search(code.begin() + (long)at, code.end(), key, key + std::strlen(key));
+  size_t k = (size_t)(it - code.begin()) + std::strlen(key);
+  if (it == code.end() || k >= code.size()) return -1;
+  const unsigned char tag = (unsigned char)code[k++];
+  const int bytes = tag < 0x80 ? 0 : (tag == 0xcc ? 1 : (tag == 0xcd ? 2 : (tag == 0xce ? 4 : -1)));
+  if (bytes < 0 || k + (size_t)bytes > code.size()) return -1;
+  long long v = bytes ? 0 : tag;
+  for (int b = 0; b < bytes; ++b) v = 256 * v + (unsigned char)code[k++];
+  at = k;
+  return v;
+}
+
+// Whether the registers of every kernel leave room for its largest work-group: a SIMD unit has 512
+// per lane for its share of the group's waves.  (The compiler keeps to that within a function; a
+// kernel that calls one which is not inlined gets the larger of the two counts of each register kind,
+// whose sum can be more.  Launched, such a kernel is refused by the queue, and the process ends.)
+bool code_fits(const std::vector<char>& code, std::string& why) {
+  for (size_t at = 0;;) {
+    const long long wg = meta_int(code, ".max_flat_workgroup_size", at);
+    const long long regs = wg < 0 ? -1 : meta_int(code, ".vgpr_count", at);
+    if (regs < 0) return true;
+    const long long room = 512 / std::max(1ll, (wg + 255) / 256) / 8 * 8;
+    if ((regs + 7) / 8 * 8 > room) {
+      why = "a kernel takes " + std::to_string(regs) + " registers per lane, work-groups of " + std::to_string(wg) +
+            " threads leave it " + std::to_string(room);
+      return false;
+    }
+  }
+}
+
 }  // namespace
 
 std::string jit_fused_source(const mol_desc* d, const JitGeom& g, std::string& err) {
@@ -2800,19 +2833,19 @@ int jit_compile(const std::string& src, std::vector<char>& code, std::string& lo
   code.resize(cs);
   hiprtcGetCode(prog, code.data());
   hiprtcDestroyProgram(&prog);
-  return 0;
+  return code_fits(code, log) ? 0 : JIT_REGISTERS;
 }
 
 // Compile (or fetch from the process-wide cache) and load the generated kernel on `device`.
 int jit_kernel(const std::string& src, const char* name, int device, hipFunction_t* fn, std::string& err) {
   std::lock_guard<std::mutex> lk(g_jit_mu);
   CacheEntry& e = g_jit_cache[src];
-  if (e.code.empty() && !disk_cache_load(src, e.code)) {
+  if (e.code.empty() && !(disk_cache_load(src, e.code) && code_fits(e.code, err))) {
     std::string log;
-    if (jit_compile(src, e.code, log)) {
+    if (const int rc = jit_compile(src, e.code, log)) {
       g_jit_cache.erase(src);
       err = "hiprtc: " + log;
-      return MOL_ERR_HIP;
+      return rc;
     }
     disk_cache_store(src, e.code);
     if (const char* dir = std::getenv("MOL_JIT_DUMP")) {
