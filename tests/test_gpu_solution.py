@@ -85,3 +85,24 @@ def test_periodic_node_one_aliases_node_n():
     x = prob.lowered.coords[0]
     X, Y = np.meshgrid(x, x, indexing="ij")
     np.testing.assert_allclose(sol["u"][0], 22 * (Y * (1 - Y)) ** 1.5, rtol=1e-14, atol=1e-14)
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_saved_grids_come_as_the_device_lays_them_out(dtype, monkeypatch):
+    """Saves fetched over several buffers: grids first axis fastest (no transposing copy), equal to
+    the expansion of the saved state, arrays of different saves apart from each other."""
+    import torch
+    from molgpu import problem
+    prob = molgpu.discretize(*systems.diffreact2d(33, 0.05, 1.0, (0, 1, 1, 0), dtype=dtype))
+    monkeypatch.setattr(problem, "SAVE_BYTES", 3 * (31 * 31 + 33 * 33) * (8 if dtype == "f64" else 4))
+    sol = molgpu.solve(prob, molgpu.RK4, dt=1e-4, saveat=1e-4, tspan=(0.0, 7e-4))
+    assert len(sol.u) == len(sol.full) == len(sol.t) == 8
+    for t, u, g in zip(sol.t, sol.u, sol.full):
+        assert g.dtype == np.float64 and g.shape == (1, 33, 33) and g.transpose([0, 2, 1]).flags.c_contiguous
+        dev = torch.tensor(u, device="cuda").to(prob.torch_dtype())
+        np.testing.assert_array_equal(g, prob.expand(dev, t).cpu().numpy())
+    before = [g.copy() for g in sol.full]
+    sol.full[3][:] = -1.0
+    sol.u[4][:] = -1.0
+    for k in (0, 1, 2, 4, 5, 6, 7):
+        np.testing.assert_array_equal(sol.full[k], before[k])
