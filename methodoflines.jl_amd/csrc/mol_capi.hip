@@ -843,12 +843,32 @@ int sweep_rows(int device, int bytes, const std::vector<std::pair<int, int>>& bo
   return best;
 }
 
+// Nodes from which the register sweep takes a step, with the compensated update or without.  What
+// it is against: tiles, whose ghost refill between stages makes them slower on axes that are not
+// periodic; four stage launches for the compensated update.  A row of a strip takes longer the more
+// values a node has, and a small grid has fewer waves than the card has SIMD units, while small
+// tiles still run side by side (from 2^17 nodes in FP64 and 2^18 in FP32 they are larger ones).
+// Measured, time on tiles over time swept, both axes periodic, at 200^2, 300^2, 430^2 and 600^2: FP64
+// three variables 0.92, 1.00, 1.14, 1.36, five 0.76, 0.87, 1.19, 1.65 (0.95 and 0.85 at 340^2); FP32
+// three 0.89, 0.98, 0.98, 1.15, seven 0.73, 0.93, 0.93, 1.03; one and two variables 0.98 to 1.5,
+// other axes 1.06 to 2.4.  Nodes of 64 bytes, where the sweep spills: periodic 0.50, 0.63, 0.75, 2.0
+// (0.98 at 512^2), compensated 1.04, 0.78, 1.26, 1.7; other axes 0.93 at 200^2, 1.05 at 300^2, 1.9 at 600^2.
+int64_t sweep_from(const mol_handle* h, const mol_desc* d, bool kahan) {
+  const bool ring = d->periodic[0] && d->periodic[1], spills = d->nfields * h->esize() >= 64;
+  if (kahan) return ring && spills ? 1 << 17 : 0;
+  if (spills) return ring ? 300000 : 1 << 16;
+  if (!ring || d->nfields <= 2) return 0;
+  return h->esize() == 8 ? 1 << 17 : 1 << 18;
+}
+
 // The fused step of a 2D system of reach one whose tiles outnumber the compute units is a register
-// sweep where the system has one (jit_sweep_source).  MOL_SWEEP=0 or 1 overrides the size rule.
-bool sweep_source(mol_handle* h, const mol_desc* d, JitGeom& g, std::string& src) {
+// sweep where the system has one (jit_sweep_source) and sweep_from allows it.  MOL_SWEEP=0 or 1
+// overrides the size rules.
+bool sweep_source(mol_handle* h, const mol_desc* d, bool kahan, JitGeom& g, std::string& src) {
   if (d->ndim != 2 || h->tile_req[0] > 0 || std::getenv("MOL_FUSED_TILE") || std::getenv("MOL_FUSED_STEPS")) return false;
   const char* e = std::getenv("MOL_SWEEP");
-  if (e ? e[0] == '0' : g.fsteps != 1) return false;
+  const int64_t nodes = (int64_t)(g.uhi[0] - g.ulo[0] + 1) * (g.uhi[1] - g.ulo[1] + 1);
+  if (e ? e[0] == '0' : (g.fsteps != 1 || nodes < sweep_from(h, d, kahan))) return false;
   JitGeom gs = g;
   const int nw = sweep_windows(d->periodic[0], g.uhi[0] - g.ulo[0] + 1);
   gs.sweep_h = sweep_rows(h->device, d->nfields * (int)h->esize(), {{g.uhi[1] - g.ulo[1] + 1, nw}});
@@ -922,19 +942,24 @@ bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool
 
 void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, const KCore<double>& kc, int ncore) {
   h->fused_fn = h->fused_kahan_fn = nullptr;
-  h->fused_tiles = 0;
+  h->fused_tiles = h->fused_kahan_tiles = 0;
+  h->fused_resident = false;
+  h->fused_steps = 1;
   h->fused_reason.clear();
   const char* e = std::getenv("MOL_FUSED");
   if (e && e[0] == '0') { h->fused_reason = "disabled (MOL_FUSED=0)"; return; }
   JitGeom g;
   if (!fused_geometry(h, d, ka, kc, ncore, g, h->fused_reason)) return;
-  std::string err, src;
-  const bool sweep = sweep_source(h, d, g, src);
-  if (!sweep) src = jit_fused_source(d, g, err);
+  std::string err, src, csrc;
+  JitGeom gc = g;
+  if (sweep_source(h, d, true, gc, csrc)) {
+    if (jit_kernel(csrc, "mol_rk4_fused_kahan", h->device, &h->fused_kahan_fn, err)) h->fused_kahan_fn = nullptr;
+    h->fused_kahan_tiles = gc.ntile[0] * gc.ntile[1];
+  }
+  if (!sweep_source(h, d, false, g, src)) src = jit_fused_source(d, g, err);
   if (src.empty()) { h->fused_reason = err; return; }
-  if (jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err) ||
-      (sweep && jit_kernel(src, "mol_rk4_fused_kahan", h->device, &h->fused_kahan_fn, err))) {
-    h->fused_fn = h->fused_kahan_fn = nullptr;
+  if (jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
+    h->fused_fn = nullptr;
     h->fused_reason = err;
     return;
   }
@@ -1111,8 +1136,8 @@ int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int
       void* args1[] = {(void*)&sp, (void*)&dst, (void*)&e, (void*)&jp, (void*)&ns};
       void* argsb[] = {(void*)&sp, (void*)&dst, (void*)&e, (void*)&insts, (void*)&swl};
       void** args = h->batch ? argsb : args1;
-      if (hipModuleLaunchKernel(kahan ? h->fused_kahan_fn : h->fused_fn, h->fused_tiles, 1, 1, h->fused_nthr, 1, 1, 0, s, args, nullptr) !=
-          hipSuccess)
+      if (hipModuleLaunchKernel(kahan ? h->fused_kahan_fn : h->fused_fn, kahan ? h->fused_kahan_tiles : h->fused_tiles, 1, 1,
+                                kahan ? 64 : h->fused_nthr, 1, 1, 0, s, args, nullptr) != hipSuccess)
         return fail(h, MOL_ERR_HIP, "fused RK4 launch failed");
       h->clk ^= 1;
       std::swap(src, dst);
@@ -1968,7 +1993,7 @@ int create_batched(const mol_desc* const* ds, const double* const* params, int32
       free_handle(h);
       return MOL_ERR_HIP;
     }
-    h->fused_tiles = (int)(P.sweep.size() / 8);
+    h->fused_tiles = h->fused_kahan_tiles = (int)(P.sweep.size() / 8);
     h->fused_nthr = 64;
   }
   h->batch_grid = std::min(h->nwork, 1 << 24);
@@ -2323,7 +2348,7 @@ int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t b
   };
   if (flags & MOL_CODEGEN_FUSED) {
     JitGeom g;
-    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, g, src))
+    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, false, g, src))
       src = jit_fused_source(d, g, err);
   } else {
     const bool vjp = (flags & MOL_CODEGEN_VJP) != 0;

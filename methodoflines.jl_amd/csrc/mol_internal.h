@@ -221,7 +221,8 @@ struct mol_handle {
   int fused_nthr = 256;
   bool fused_resident = false;     // one 1D tile: many steps per fused launch
   int fused_steps = 1;             // steps per fused launch otherwise (1, or 2 with an 8-reach halo)
-  hipFunction_t fused_kahan_fn = nullptr;   // its compensated update (register sweep only)
+  hipFunction_t fused_kahan_fn = nullptr;   // the step with the compensated update (register sweep, 64 threads)
+  int fused_kahan_tiles = 0;
   std::string fused_reason;               // why there is no fused kernel
   bool no_fuse = false;                   // this integration runs the stage kernels (MOL_FLAG_UNFUSED)
   int vjp_nthr = 256;                     // threads per work-group of the generated VJP kernel

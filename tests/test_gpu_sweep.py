@@ -6,7 +6,7 @@ import molgpu
 from molgpu import systems
 from molgpu.batch import BatchProblem
 from molgpu.discretization import lower
-from test_sweep import axis_system
+from test_sweep import axis_system, coupled_system
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +116,19 @@ def test_swept_steps_with_one_periodic_axis(xper, yper, nx, ny, rows, kahan, mon
     ref = _run(prob, u0, 0.0, 1e-5, 5, kahan=kahan, fused=False)
     got = _run(prob, u0, 0.0, 1e-5, 5, kahan=kahan)
     assert np.max(np.abs(got - ref)) <= 1e-13 * (1 + np.max(np.abs(ref)))
+
+
+# systems whose plain step runs on tiles and whose compensated step is swept (199^2), both swept, and
+# eight FP64 variables, whose sweep keeps part of its rows in scratch memory
+@pytest.mark.parametrize("nf,dtype,n", [(3, "f64", 200), (4, "f32", 200), (3, "f64", 364), (8, "f64", 200), (8, "f64", 364)])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_steps_of_many_variables_equal_stage_launches(nf, dtype, n, periodic):
+    prob = molgpu.ODEProblem(lower(*coupled_system(nf, n, periodic, dtype)))
+    u0 = np.random.default_rng(n).uniform(0.1, 0.9, prob.lowered.n_unknowns)
+    dt = 0.5 / n ** 2
+    eps = 1e-13 if dtype == "f64" else 16 * 2.0 ** -24
+    for kahan in (False, True):
+        print("  many variables nf=%d %s n=%d kahan=%s" % (nf, dtype, n, kahan), flush=True)
+        ref = _run(prob, u0, 0.0, dt, 5, kahan=kahan, fused=False)
+        got = _run(prob, u0, 0.0, dt, 5, kahan=kahan)
+        assert np.max(np.abs(got - ref)) <= eps * (1 + np.max(np.abs(ref)))

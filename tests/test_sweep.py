@@ -128,3 +128,35 @@ def test_waves_of_a_mixed_batch_own_every_node_once(first, monkeypatch):
         own[i][x0:x1, y0:y1] += 1
     for i, m in enumerate(own):
         assert np.all(m == 1), (order[i], m.min(), m.max())
+
+
+def coupled_system(nf, n, periodic, dtype="f64"):
+    """u_t = (0.05 + 0.01 k) (u_xx + u_yy) + u (1 - v), and so on around nf variables."""
+    t, x, y = parameters("t x y")
+    vs = [variables("u%d" % k) for k in range(nf)]
+    Dx, Dy = Differential(x), Differential(y)
+    U = [v(t, x, y) for v in vs]
+    eqs, bcs = [], []
+    for k, v in enumerate(vs):
+        eqs.append(Eq(Differential(t)(U[k]), (0.05 + 0.01 * k) * ((Dx ** 2)(U[k]) + (Dy ** 2)(U[k])) +
+                      U[k] * (1 - U[(k + 1) % nf])))
+        bcs.append(Eq(v(0, x, y), 0.5))
+        if periodic:
+            bcs += [Eq(v(t, 0, y), v(t, 1, y)), Eq(v(t, x, 0), v(t, x, 1))]
+        else:
+            bcs += [Eq(v(t, 0, y), 0.2), Eq(Dx(v(t, 1, y)), 0), Eq(Dy(v(t, x, 0)), 0), Eq(v(t, x, 1), 0.4)]
+    return PDESystem(eqs, bcs, [Interval(q, 0.0, 1.0) for q in (t, x, y)], [t, x, y], U), \
+        MOLFiniteDifference({x: n, y: n}, t, dtype=dtype)
+
+
+# (variables, type, both axes periodic, nodes per side swept from or None for every size)
+@pytest.mark.parametrize("nf,dtype,periodic,line", [
+    (1, "f64", True, None), (2, "f64", True, None), (3, "f64", True, 363), (7, "f64", True, 363),
+    (8, "f64", True, 548), (8, "f64", False, 256), (7, "f64", False, None), (3, "f32", True, 512),
+    (8, "f32", True, 512), (8, "f32", False, None)])
+def test_sizes_that_the_sweep_takes_by_number_of_variables(nf, dtype, periodic, line):
+    """Systems whose tiles are faster on small grids (many variables, periodic axes) keep them."""
+    import molgpu
+    for side in ([200] if line is None else [line - 1, line]):
+        low = lower(*coupled_system(nf, side + (1 if periodic else 2), periodic, dtype))
+        assert ("mol_rk4_sweep<" in molgpu.codegen(low, fused=True)) == (line is None or side >= line)
