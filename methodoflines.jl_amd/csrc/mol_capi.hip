@@ -956,12 +956,17 @@ void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, cons
     if (jit_kernel(csrc, "mol_rk4_fused_kahan", h->device, &h->fused_kahan_fn, err)) h->fused_kahan_fn = nullptr;
     h->fused_kahan_tiles = gc.ntile[0] * gc.ntile[1];
   }
-  if (!sweep_source(h, d, false, g, src)) src = jit_fused_source(d, g, err);
-  if (src.empty()) { h->fused_reason = err; return; }
-  if (jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
-    h->fused_fn = nullptr;
-    h->fused_reason = err;
-    return;
+  // the sweep where it is wanted and builds, else the tiles
+  JitGeom gs = g;
+  if (sweep_source(h, d, false, gs, src) && !jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
+    g = gs;
+  } else {
+    src = jit_fused_source(d, g, err);
+    if (src.empty() || jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
+      h->fused_fn = nullptr;
+      h->fused_reason = err;
+      return;
+    }
   }
   h->fused_tiles = g.ntile[0] * g.ntile[1] * g.ntile[2];
   h->fused_nthr = g.nthr;
@@ -1002,11 +1007,12 @@ int setup_paths(mol_handle* h, const mol_desc* d) {
     jg.nthr = kernel_threads(jg, false);
     JitGeom fg;
     std::string src;
-    const bool flux = flux_source(h, d, jg, false, fg, src);
+    // the march where there is one and it builds, else the tiles
+    const bool flux = flux_source(h, d, jg, false, fg, src) && !jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err);
     if (!flux) src = jit_source(d, jg, err);
     h->jit_nthr = flux ? fg.nthr : jg.nthr;
     if (src.empty()) h->jit_reason = err;
-    else if (jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err)) {
+    else if (!flux && jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err)) {
       h->jit_fn = nullptr;
       h->jit_reason = err;
     }
@@ -1363,25 +1369,27 @@ std::string vjp_tiles_source(const mol_desc* d, JitGeom& g, std::string& err, co
 int ensure_vjp(mol_handle* h) {
   if (h->vjp_fn) return 0;
   const mol_desc* d = &h->desc.d;
-  int ntiles = 0;
+  int ntiles = 0, built = 0;
   JitGeom g = vjp_geometry(h, d, &ntiles), gf;
   std::string err, src;
-  h->vjp_whole = flux_source(h, d, g, true, gf, src);
-  if (h->vjp_whole) {
-    g = gf;
-    ntiles = g.ntile[0] * g.ntile[1] * g.ntile[2];
-    // (a result over its own seed or state is made here first)
-    if (!h->adj_y[0]) HIPCHK(h, hipMalloc(&h->adj_y[0], (size_t)h->nunk * h->esize()));
-  }
-  int built = 0;
   auto build = [&](const std::string& text, std::string& why) {
     built = jit_kernel(text, "mol_vjp_tiles", h->device, &h->vjp_fn, why);
     if (!built) built = jit_kernel(text, "mol_vjp_gather", h->device, &h->vjp_gather_fn, why);
     if (built) h->vjp_fn = nullptr;
     return built;
   };
+  // the march where there is one and it builds, else the tiles
+  h->vjp_whole = flux_source(h, d, g, true, gf, src) && build(src, err) == 0;
   if (h->vjp_whole) {
-    if (build(src, err)) src.clear();
+    g = gf;
+    ntiles = g.ntile[0] * g.ntile[1] * g.ntile[2];
+    // (a result over its own seed or state is made here first)
+    if (!h->adj_y[0] && hipMalloc(&h->adj_y[0], (size_t)h->nunk * h->esize()) != hipSuccess) {
+      (void)hipGetLastError();
+      h->adj_y[0] = nullptr;
+      h->vjp_fn = nullptr;
+      return fail(h, MOL_ERR_HIP, "vector-Jacobian product: not enough device memory");
+    }
   } else {
     src = vjp_tiles_source(d, g, err, build);
   }
@@ -1703,6 +1711,7 @@ struct BatchPlan {
   int nclasses = 0;
   int tile[3] = {1, 1, 1};
   std::string src;
+  size_t tiles_src = 0;   // characters of src before the step kernels
   // register sweep of a whole RK4 step: per wave instance, class, first column of its window, first
   // and end of the columns it owns and of its rows, 0; empty when an instance does not qualify
   std::vector<int32_t> sweep;
@@ -1883,6 +1892,7 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
   for (size_t c = 0; c < cls_src.size(); ++c)
     src << "    case " << c << ": mol_batch_tile<Geo" << c << ">(L, hd, tile, u, ep, t); break;\n";
   src << "    default: break;\n    }\n  }\n}\n";
+  P.tiles_src = src.str().size();
   if (sweep) {
     // a whole RK4 step per launch: a wave per window and strip of an instance, longest first
     // (the windows of each instance follow its own x axis: a batch may mix periodic and other axes)
@@ -1981,18 +1991,19 @@ int create_batched(const mol_desc* const* ds, const double* const* params, int32
     return MOL_ERR_HIP;
   }
   std::string err;
+  if (!P.sweep.empty() && (jit_kernel(P.src, "mol_batch_rk4", h->device, &h->fused_fn, err) ||
+                           jit_kernel(P.src, "mol_batch_rk4_kahan", h->device, &h->fused_kahan_fn, err))) {
+    // the step kernels do not build: stage launches
+    h->fused_fn = h->fused_kahan_fn = nullptr;
+    h->fused_reason = err;
+    P.src.resize(P.tiles_src);
+  }
   if (jit_kernel(P.src, "mol_batch_tiles", h->device, &h->batch_fn, err)) {
     set_global_error("batched kernel: " + err);
     free_handle(h);
     return MOL_ERR_HIP;
   }
-  if (!P.sweep.empty()) {
-    if (jit_kernel(P.src, "mol_batch_rk4", h->device, &h->fused_fn, err) ||
-        jit_kernel(P.src, "mol_batch_rk4_kahan", h->device, &h->fused_kahan_fn, err)) {
-      set_global_error("batched kernel: " + err);
-      free_handle(h);
-      return MOL_ERR_HIP;
-    }
+  if (h->fused_fn) {
     h->fused_tiles = h->fused_kahan_tiles = (int)(P.sweep.size() / 8);
     h->fused_nthr = 64;
   }
@@ -2069,7 +2080,12 @@ int64_t mol_codegen_batched(const mol_desc* const* ds, const double* const* para
   if (flags & MOL_CODEGEN_COMPILE) {
     std::vector<char> code;
     std::string log;
-    if (jit_compile(P.src, code, log)) return fail(nullptr, MOL_ERR_HIP, "hiprtc: " + log);
+    if (!P.sweep.empty() && jit_compile(P.src, code, log)) {   // stage launches (create_batched)
+      P.sweep.clear();
+      P.src.resize(P.tiles_src);
+      code.clear();
+    }
+    if (code.empty() && jit_compile(P.src, code, log)) return fail(nullptr, MOL_ERR_HIP, "hiprtc: " + log);
   }
   std::string& text = P.src;
   if (flags & MOL_CODEGEN_WAVES) {
@@ -2346,15 +2362,20 @@ int64_t mol_codegen(const mol_desc* d, const int32_t* tile, char* buf, int64_t b
     else done = text;
     return r;
   };
+  // (compiled: what runs instead of a march or sweep that does not build)
+  auto taken = [&]() { return !(flags & MOL_CODEGEN_COMPILE) || compiled(src, err) == 0; };
   if (flags & MOL_CODEGEN_FUSED) {
-    JitGeom g;
-    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err) && !sweep_source(&tmp, d, false, g, src))
-      src = jit_fused_source(d, g, err);
+    JitGeom g, gs;
+    if (fused_geometry(&tmp, d, tmp.ka64, tmp.kc64, ncore, g, err)) {
+      gs = g;
+      if (!(sweep_source(&tmp, d, false, gs, src) && taken())) src = jit_fused_source(d, g, err);
+    }
   } else {
     const bool vjp = (flags & MOL_CODEGEN_VJP) != 0;
     JitGeom g = vjp ? vjp_geometry(&tmp, d, nullptr) : fwd_geom(tmp, ncore), gf;
-    if (!flux_source(&tmp, d, g, vjp, gf, src) && !vjp) src = jit_source(d, g, err);
-    if (vjp && src.empty()) {
+    const bool flux = flux_source(&tmp, d, g, vjp, gf, src) && taken();
+    if (!flux && !vjp) src = jit_source(d, g, err);
+    if (!flux && vjp) {
       src = vjp_tiles_source(d, g, err, [&](const std::string& text, std::string& why) {
         return flags & MOL_CODEGEN_COMPILE ? (rc = compiled(text, why)) : 0;
       });

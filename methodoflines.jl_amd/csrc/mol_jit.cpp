@@ -2808,7 +2808,16 @@ std::string jit_flux_source(const mol_desc* d, const JitGeom& g, bool vjp, std::
   return s;
 }
 
+// MOL_JIT_FAIL=text: sources that hold the text are taken not to compile (for tests of what runs then).
+static bool refused(const std::string& src, std::string& why) {
+  const char* const e = std::getenv("MOL_JIT_FAIL");
+  if (!e || !e[0] || src.find(e) == std::string::npos) return false;
+  why = "refused (MOL_JIT_FAIL)";
+  return true;
+}
+
 int jit_compile(const std::string& src, std::vector<char>& code, std::string& log) {
+  if (refused(src, log)) return MOL_ERR_HIP;
   hiprtcProgram prog;
   const char* hdr_names[] = {"mol_jit_prelude.h"};
   const char* hdrs[] = {mol_jit_prelude_text};
@@ -2838,6 +2847,7 @@ int jit_compile(const std::string& src, std::vector<char>& code, std::string& lo
 
 // Compile (or fetch from the process-wide cache) and load the generated kernel on `device`.
 int jit_kernel(const std::string& src, const char* name, int device, hipFunction_t* fn, std::string& err) {
+  if (refused(src, err)) return MOL_ERR_HIP;
   std::lock_guard<std::mutex> lk(g_jit_mu);
   CacheEntry& e = g_jit_cache[src];
   if (e.code.empty() && !(disk_cache_load(src, e.code) && code_fits(e.code, err))) {

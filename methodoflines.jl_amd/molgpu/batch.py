@@ -46,6 +46,9 @@ def codegen_batched(lows: Sequence[Lowered], compile: bool = False, tile=None, w
     native.check(lib, n if n < 0 else 0, None)
     buf = C.create_string_buffer(int(n) + 1)
     n = lib.mol_codegen_batched(ds, ps, len(lows), tl, buf, len(buf), what | (1 if compile else 0))
+    if n >= len(buf):   # (compiled: another kernel than the first choice may be the one that builds)
+        buf = C.create_string_buffer(int(n) + 1)
+        n = lib.mol_codegen_batched(ds, ps, len(lows), tl, buf, len(buf), what | (1 if compile else 0))
     native.check(lib, n if n < 0 else 0, None)
     return buf.value.decode()
 

@@ -363,6 +363,9 @@ def codegen(low: Lowered, compile: bool = False, tile=None, vjp: bool = False, f
     native.check(lib, n if n < 0 else 0, None)
     buf = C.create_string_buffer(int(n) + 1)
     n = lib.mol_codegen(C.byref(desc), tl, buf, len(buf), what | (1 if compile else 0))
+    if n >= len(buf):   # (compiled: another kernel than the first choice may be the one that builds)
+        buf = C.create_string_buffer(int(n) + 1)
+        n = lib.mol_codegen(C.byref(desc), tl, buf, len(buf), what | (1 if compile else 0))
     native.check(lib, n if n < 0 else 0, None)
     return buf.value.decode()
 
