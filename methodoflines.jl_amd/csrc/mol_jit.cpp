@@ -122,6 +122,7 @@ class Gen {
   // RK4 step swept along y in registers (mol_rk4_sweep): 2D, reach one, cross-shaped taps
   std::string source_sweep(bool f64);
   std::string sweep_class(const std::string& name);
+  bool reads_both(const std::vector<int>& outs, int f, int ax) const;
   std::string sweep_class_of(const std::string& name) {   // parametric, for batched instances
     param_ = true;
     return sweep_class(name);
@@ -2191,6 +2192,31 @@ std::string Gen::source_class(const std::string& name) {
   return o.str();
 }
 
+// Whether every output that reads variable f on one side of the node along an axis carries what it
+// finds on the other side too, by sums and products (a choice between the sides does not).
+bool Gen::reads_both(const std::vector<int>& outs, int f, int ax) const {
+  for (int o : outs) {
+    bool any[2] = {false, false}, sure[2] = {false, false};
+    std::vector<std::pair<int, bool>> todo = {{o, true}};
+    std::set<std::pair<int, bool>> seen;
+    while (!todo.empty()) {
+      const std::pair<int, bool> at = todo.back();
+      todo.pop_back();
+      if (!seen.insert(at).second) continue;
+      const Node& n = nodes_[at.first];
+      if (n.kind == N_LDS && n.arr == f && n.dv[ax] != 0) {
+        any[n.dv[ax] > 0] = true;
+        if (at.second) sure[n.dv[ax] > 0] = true;
+      }
+      const bool on = at.second && n.kind == N_OP && (n.op == X_LINCOMB || n.op == MOL_OP_ADD || n.op == MOL_OP_SUB ||
+                                                      n.op == MOL_OP_MUL || n.op == MOL_OP_NEG);
+      for (int a : n.a) todo.push_back({a, on});
+    }
+    if ((any[0] && !sure[1]) || (any[1] && !sure[0])) return false;
+  }
+  return true;
+}
+
 // Class body of the register sweep: window geometry, ghosts next to the four sides, node function
 // and its node-invariant part.  Empty when the system does not qualify.
 std::string Gen::sweep_class(const std::string& name) {
@@ -2267,7 +2293,10 @@ std::string Gen::sweep_class(const std::string& name) {
       const std::string tw = param_ ? "hd.g[f][side][" + istr(m) + "]" : lit(w);
       e += (e.empty() ? "" : " + ") + tw + " * " + x;
     };
-    for (int m = 0; m < (param_ ? 2 : cl.K); ++m) term(m, param_ ? 1.0 : d_->pool_h[cl.wC + m], m == 0 ? "y0" : "y1");
+    // batched: sides whatever their terms share a class, those with fewer by zero factors, where a node
+    // next to the side reads both nodes anyway (zero times an infinite node is not zero)
+    const bool either = param_ && reads_both(outs, cl.field, cl.axis);
+    for (int m = 0; m < (either ? 2 : cl.K); ++m) term(m, param_ ? 1.0 : d_->pool_h[cl.wC + m], m == 0 ? "y0" : "y1");
     if (cl.gprog >= 0) term(2, param_ ? 1.0 : d_->pool_h[cl.wc], G);
     o << "    return " << (e.empty() ? "T(0)" : e) << ";\n    }\n";
   }

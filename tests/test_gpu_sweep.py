@@ -5,7 +5,8 @@ import pytest
 import molgpu
 from molgpu import systems
 from molgpu.batch import BatchProblem
-from molgpu.discretization import lower
+from molgpu.discretization import MOLFiniteDifference, UpwindScheme, lower
+from molgpu.pdesys import Differential, Eq, Interval, PDESystem, parameters, variables
 from test_sweep import axis_system, coupled_system
 
 pytestmark = pytest.mark.gpu
@@ -132,3 +133,44 @@ def test_steps_of_many_variables_equal_stage_launches(nf, dtype, n, periodic):
         ref = _run(prob, u0, 0.0, dt, 5, kahan=kahan, fused=False)
         got = _run(prob, u0, 0.0, dt, 5, kahan=kahan)
         assert np.max(np.abs(got - ref)) <= eps * (1 + np.max(np.abs(ref)))
+
+
+def _advected(nx, ny, left, dtype="f64"):
+    """u_t = -u_x - u_y, upwind: a node reads itself and the nodes below it on either axis."""
+    t, x, y = parameters("t x y")
+    u = variables("u")
+    Dx, Dy = Differential(x), Differential(y)
+    U = u(t, x, y)
+    bcs = [Eq(u(0, x, y), 0.5), Eq(u(t, 0, y), 0.2) if left == 0 else Eq(Dx(u(t, 0, y)), 0), Eq(u(t, 1, y), 0.1),
+           Eq(u(t, x, 0), 0.3), Eq(u(t, x, 1), 0.4)]
+    return lower(PDESystem([Eq(Differential(t)(U), -Dx(U) - Dy(U))], bcs, [Interval(v, 0.0, 1.0) for v in (t, x, y)],
+                           [t, x, y], [U]), MOLFiniteDifference({x: nx, y: ny}, t, advection_scheme=UpwindScheme(1), dtype=dtype))
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("kind", ["upwind", "centred"])
+def test_batch_sides_with_a_value_do_not_read_the_nodes_next_to_them(kind, bad, dtype, monkeypatch):
+    """One infinite or undefined node, the second from each side that has a value: it spreads
+    where the stencil carries it, as with stage launches, and not through the side's ghost."""
+    if kind == "upwind":
+        lows = [_advected(30, 25, 0, dtype), _advected(80, 20, 1, dtype), _advected(70, 40, 0, dtype)]
+    else:
+        lows = [lower(*systems.diffreact2d(n, 0.05, 1.0, bc, dtype=dtype)) for n, bc in
+                ((30, (0, 0, 0, 0)), (80, (0, 1, 1, 0)), (70, (1, 0, 0, 1)))]
+    batch = BatchProblem(lows)
+    monkeypatch.setenv("MOL_SWEEP", "0")
+    stage = BatchProblem(lows)
+    u0 = np.random.default_rng(2).uniform(0.1, 0.9, batch.n_unknowns)
+    for low, at in zip(lows, batch.offsets):
+        nx, ny = (int(n) - 2 for n in low.n[:2])
+        v = u0[at:at + nx * ny].reshape(ny, nx)
+        v[ny // 2, 1] = v[1, nx // 2] = bad
+    for kahan in (False, True):
+        print("  batch sides %s %s %s kahan=%s" % (kind, bad, dtype, kahan), flush=True)
+        got = _run(batch, u0, 0.0, 1e-4, 1, kahan=kahan)
+        ref = _run(stage, u0, 0.0, 1e-4, 1, kahan=kahan)
+        assert np.isfinite(ref).sum() > 0.5 * ref.size
+        np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+        ok = np.isfinite(ref)
+        assert np.max(np.abs(got[ok] - ref[ok])) <= (1e-13 if dtype == "f64" else 16 * 2.0 ** -24)

@@ -160,3 +160,25 @@ def test_sizes_that_the_sweep_takes_by_number_of_variables(nf, dtype, periodic, 
     for side in ([200] if line is None else [line - 1, line]):
         low = lower(*coupled_system(nf, side + (1 if periodic else 2), periodic, dtype))
         assert ("mol_rk4_sweep<" in molgpu.codegen(low, fused=True)) == (line is None or side >= line)
+
+
+def test_one_sided_operators_keep_boundary_kinds_apart():
+    """A class of batched instances serves sides of any kind by zero factors only where the node next
+    to a side reads the nodes that the factors stand for; upwind operators get a class per kind."""
+    from molgpu.batch import codegen_batched
+    from molgpu.discretization import UpwindScheme
+    t, x, y = parameters("t x y")
+    u = variables("u")
+    Dx, Dy = Differential(x), Differential(y)
+    U = u(t, x, y)
+
+    def low(left, rhs, **kw):
+        bcs = [Eq(u(0, x, y), 0.5), Eq(u(t, 0, y), 0) if left == 0 else Eq(Dx(u(t, 0, y)), 0), Eq(u(t, 1, y), 0),
+               Eq(u(t, x, 0), 0), Eq(u(t, x, 1), 0)]
+        return lower(PDESystem([Eq(Differential(t)(U), rhs)], bcs, [Interval(v, 0.0, 1.0) for v in (t, x, y)], [t, x, y],
+                               [U]), MOLFiniteDifference({x: 30, y: 25}, t, **kw))
+
+    for rhs, kw, classes in ((-Dx(U) - Dy(U), {"advection_scheme": UpwindScheme(1)}, 2),
+                             ((Dx ** 2)(U) + (Dy ** 2)(U), {}, 1)):
+        src = codegen_batched([low(0, rhs, **kw), low(1, rhs, **kw)], compile=True)
+        assert src.count("struct SwpY") == classes
