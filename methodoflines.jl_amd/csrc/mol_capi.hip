@@ -1769,7 +1769,11 @@ int plan_batched(const mol_desc* const* ds, const double* const* params, int32_t
       cls = it->second;
     }
     // instances of one class share the sweep's class too (its body has the same structure)
-    for (int a = 0; a < 2 && sweep; ++a) sweep = a >= d->ndim || ka.uhi[a] - ka.ulo[a] + 1 >= 8;
+    // (but its boxes are the instance's own)
+    for (int a = 0; a < 2 && sweep; ++a) {
+      sweep = a >= d->ndim || ka.uhi[a] - ka.ulo[a] + 1 >= 8;
+      for (int f = 1; f < d->nfields && sweep; ++f) sweep = ka.lo[f][a] == ka.lo[0][a] && ka.hi[f][a] == ka.hi[0][a];
+    }
     if (sweep && fresh) {
       const std::string ss = jit_sweep_class(d, geom_of(ka, th.kc64, ncore), "SwpY", err);
       sweep = !ss.empty();

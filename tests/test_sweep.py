@@ -182,3 +182,17 @@ def test_one_sided_operators_keep_boundary_kinds_apart():
                              ((Dx ** 2)(U) + (Dy ** 2)(U), {}, 1)):
         src = codegen_batched([low(0, rhs, **kw), low(1, rhs, **kw)], compile=True)
         assert src.count("struct SwpY") == classes
+
+
+def test_every_instance_of_a_class_is_asked_whether_it_can_be_swept():
+    """Two variables on unequal boxes step by stage launches, also behind an instance of the same
+    class (boxes are numbers of the instance, not of the class) whose boxes are equal."""
+    import copy
+    from molgpu.batch import codegen_batched
+    low = lower(*coupled_system(2, 30, False))
+    other = copy.deepcopy(low)
+    other.hi[1][0] -= 1
+    assert "mol_rk4_sweep<" in codegen_batched([low, low])
+    for order in ([low, other], [other, low]):
+        src = codegen_batched(order)
+        assert "2 instances, 1 classes" in src and "mol_rk4_sweep<" not in src
