@@ -747,17 +747,23 @@ bool fused_geometry(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, c
   }
   // two threads per tile node (every stage region is larger than the tile), at most 1024
   g.nthr = std::max(256, std::min(1024, (2 * g.tile[0] * g.tile[1] * g.tile[2] + 63) / 64 * 64));
+  const char* const ne = std::getenv("MOL_FUSED_NTHR");
+  if (ne) g.nthr = (std::max(64, std::min(1024, std::atoi(ne))) + 63) / 64 * 64;
   if (whole && g.ntile[0] == 1) {
     // resident steps in registers (mol_rk4_ring): one wave, or four (one per SIMD) once a lane
     // would hold more than five values.  Heat, FP64, us per step with one wave / four / eight:
     // 99 unknowns 0.157 / 0.245 / 0.309, 255: 0.212 / 0.273 / 0.305, 398: 0.325 / 0.285 / 0.314,
     // 598: 0.447 / 0.406 / 0.357, 998: 0.629 / 0.521 / 0.525 (the tile in LDS with frames and
-    // two barriers per stage took 0.88, 0.91, 1.04, 1.10 and 1.23).  Each of the four waves
-    // holds at least its neighbour's overlap and the unknowns of a boundary closure.
-    const int n = g.tile[0], own = (n + 3) / 4, least = 4 * ka.halo[0] + std::max(kmax, 1);
-    g.nthr = n * d->nfields > 320 && own >= least && n - 3 * own >= least ? 256 : 64;
+    // two barriers per stage took 0.88, 0.91, 1.04, 1.10 and 1.23).  Up to eight variables of 32 to
+    // 998 unknowns, FP64 and FP32, four waves are within 17 % of the best of one to sixteen past that
+    // line (998 unknowns of eight FP64 variables, where it spills, 4.3 us, tile in LDS 29).
+    if (!ne) g.nthr = g.tile[0] * d->nfields > 320 ? 256 : 64;
+    // each of several waves holds at least its neighbour's overlap and the unknowns of a boundary closure
+    const int n = g.tile[0], least = 4 * ka.halo[0] + std::max(kmax, 1);
+    auto fits = [&](const int w) { return w == 1 || n - (w - 1) * ((n + w - 1) / w) >= least; };
+    if (!ne && !fits(4)) g.nthr = 64;
+    while (!fits(g.nthr / 64)) g.nthr -= 64;
   }
-  if (const char* ne = std::getenv("MOL_FUSED_NTHR")) g.nthr = (std::max(64, std::min(1024, std::atoi(ne))) + 63) / 64 * 64;
   // Two steps per launch (an 8-reach halo, a fourth LDS array for the first step's running
   // sums) when every tile is resident at once: the launch overhead, the staging latency and the
   // store drain then come once per two steps, against stage regions about a quarter larger

@@ -475,3 +475,13 @@ def test_reverse_mode_with_a_variable_read_only_at_its_node():
         d2 = (val(5e-5) - val(-5e-5)) / 1e-4
         fd = (4 * d2 - d1) / 3
         assert abs(out @ v - fd) <= 1e-7 * abs(fd) + 1e-9 * np.linalg.norm(out) * np.linalg.norm(v), tile
+
+
+@pytest.mark.parametrize("unknowns", [4, 6, 38, 128, 321, 1024])
+@pytest.mark.parametrize("threads", [64, 512, 1024])
+def test_resident_step_builds_with_any_number_of_threads_asked_for(unknowns, threads, monkeypatch):
+    """MOL_FUSED_NTHR asks for more waves than the unknowns fill: as many as do are taken."""
+    import molgpu
+    monkeypatch.setenv("MOL_FUSED_NTHR", str(threads))
+    low = lower(*systems.heat1d(n=unknowns + 2, bcl=(1.0, 2.0, 0.1), bch=(2.0, -1.0, 0.4)))
+    assert "// resident steps per launch: any" in molgpu.codegen(low, fused=True, compile=True)
