@@ -314,6 +314,7 @@ void fill_kargs(mol_handle* h, const mol_desc* d, KArgs<T>& ka, size_t lds_pos =
     tile[big] = (tile[big] + 1) / 2;
   }
   if (lds_pos == 0) lds_pos = (size_t)nload * sizeof(T);
+  if (jit_tiles == 1) h->level_rows = false;
   if (jit_tiles && h->tile_req[0] <= 0 && d->ndim >= 2) {
     // generated kernels run several nodes per thread along the slowest axis: the first
     // candidate whose tile + halo of the staged arrays fits the LDS budget (forward: about
@@ -372,6 +373,7 @@ void fill_kargs(mol_handle* h, const mol_desc* d, KArgs<T>& ka, size_t lds_pos =
         if (share(ty) < least) {
           least = share(ty);
           tile[1] = ty;
+          h->level_rows = true;
         }
     }
   }
@@ -1011,6 +1013,7 @@ int setup_paths(mol_handle* h, const mol_desc* d) {
     std::string err;
     JitGeom jg = geom_of(h->ka64, h->kc64, n64);
     jg.nthr = kernel_threads(jg, false);
+    jg.level = h->level_rows;
     JitGeom fg;
     std::string src;
     // the march where there is one and it builds, else the tiles
@@ -2337,6 +2340,7 @@ void mol_destroy(mol_handle* h) { free_handle(h); }
 JitGeom fwd_geom(const mol_handle& h, int ncore) {
   JitGeom g = geom_of(h.ka64, h.kc64, ncore);
   g.nthr = kernel_threads(g, false);
+  g.level = h.level_rows;
   return g;
 }
 

@@ -21,6 +21,7 @@ struct JitGeom {
   int nthr;                                           // threads per work-group (multiple of 64)
   int fsteps = 1;                                     // fused RK4: steps per launch (1 or 2)
   int sweep_h = 0;                                    // fused RK4 as a register sweep: rows per strip
+  bool level = false;                                 // rows per tile chosen for even shares (level_rows)
 };
 
 // Pointer arguments of the generated kernel (layout identical to JPtrs of mol_jit_prelude.h).
@@ -214,6 +215,7 @@ struct mol_handle {
   void* d_swl = nullptr;                  // wave list of the batch's RK4 register sweep
   void* d_bdata = nullptr;                // weights, constants and coordinates of all instances
   std::vector<int64_t> inst_off;          // first unknown of each instance
+  bool level_rows = false;                // the tile's rows even out the compute units (WENO5)
   int jit_grid = 0;                       // work-groups of the persistent generated RHS kernel
   int jit_nthr = 256;                     // threads per work-group of the generated RHS kernel
   hipFunction_t fused_fn = nullptr;       // generated fused RK4 step (periodic 1D/2D systems)

@@ -437,13 +437,13 @@ class Gen {
     // the Burgers WENO5 right-hand side at 1024^2).  WENO5 in FP32 with tiles that the box cuts: one,
     // four groups in turn (4100^2 80.3 -> 73.6 us, 2900^2 43.1 -> 39.8; whole tiles, 4096^2: 73.2
     // against 70.9 with two; FP64 46.3 -> 47.5 at 2900^2; fourth-order diffusion 18.8 -> 22.3).  One
-    // also for its tiles of 28, 20 or 12 rows.
+    // also for tiles of fewer rows that even out the compute units (1447^2: see fill_kargs).
     bool weno = false;
     for (int k = 0; k < d_->nslots; ++k) weno = weno || d_->slots_h[k].kind == MOL_SLOT_WENO;
     weno = weno && d_->ndim == 2 && g_.halo[0] >= 2 && g_.halo[1] >= 2;
     bool cut = false;
     for (int a = 0; a < 2; ++a) cut = cut || (g_.uhi[a] - g_.ulo[a] + 1) % g_.tile[a] != 0;
-    const bool one = weno && ((g_.nthr >= 512 && d_->dtype != MOL_F64 && cut) || (g_.tile[0] == 64 && g_.tile[1] % 8 == 4));
+    const bool one = weno && ((g_.nthr >= 512 && d_->dtype != MOL_F64 && cut) || g_.level);
     const int want = e ? std::max(1, std::atoi(e)) : (one ? 1 : g_.nthr >= 512 ? 2 : 4);
     for (int r = want; r > 1; r /= 2)
       if (g_.tile[ba] % r == 0 && (e || vol / r >= g_.nthr)) {

@@ -392,3 +392,19 @@ def test_solution_interpolation_is_multilinear():
     assert sol(0.5, x[3], y[5]) == f(0.5, x[3], y[5])
     np.testing.assert_array_equal(sol["u"], np.stack([g[0] for g in full]))
     np.testing.assert_array_equal(sol[low.axes[1]], y)
+
+
+def test_tiles_asked_for_keep_their_blocking():
+    """WENO5 tiles whose rows the library chooses for even shares of the compute units run one node per
+    thread; a tile of the same shape that the caller asks for is blocked like any other."""
+    import re
+    import molgpu
+    from molgpu import systems as S
+    low = lower(*S.burgers2d(1448))
+    const = lambda src, k: int(re.search(r"static constexpr int %s = (\d+);" % k, src)[1])
+    own = molgpu.codegen(low)
+    tile = (const(own, "TX"), const(own, "TY"), 1)
+    assert tile[0] == 64 and tile[1] < 32 and const(own, "RB") == 1
+    asked = molgpu.codegen(low, tile=tile)
+    assert (const(asked, "TX"), const(asked, "TY")) == tile[:2]
+    assert const(asked, "RB") == (4 if tile[1] % 4 == 0 and 64 * tile[1] >= 1024 else 2)
