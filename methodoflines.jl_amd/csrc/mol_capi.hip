@@ -904,7 +904,8 @@ bool sweep_source(mol_handle* h, const mol_desc* d, bool kahan, JitGeom& g, std:
 // size rule is against it.  MOL_FLUX=0 or 1 overrides the size rule, MOL_FLUX_TILE=tx,ty,planes and
 // MOL_FLUX_VJP_TILE ask for other columns and chunks.
 //
-// Size: forward from 48^3 unknowns, reverse from 2^16, and not where half of the columns or more
+// Size: forward from 48^3 unknowns (50^3 with two interpolated fields: 48^3 FP64 7.8 -> 8.2 us, 51^3
+// 12.3 -> 8.3), reverse from 2^16, and not where half of the columns or more
 // would be padding.  Fewer leave compute units without a work-group.  Per right-hand side and per
 // reverse step with its gradients (FP64, us, tiles -> march): 28^3 5.7 -> 6.9 and 13.4 -> 13.6, 44^3
 // 6.7 -> 7.3 and 16.6 -> 13.6, 48^3 6.8 -> 6.4 and 16.4 -> 14.2, 52^3 7.9 -> 7.1 and 21.1 -> 13.8,
@@ -931,7 +932,15 @@ bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool
   for (int a = 0; a < 3; ++a) m[a] = g.n[a] - 2;
   if (m[0] < 3 || m[1] < 3 || m[2] < 3) return false;
   const long long nt = (long long)((m[0] + tile[0] - 1) / tile[0]) * ((m[1] + tile[1] - 1) / tile[1]);
-  if (!force && ((long long)m[0] * m[1] * m[2] < (vjp ? 1 << 16 : 48 * 48 * 48) || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
+  bool half[MOL_MAX_AUX] = {};   // grid fields that the coefficients interpolate
+  for (int k = 0; k < d->nslots; ++k) {
+    const int prog = d->slots_h[k].prog;
+    const int st = prog < 0 ? 0 : d->prog_h[2 * prog], ln = prog < 0 ? 0 : d->prog_h[2 * prog + 1];
+    for (int pc = st; pc < st + ln; ++pc)
+      if ((d->code_h[pc] & 0xffu) == MOL_OP_AUX) half[d->code_h[pc] >> 21] = true;
+  }
+  const long long least = vjp ? 1 << 16 : (std::count(half, half + MOL_MAX_AUX, true) > 1 ? 50 * 50 * 50 : 48 * 48 * 48);
+  if (!force && ((long long)m[0] * m[1] * m[2] < least || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
   if (tile[2] == 0) {
     const int occ = vjp ? (f64 ? 3 : 4) : (f64 ? 5 : 8);   // resident work-groups per compute unit
     const int ncu = compute_units(h->device);

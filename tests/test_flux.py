@@ -119,3 +119,14 @@ def test_march_compiles_for_gfx950(name, monkeypatch):
     monkeypatch.setenv("MOL_FLUX", "1")
     for vjp in (False, True):
         assert "mol_flux_" in molgpu.codegen(SYSTEMS[name](), vjp=vjp, compile=True)
+
+
+def test_sizes_that_the_march_takes():
+    """Right-hand sides from 48^3 unknowns, with two interpolated fields from 50^3 (at 48^3 tiles are as
+    fast or faster)."""
+    import molgpu
+    one, two = [d0(*F) * (1 + U ** 2)] * 3, [d0(*F) * (1 + U ** 2), d0(*F) + s0(*F), 1 + U]
+    for coef, least in ((one, 50), (two, 52)):
+        for n in (least - 1, least):
+            src = molgpu.codegen(system(coef, 0, neumann(), n=(n, n, n)))
+            assert ("mol_flux_rhs<GeoB>(" in src) == (n >= least)
