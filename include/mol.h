@@ -250,8 +250,13 @@ int mol_set_tile(mol_handle* h, int32_t tx, int32_t ty, int32_t tz);
 
 /* Launch plan: info[0..2] tile shape, info[3] core tiles, info[4] generic tiles, info[5] WENO tiles,
  * info[6] 1 when the core tiles run the generated kernel, info[7] 1 when the IR fits the
- * interpreter's core kernel, info[8] tiles of the fused RK4 step kernel (0: none), info[9] RK4 steps
- * per fused launch (1, or 2 with an 8-reach halo; 0: none, or a resident 1D tile). */
+ * interpreter's core kernel, info[8] tiles (or waves) of the fused RK4 step kernel (0: none), info[9]
+ * RK4 steps per fused launch (1, or 2 with an 8-reach halo; 0: none, or a resident 1D system),
+ * info[10] 1 when the right-hand side is marched along z (info[0..2] are then the columns and planes
+ * of a work-group and info[3] their number), info[11] the step kernel: 0 none, 1 tiles, 2 resident 1D
+ * system, 3 register sweep, info[12] waves of the step with the compensated update (0: stage launches).
+ * Batched handles: info[0..2] tile, info[3] work items of a stage, info[6] 1, info[7] classes, info[8]
+ * waves of the RK4 step (0: stage launches). */
 int mol_get_plan(const mol_handle* h, int32_t* info, int32_t ninfo);
 
 /* Bind auxiliary full-grid arrays (device pointers, naux of them, each prod(n) values). */

@@ -969,7 +969,7 @@ bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool
 void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, const KCore<double>& kc, int ncore) {
   h->fused_fn = h->fused_kahan_fn = nullptr;
   h->fused_tiles = h->fused_kahan_tiles = 0;
-  h->fused_resident = false;
+  h->fused_resident = h->fused_sweep = false;
   h->fused_steps = 1;
   h->fused_reason.clear();
   const char* e = std::getenv("MOL_FUSED");
@@ -986,6 +986,7 @@ void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, cons
   JitGeom gs = g;
   if (sweep_source(h, d, false, gs, src) && !jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
     g = gs;
+    h->fused_sweep = true;
   } else {
     src = jit_fused_source(d, g, err);
     if (src.empty() || jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
@@ -1037,6 +1038,7 @@ int setup_paths(mol_handle* h, const mol_desc* d) {
     // the march where there is one and it builds, else the tiles
     const bool flux = flux_source(h, d, jg, false, fg, src) && !jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err);
     if (!flux) src = jit_source(d, jg, err);
+    for (int a = 0; a < 3; ++a) h->march[a] = flux ? fg.tile[a] : 0;
     h->jit_nthr = flux ? fg.nthr : jg.nthr;
     if (src.empty()) h->jit_reason = err;
     else if (!flux && jit_kernel(src, "mol_rhs_tiles", h->device, &h->jit_fn, err)) {
@@ -2168,16 +2170,21 @@ int mol_set_tile(mol_handle* h, int32_t tx, int32_t ty, int32_t tz) {
 int mol_get_plan(const mol_handle* h, int32_t* info, int32_t ninfo) {
   if (!h || !info) return MOL_ERR_INVALID;
   if (h->batch) {
-    // batch: tile, work items, 0, 0, generated, number of classes
-    const int32_t b[8] = {h->ka64.tile[0], h->ka64.tile[1], h->ka64.tile[2], h->nwork, 0, 0, 1, h->nclasses};
-    for (int i = 0; i < ninfo && i < 8; ++i) info[i] = b[i];
+    // batch: tile, work items, 0, 0, generated, number of classes, waves of the step kernel
+    const int32_t b[9] = {h->ka64.tile[0], h->ka64.tile[1], h->ka64.tile[2], h->nwork, 0, 0, 1, h->nclasses,
+                          h->fused_fn ? h->fused_tiles : 0};
+    for (int i = 0; i < ninfo && i < 9; ++i) info[i] = b[i];
     return 0;
   }
-  int32_t v[10] = {h->ka64.tile[0], h->ka64.tile[1], h->ka64.tile[2], h->ncore, h->nbound,
+  const bool march = h->jit_fn && h->march[0] > 0;
+  const int32_t* tile = march ? h->march : h->ka64.tile;
+  const int step = !h->fused_fn ? 0 : (h->fused_sweep ? 3 : (h->fused_resident ? 2 : 1));
+  int32_t v[13] = {tile[0], tile[1], tile[2], march ? h->jit_grid : h->ncore, march ? 0 : h->nbound,
                    0, h->jit_fn != nullptr ? 1 : 0,
                    h->core_interp_ok ? 1 : 0, h->fused_fn ? h->fused_tiles : 0,
-                   h->fused_fn ? (h->fused_resident ? 0 : h->fused_steps) : 0};
-  for (int i = 0; i < ninfo && i < 10; ++i) info[i] = v[i];
+                   h->fused_fn ? (h->fused_resident ? 0 : h->fused_steps) : 0,
+                   march ? 1 : 0, step, h->fused_kahan_fn ? h->fused_kahan_tiles : 0};
+  for (int i = 0; i < ninfo && i < 13; ++i) info[i] = v[i];
   return 0;
 }
 

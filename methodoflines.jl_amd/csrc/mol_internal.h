@@ -221,6 +221,8 @@ struct mol_handle {
   hipFunction_t fused_fn = nullptr;       // generated fused RK4 step (periodic 1D/2D systems)
   int fused_tiles = 0;
   int fused_nthr = 256;
+  int32_t march[3] = {0, 0, 0};    // columns and planes of the 3D march's work-groups (0: tiles)
+  bool fused_sweep = false;        // the fused step is the register sweep
   bool fused_resident = false;     // one 1D tile: many steps per fused launch
   int fused_steps = 1;             // steps per fused launch otherwise (1, or 2 with an 8-reach halo)
   hipFunction_t fused_kahan_fn = nullptr;   // the step with the compensated update (register sweep, 64 threads)

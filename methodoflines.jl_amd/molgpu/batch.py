@@ -90,9 +90,9 @@ class BatchProblem:
         return np.concatenate([low.u0 for low in self.lowered])
 
     def plan(self) -> dict:
-        info = (C.c_int32 * 8)()
-        self.lib.mol_get_plan(self.h, info, 8)
-        return {"tile": (info[0], info[1], info[2]), "work_items": info[3], "classes": info[7]}
+        info = (C.c_int32 * 9)()
+        self.lib.mol_get_plan(self.h, info, 9)
+        return {"tile": (info[0], info[1], info[2]), "work_items": info[3], "classes": info[7], "step_waves": info[8]}
 
     def split(self, u) -> List[np.ndarray]:
         u = np.asarray(u)
