@@ -1403,12 +1403,13 @@ int ensure_vjp(mol_handle* h) {
   std::string err, src;
   auto build = [&](const std::string& text, std::string& why) {
     built = jit_kernel(text, "mol_vjp_tiles", h->device, &h->vjp_fn, why);
-    if (!built) built = jit_kernel(text, "mol_vjp_gather", h->device, &h->vjp_gather_fn, why);
+    if (!built && !h->vjp_whole) built = jit_kernel(text, "mol_vjp_gather", h->device, &h->vjp_gather_fn, why);
     if (built) h->vjp_fn = nullptr;
     return built;
   };
   // the march where there is one and it builds, else the tiles
-  h->vjp_whole = flux_source(h, d, g, true, gf, src) && build(src, err) == 0;
+  h->vjp_whole = flux_source(h, d, g, true, gf, src);
+  h->vjp_whole = h->vjp_whole && build(src, err) == 0;
   if (h->vjp_whole) {
     g = gf;
     ntiles = g.ntile[0] * g.ntile[1] * g.ntile[2];

@@ -2644,7 +2644,9 @@ std::string Gen::source_flux(bool f64, bool vjp) {
          "  const double t = (va.tnow ? va.tnow[0] : 0.0) + va.tofs;\n"
          "  mol_flux_vjp<GeoB>(S, va, jp, t);\n}\n"
          "// adjoint gather stores every unknown; nothing is left to gather\n"
-         "extern \"C\" __global__ void __launch_bounds__(256) mol_vjp_gather(VArgs va) { (void)va; }\n";
+         "#ifndef __AMDGCN__\n"
+         "extern \"C\" void mol_vjp_gather(VArgs va) { (void)va; }\n"
+         "#endif\n";
   }
   return o.str();
 }
