@@ -544,12 +544,13 @@ __device__ __forceinline__ T mol_weno5_nu_tab(T u1, T u2, T u3, T u4, T u5, cons
   else return mol_weno5_nu_apply<T>(u1, u2, u3, u4, u5, c, eps);
 }
 
-// Coordinate of (unwrapped) node k of a periodic axis: the image across an end is continued by
-// the period x[n] - x[1] (bcoord, src/discretization/interface_boundary.jl:120-151).
-__device__ __forceinline__ double mol_pcoord(const double* x, const int k, const int n) {
-  if (k <= 1) return x[k + n - 2] - (x[n - 1] - x[0]);
-  if (k > n) return x[k - n] + (x[n - 1] - x[0]);
-  return x[k - 1];
+// Distance of (unwrapped) node k of an axis from node i: past an end of a periodic axis the image's,
+// continued by the period x[n] - x[1] (bcoord, src/discretization/interface_boundary.jl:120-151) and
+// summed from differences on either side of the end.
+__device__ __forceinline__ double mol_offset(const double* x, const int k, const int i, const int n) {
+  if (k < 1) return (x[k + n - 2] - x[n - 1]) - (x[i - 1] - x[0]);
+  if (k > n) return (x[n - 1] - x[i - 1]) + (x[k - n] - x[0]);
+  return x[k - 1] - x[i - 1];
 }
 
 // The gradient from a node's row of precomputed coefficients.
@@ -564,7 +565,9 @@ __device__ __noinline__ void mol_weno5_nu_tab_grad(T u1, T u2, T u3, T u4, T u5,
 
 // Row of coefficients (MOL_NU3 or MOL_NU_NC values) of node i = 1..n of an axis with coordinates x: the
 // stencil and target of the generated code (one-sided at nodes 1, 2, n-1, n of a non-periodic
-// axis, centred elsewhere; periodic images through mol_pcoord).
+// axis, centred elsewhere).  They depend on differences of coordinates only and are made from the
+// stencil's distances to the node: half points of whole coordinates carry their rounding, eps / h of
+// a spacing h (705 nodes, largest error of the derivative of random values 6.1e-11 -> 1e-12).
 __device__ __forceinline__ void mol_weno_nu_row(const double* x, const int n, const bool periodic, const int i,
                                                 double* c) {
   int first = -2, target = 3;
@@ -580,7 +583,7 @@ __device__ __forceinline__ void mol_weno_nu_row(const double* x, const int n, co
   double xs[5];
   for (int q = 0; q < 5; ++q) {
     const int k = i + first + q;
-    xs[q] = periodic ? mol_pcoord(x, k, n) : x[k - 1];
+    xs[q] = mol_offset(x, k, i, n);
   }
   switch (target) {
     case 1: mol_weno5_nu_coefs<1>(xs[0], xs[1], xs[2], xs[3], xs[4], c); break;

@@ -224,3 +224,50 @@ def test_generated_rhs_on_stretched_2d_nodes(periodic, tile):
     ref = ref + np.stack([orc.weno_nu1d_rhs(nodes[1], 0.5, 1e-6, periodic, 0.1, 0.4, np.ascontiguousarray(col))
                           for col in v.T]).T
     assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(ref))
+
+
+def exact_derivative(x, v, periodic, eps=1e-6):
+    """The centred-target derivative along the last axis in extended precision (values on every node;
+    the first and last two of a non-periodic axis are left out): three quadratics, smoothness by
+    Simpson's rule over the node's cell, ideal weights of the five-point derivative."""
+    L = np.longdouble
+    x, v = x.astype(L), v.astype(L)
+    if periodic:     # nodes 2..n, images continued by the period
+        m, ring = len(x) - 1, x[1:]
+        i = np.arange(m)
+        at = [np.roll(ring, -k) + (x[-1] - x[0]) * ((i + k >= m).astype(L) - (i + k < 0).astype(L)) for k in range(-2, 3)]
+        vals = [np.roll(v, -k, axis=-1) for k in range(-2, 3)]
+    else:
+        at = [x[2 + k:len(x) - 2 + k] for k in range(-2, 3)]
+        vals = [v[..., 2 + k:len(x) - 2 + k] for k in range(-2, 3)]
+    lo, hi = (at[1] + at[2]) / 2, (at[2] + at[3]) / 2
+    mid, dx = (lo + hi) / 2, hi - lo
+    r, w = [], []
+    for k in range(3):
+        a, b, c = at[k:k + 3]
+        la, lb, lc = 1 / ((a - b) * (a - c)), 1 / ((b - a) * (b - c)), 1 / ((c - a) * (c - b))
+        d1 = lambda z: (2 * z - b - c) * la * vals[k] + (2 * z - a - c) * lb * vals[k + 1] + (2 * z - a - b) * lc * vals[k + 2]
+        d2 = 2 * (la * vals[k] + lb * vals[k + 1] + lc * vals[k + 2])
+        w.append(1 / (L(eps) + dx * dx / 6 * (d1(lo) ** 2 + 4 * d1(mid) ** 2 + d1(hi) ** 2) + dx ** 4 * d2 ** 2) ** 2)
+        r.append(d1(at[2]))
+    a, b, c, d, e = at
+    g0, g2 = (c - d) * (c - e) / ((a - d) * (a - e)), (c - a) * (c - b) / ((e - a) * (e - b))
+    w = [g * q for g, q in zip((g0, 1 - g0 - g2, g2), w)]
+    return sum(p * q for p, q in zip(w, r)) / sum(w)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("n", [38, 151, 705])
+def test_coefficients_do_not_carry_the_rounding_of_whole_coordinates(n, periodic):
+    """Random values: the derivative is exact to some roundings of u / h, on any number of nodes (half
+    points made from whole coordinates were off by eps / h of a spacing, at 705 nodes eight times
+    this bound)."""
+    h = 1.0 + 0.3 * (2 * np.random.default_rng(3).random(n - 1) - 1)
+    x = np.concatenate([[0.0], np.cumsum(h)]) / h.sum()
+    x[-1] = 1.0
+    low = lower(*systems.weno1d_nonuniform(x, 1.0, 0.25, 0.375, periodic=periodic))
+    u = np.random.default_rng(1).uniform(0.0, 1.0, low.n_unknowns)
+    got = genhost.rhs(low, u)
+    v, inner = (u, slice(None)) if periodic else (np.concatenate([[0.25], u, [0.375]]), slice(1, -1))
+    err = np.max(np.abs(got[inner] + exact_derivative(x, v, periodic)))
+    assert err <= 64 * 2.0 ** -53 / np.diff(x).min()
