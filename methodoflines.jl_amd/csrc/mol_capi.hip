@@ -697,8 +697,9 @@ int kernel_threads(const JitGeom& g, bool vjp) {
   return vjp ? std::max(256, n) : n;
 }
 
-// Fused RK4 step kernel for periodic 1D/2D systems of reach 1 (MOL_FUSED=0 disables it): the
-// tile + 4-node halo of u and two stage buffers in LDS, one launch per step.
+// Fused RK4 step of 1D/2D systems of reach one (two on periodic axes; MOL_FUSED=0 disables it): the
+// tile + halo of u and two stage buffers in LDS, one launch per step or two steps, or a 1D system
+// whole in the registers of one work-group.
 bool fused_geometry(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, const KCore<double>& kc, int ncore,
                     JitGeom& g, std::string& why) {
   if (d->ndim > 2) { why = "not a 1D/2D system"; return false; }
@@ -733,7 +734,7 @@ bool fused_geometry(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, c
   }
   if (best < 0) { why = "tile does not fit LDS"; return false; }
   // a 1D box of up to 1024 unknowns is one tile: the kernel then runs many steps per launch
-  // with the state resident in LDS
+  // with the state in registers (mol_rk4_ring)
   static const int whole1[3] = {1024, 1, 1};
   const bool whole = d->ndim == 1 && ka.uhi[0] - ka.ulo[0] + 1 <= whole1[0];
   if (whole) cand = &whole1, best = 0;
@@ -1124,14 +1125,14 @@ struct Work {
 
 Work handle_work(const mol_handle* h) { return Work{h->w_y1, h->w_y2, h->w_acc, h->w_comp, h->d_tnow}; }
 
-// t0v: the start time, passed by value to the first fused launch instead of read from the
-// device clock (which that launch then sets for the next); null: the clock holds it.
-// comp_zero: the first fused launch takes the compensation as zero instead of reading it.
 // RK4 runs as fused launches (the compensated update only where the fused kernel has it).
 bool use_fused(const mol_handle* h, int scheme, bool kahan) {
   return scheme == MOL_RK4 && (kahan ? h->fused_kahan_fn : h->fused_fn) && !h->no_fuse;
 }
 
+// t0v: the start time, passed by value to the first fused launch instead of read from the
+// device clock (which that launch then sets for the next); null: the clock holds it.
+// comp_zero: the first fused launch takes the compensation as zero instead of reading it.
 template <typename T>
 int enqueue_steps(mol_handle* h, const Work& w, T* u, const T* p, double dt, int64_t nsteps, int scheme,
                   bool kahan, hipStream_t s, const double* t0v = nullptr, bool comp_zero = false) {
@@ -1335,8 +1336,6 @@ bool prog_uses(const mol_desc* d, int prog, uint32_t op) {
   return false;
 }
 
-// Generate and load the vector-Jacobian product kernel (first use).  Its tiles are sized for
-// the state, the auxiliary arrays and their adjoint buffers in LDS.
 // Tiling of the reverse-mode kernel: LDS holds the state, the grid fields and their adjoint
 // buffers (FP64 for every array).
 JitGeom vjp_geometry(mol_handle* h, const mol_desc* d, int* ntiles) {
@@ -1395,6 +1394,7 @@ std::string vjp_tiles_source(const mol_desc* d, JitGeom& g, std::string& err, co
   }
 }
 
+// Generate and load the vector-Jacobian product kernel (first use).
 int ensure_vjp(mol_handle* h) {
   if (h->vjp_fn) return 0;
   const mol_desc* d = &h->desc.d;

@@ -2,10 +2,12 @@
 
 The reference discretizes and solves one problem at a time (an ensemble of MOL problems is a
 loop of ``discretize``/``solve``).  A ``BatchProblem`` takes many lowered instances — uneven
-grids, coefficients and boundary kinds — and runs their right-hand sides in one launch per
-Runge–Kutta stage (a work-group per tile of an instance, largest tiles first): instances of one
-structure share generated code, per-instance numbers are read from instance headers
-(``mol_create_batched`` in include/mol.h).
+grids, coefficients and boundary kinds — and runs their right-hand sides in one launch (a
+work-group per tile of an instance, largest tiles first), and where every instance is a 2D system
+of reach one a whole RK4 step in one launch (a wave per window of columns and strip of rows of an
+instance); other batches take a launch per Runge–Kutta stage.  Instances of one structure share
+generated code, per-instance numbers are read from instance headers (``mol_create_batched`` in
+include/mol.h).
 """
 from __future__ import annotations
 
