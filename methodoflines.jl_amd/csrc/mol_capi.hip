@@ -978,14 +978,15 @@ void setup_fused(mol_handle* h, const mol_desc* d, const KArgs<double>& ka, cons
   JitGeom g;
   if (!fused_geometry(h, d, ka, kc, ncore, g, h->fused_reason)) return;
   std::string err, src, csrc;
-  JitGeom gc = g;
+  JitGeom gs = g, gc = g;
+  const bool sweep = sweep_source(h, d, false, gs, src);
+  gc.kahan_only = !sweep;
   if (sweep_source(h, d, true, gc, csrc)) {
     if (jit_kernel(csrc, "mol_rk4_fused_kahan", h->device, &h->fused_kahan_fn, err)) h->fused_kahan_fn = nullptr;
     h->fused_kahan_tiles = gc.ntile[0] * gc.ntile[1];
   }
   // the sweep where it is wanted and builds, else the tiles
-  JitGeom gs = g;
-  if (sweep_source(h, d, false, gs, src) && !jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
+  if (sweep && !jit_kernel(src, "mol_rk4_fused", h->device, &h->fused_fn, err)) {
     g = gs;
     h->fused_sweep = true;
   } else {

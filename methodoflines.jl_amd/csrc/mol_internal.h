@@ -21,6 +21,7 @@ struct JitGeom {
   int nthr;                                           // threads per work-group (multiple of 64)
   int fsteps = 1;                                     // fused RK4: steps per launch (1 or 2)
   int sweep_h = 0;                                    // fused RK4 as a register sweep: rows per strip
+  bool kahan_only = false;                            // register sweep: only the compensated step's kernel
   bool level = false;                                 // rows per tile chosen for even shares (level_rows)
 };
 

@@ -2347,6 +2347,7 @@ std::string Gen::source_sweep(bool f64) {
   o << "struct GeoBase {\n" << geo_common() << "};\n\n" << body;
   // two kernels: the compensated update's registers would cost the plain one occupancy
   for (const char* kahan : {"false", "true"}) {
+    if (g_.kahan_only && kahan[0] == 'f') continue;
     o << "extern \"C\" __global__ void __launch_bounds__(64) mol_rk4_fused" << (kahan[0] == 't' ? "_kahan" : "")
       << "(const T* __restrict__ u, T* __restrict__ unew,\n"
          "    Epi ep, JPtrs jp, int nsub) {\n"
