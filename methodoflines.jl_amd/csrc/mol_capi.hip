@@ -257,13 +257,6 @@ int validate(const mol_desc* d, std::string& msg) {
 
 // lds_pos: LDS bytes per tile + halo position (0: the forward kernels' arrays)
 // clamp: shrink the tile to the box (a batch keeps one tile shape for all its instances)
-// Compute units of a device (256 where there is none: generated source without a GPU).
-int compute_units(int device) {
-  int n = 0;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
-  return n;
-}
-
 template <typename T>
 void fill_kargs(mol_handle* h, const mol_desc* d, KArgs<T>& ka, size_t lds_pos = 0, bool clamp = true,
                 int jit_tiles = 0, size_t lds_cap = 60000) {
@@ -371,10 +364,9 @@ void fill_kargs(mol_handle* h, const mol_desc* d, KArgs<T>& ka, size_t lds_pos =
       // of a node per staged position.  Taken from a gain of 8% (below it measurements are even).
       // Burgers at 1447^2 (five tiles on some units, 4.1 on average): FP32 14.7 -> 13.2 us, FP64
       // 16.4 -> 15.8; 1300^2: 13.2 -> 11.5 and 14.2 -> 13.0.  (Lighter stencils: no gain.)
-      const int ncu = compute_units(h->device);
       auto share = [&](const int ty) {
         const int64_t nt = (int64_t)((ka.uhi[0] - ka.ulo[0] + 64) / 64) * ((ka.uhi[1] - ka.ulo[1] + ty) / ty);
-        return (double)((nt + ncu - 1) / ncu) * (64 * ty + 0.2 * (64 + 2 * ka.halo[0]) * (ty + 2 * ka.halo[1]));
+        return (double)((nt + 255) / 256) * (64 * ty + 0.2 * (64 + 2 * ka.halo[0]) * (ty + 2 * ka.halo[1]));
       };
       double least = 0.92 * share(32);
       for (int ty : {28, 20, 12})
@@ -840,8 +832,8 @@ int build_wenonu_tables(mol_handle* h, const mol_desc* d, const std::string& src
 // MOL_SWEEP_ROWS overrides.
 int sweep_rows(int device, int bytes, const std::vector<std::pair<int, int>>& box) {
   if (const char* e = std::getenv("MOL_SWEEP_ROWS")) return std::max(4, std::atoi(e));
-  const int ncu = compute_units(device);
-  int top = 4;
+  int ncu = 0, top = 4;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0) ncu = 256;
   for (const auto& b : box) top = std::max(top, b.first);
   const int64_t w = std::max(1, 32 / bytes);
   const double fixed = std::min(1.5, 8.0 / bytes);
@@ -944,10 +936,9 @@ bool flux_source(const mol_handle* h, const mol_desc* d, const JitGeom& gt, bool
   if (!force && ((long long)m[0] * m[1] * m[2] < least || nt * tile[0] * tile[1] >= 2ll * m[0] * m[1])) return false;
   if (tile[2] == 0) {
     const int occ = vjp ? (f64 ? 3 : 4) : (f64 ? 5 : 8);   // resident work-groups per compute unit
-    const int ncu = compute_units(h->device);
     double best = 0.0;
     for (int z = vjp ? 4 : 3; z <= 16; ++z) {
-      const long long k = (nt * std::min((m[2] + z - 1) / z, m[2] / 3) + ncu - 1) / ncu;
+      const long long k = (nt * std::min((m[2] + z - 1) / z, m[2] / 3) + 255) / 256;
       const double cost = (z + 2) * ((k / occ) * (2.6 + occ) + (k % occ ? 2.6 + k % occ : 0.0));
       if (tile[2] == 0 || cost < best) {
         best = cost;
