@@ -1220,9 +1220,9 @@ inline U mol_lane(const U x, const int) { return x; }
 // Otherwise (several waves, or a periodic ring) a wave holds S nodes and, evaluated redundantly,
 // the HL = 4 reach nodes past either end: a whole step needs no other wave, and the end nodes
 // are exchanged once per step through LDS (two buffers in turn, one barrier).
-// What bounds it is the issue of a wave's serial chain (about 100 VALU instructions per step of
-// the 101-node FP64 heat equation: 0.155 us, against 0.88 us for the stages on an LDS tile with
-// two barriers each).
+// What bounds it is the serial chain of a stage (the 101-node FP64 heat equation: 71 VALU instructions
+// and 341 cycles per step, 0.142 us, against 0.88 us for the stages on an LDS tile with two
+// barriers each).
 template <class G>
 struct MolRing {
   static constexpr int LN = G::NTHR < MOL_WAVE ? G::NTHR : MOL_WAVE;   // lanes per wave
